@@ -60,6 +60,10 @@ struct EntArgs {
 // True when launch_local_ent can produce the quantized outputs in one fused kernel.
 bool ent_fused_ok(const EntArgs& a);
 
+// The fused kernel of wide bf16 rows (entangle_mfma.hip): the shapes it takes, and its launch.
+bool ent_mfma_ok(const EntArgs& a, int64_t weff);
+int launch_ent_mfma(const EntArgs& a, int64_t weff, hipStream_t st);
+
 int64_t ent_ws_bytes(int64_t B, int64_t L, int64_t H, int64_t W);
 int launch_local_ent(const EntArgs& a, hipStream_t st);
 

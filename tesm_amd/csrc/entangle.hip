@@ -1567,7 +1567,7 @@ static bool fused16_fits(const EntArgs& a, int64_t weff) {
 bool ent_fused_ok(const EntArgs& a) {
   if (a.mimo || a.H != 1) return false;
   const int64_t weff = eff_window(a);
-  return fused16_fits(a, weff) || reg_fits(a, weff);
+  return fused16_fits(a, weff) || reg_fits(a, weff) || ent_mfma_ok(a, weff);
 }
 
 int64_t ent_ws_bytes(int64_t B, int64_t L, int64_t H, int64_t W) {
@@ -1590,7 +1590,8 @@ int launch_local_ent(const EntArgs& a, hipStream_t st) {
   const int64_t weff = eff_window(a);
   if (a.q_te) {
     TESM_REQUIRE(ent_fused_ok(a), kErrUnsupported,
-                 "local_ent: fused quantization needs SISO, D <= 512 and a small enough window/rank");
+                 "local_ent: fused quantization needs SISO, D <= 512 (bf16: D <= 4096, a multiple of 16) and a small enough "
+                 "window/rank");
     TESM_REQUIRE(a.q_c && a.s_te && a.s_c && a.rs_te && a.rs_c && a.ldq >= a.D && a.ldq % 16 == 0 &&
                      aligned(a.q_te, 16) && aligned(a.q_c, 16),
                  kErrInvalidArg, "local_ent: bad quantized outputs");
@@ -1605,6 +1606,7 @@ int launch_local_ent(const EntArgs& a, hipStream_t st) {
     };
     const bool big = !fits(4) && fits(8);
     if (fused2_fits(a, weff)) return run_fused2<true>(a, weff, st);
+    if (ent_mfma_ok(a, weff)) return launch_ent_mfma(a, weff, st);
     if (!fused16_fits(a, weff)) return a.dt == kBF16 ? run_reg<kBF16>(a, weff, st) : run_reg<kF32>(a, weff, st);
     if (a.dt == kBF16) {
       if (big)
