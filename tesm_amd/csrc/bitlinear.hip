@@ -8,22 +8,21 @@
 //   acc = sum_k q_x * u_w - sum_k q_x      (u = code + 1)
 // and the per-row sum of activation codes (from the quantization kernel) removes the offset.
 //
-// Two kernels:
+// Kernels:
 //   * gemv_kernel  (M <= 4): bandwidth-bound decode path.  Each lane streams 16-byte packed
 //     chunks (64 codes) with one 128-bit load, unpacks in registers with shift/and and
 //     multiplies with v_dot4_i32_i8 against activation codes held in registers.
-//   * mfma_kernel  (M > 4): LDS-tiled int8 MFMA (v_mfma_i32_16x16x64_i8).  Packed weight tiles
-//     are unpacked to int8 while being staged in LDS; A and B fragments are stored in MFMA
-//     lane order so every ds_read_b128 of a wave is one contiguous 1 KiB block.
+//   * skinny_kernel / skinny_fq_kernel (M <= 32): 16x16x64 int8 MFMA with the K loop split over a workgroup's
+//     waves, operands straight from memory.
+//   * the 32x32x32 kernels of mfma32.hip (M > 32).
+//   * the output gate's row kernels (gate32_kernel, gate_rowq_lds_kernel, gate_rowq_kernel).
 #include <cstdlib>
 
-#include "tesm_hip_internal.h"
+#include "linear_dev.h"
 
 namespace tesm {
 
 namespace {
-
-__device__ __forceinline__ uint32_t unpack_u(uint32_t w, int s) { return (w >> (2 * s)) & 0x03030303u; }
 
 // ---------------------------------------------------------------------------
 // GEMV
@@ -155,258 +154,6 @@ __global__ __launch_bounds__(256) void gemv_kernel(LinearArgs a) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// MFMA GEMM
-// ---------------------------------------------------------------------------
-template <int WM, int WN, int TM, int TN>
-struct Cfg {
-  static constexpr int NT = WM * WN * 64;
-  static constexpr int BM = WM * TM * 16, BN = WN * TN * 16, BK = 128;
-  static constexpr int A_BYTES = BM * BK;        // int8 codes, fragment order
-  static constexpr int B_BYTES = BN * BK / 4;    // packed INT2, fragment order (one dword per lane)
-  static constexpr int STAGE = A_BYTES + B_BYTES;
-  static constexpr int A_CHUNKS = BM * BK / 16;  // 16-byte code chunks per K tile
-  static constexpr int B_CHUNKS = BN * BK / 64;  // 16-byte packed chunks per K tile
-  static constexpr int A_PT = (A_CHUNKS + NT - 1) / NT;
-  static constexpr int B_PT = (B_CHUNKS + NT - 1) / NT;
-};
-
-// LDS fragment order.  A: fragment (tile t of 16 rows, k-step ks of 64 codes) is 1 KiB; lane L holds
-// the 16 code bytes of row 16t + L%16, code group 4ks + L/16.  B: fragment (tile t of 16 columns,
-// ks) is 256 bytes; lane L holds the packed dword (16 codes) of column 16t + L%16, group 4ks + L/16.
-// Lane L's A and B operands therefore cover the same 16 codes, in the order the unpack produces.
-// Inside an A fragment lane L's 16 bytes sit at slot a_slot(L, ks): the low 4 bits are XORed with
-// the code group so that the staging stores (8 lanes per row, one row's 8 code groups) hit
-// distinct banks; the 64 lanes of a fragment read still form a permutation of its 64 slots.
-__device__ __forceinline__ int a_slot(int lane, int ks) {
-  return ((lane & 15) ^ (4 * (lane >> 4)) ^ (2 * ks)) + 16 * (lane >> 4);
-}
-__device__ __forceinline__ int a_frag_off(int r, int kg) {
-  return (((r >> 4) * 2 + (kg >> 2)) << 10) + (a_slot((r & 15) + 16 * (kg & 3), kg >> 2) << 4);
-}
-// B stays in its global order in LDS: column n of the tile owns 32 bytes (the 128 codes of the K
-// tile), its two 16-byte halves swapped on every other group of 8 columns so that a fragment read
-// (16 columns x 4 dwords) covers 64 distinct banks.
-__device__ __forceinline__ int b_col_off(int n, int half) { return n * 32 + 16 * (half ^ ((n >> 3) & 1)); }
-
-__device__ __forceinline__ v4i unpack_frag(uint32_t w) {
-  return v4i{static_cast<int>(unpack_u(w, 0)), static_cast<int>(unpack_u(w, 1)), static_cast<int>(unpack_u(w, 2)),
-             static_cast<int>(unpack_u(w, 3))};
-}
-
-template <class C>
-__device__ __forceinline__ void gemm_gload(const int8_t* const (&pa)[C::A_PT], const uint8_t* const (&pb)[C::B_PT],
-                                           const bool (&vb)[C::B_PT], int64_t k0, v4i (&ra)[C::A_PT],
-                                           v4i (&rb)[C::B_PT]) {
-#pragma unroll
-  for (int p = 0; p < C::A_PT; ++p) ra[p] = *reinterpret_cast<const v4i*>(pa[p] + k0);
-#pragma unroll
-  for (int p = 0; p < C::B_PT; ++p)
-    if (vb[p]) rb[p] = *reinterpret_cast<const v4i*>(pb[p] + k0 / 4);
-}
-
-template <class C>
-__device__ __forceinline__ void gemm_sstore(const int (&la)[C::A_PT], const int (&lb)[C::B_PT],
-                                            const bool (&vb)[C::B_PT], const v4i (&ra)[C::A_PT],
-                                            const v4i (&rb)[C::B_PT], char* stage) {
-#pragma unroll
-  for (int p = 0; p < C::A_PT; ++p) *reinterpret_cast<v4i*>(stage + la[p]) = ra[p];
-#pragma unroll
-  for (int p = 0; p < C::B_PT; ++p)
-    if (vb[p]) *reinterpret_cast<v4i*>(stage + lb[p]) = rb[p];
-}
-
-template <class C, int WN, int TM, int TN>
-__device__ __forceinline__ void mfma_mainloop(const LinearOperand& o, int64_t M, int64_t N, int64_t m0, int64_t n0,
-                                              int64_t Kp, v4i (&acc)[TM][TN], char* smem) {
-  const int t = threadIdx.x;
-  __builtin_assume(t < C::NT);
-  const int lane = t & 63, w = t >> 6;
-  const int wm = w / WN, wn = w % WN;
-  constexpr bool kAllB = (C::B_CHUNKS % C::NT) == 0;
-
-  // per-chunk global sources and LDS destinations; rows past M / columns past N read the last
-  // valid one and only feed accumulator entries that are never stored
-  const int8_t* pa[C::A_PT];
-  int la[C::A_PT];
-#pragma unroll
-  for (int p = 0; p < C::A_PT; ++p) {
-    const int c = t + p * C::NT;
-    const int64_t m = m0 + (c >> 3);
-    pa[p] = o.q + (m < M ? m : M - 1) * o.ldq + 16 * (c & 7);
-    la[p] = a_frag_off(c >> 3, c & 7);
-  }
-  const uint8_t* pb[C::B_PT];
-  int lb[C::B_PT];
-  bool vb[C::B_PT];
-#pragma unroll
-  for (int p = 0; p < C::B_PT; ++p) {
-    const int c = t + p * C::NT;
-    vb[p] = kAllB || c < C::B_CHUNKS;
-    const int64_t n = n0 + (c >> 1);
-    pb[p] = o.w + (n < N ? n : N - 1) * o.ldw + 16 * (c & 1);
-    lb[p] = C::A_BYTES + b_col_off(c >> 1, c & 1);
-  }
-  const int64_t nk = Kp / C::BK;
-  const int aoff0 = a_slot(lane, 0) * 16, aoff1 = a_slot(lane, 1) * 16;
-  // one 128-deep K tile from an LDS stage
-  auto compute = [&](const char* cur) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      v4i af[TM];
-      uint32_t bw[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        af[i] = *reinterpret_cast<const v4i*>(cur + (((wm * TM + i) * 2 + ks) << 10) + (ks ? aoff1 : aoff0));
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        bw[j] = *reinterpret_cast<const uint32_t*>(cur + C::A_BYTES + b_col_off((wn * TN + j) * 16 + (lane & 15), ks) +
-                                                   4 * (lane >> 4));
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const v4i bf = unpack_frag(bw[j]);
-        // weights as the MFMA's A operand: the accumulator comes out transposed, so each lane holds
-        // 4 consecutive output columns of one row (vector stores in the epilogue)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf, af[i], acc[i][j], 0, 0, 0);
-      }
-    }
-  };
-  // Two register sets keep two K tiles of global loads in flight beyond the one in LDS: set 0
-  // holds even tiles, set 1 odd tiles; loads past the last tile re-read it (never computed).
-  v4i ra0[C::A_PT], rb0[C::B_PT], ra1[C::A_PT], rb1[C::B_PT];
-  auto kofs = [&](int64_t kt) { return (kt < nk ? kt : nk - 1) * C::BK; };
-  char* const s0 = smem;
-  char* const s1 = smem + C::STAGE;
-  gemm_gload<C>(pa, pb, vb, kofs(0), ra0, rb0);
-  gemm_gload<C>(pa, pb, vb, kofs(1), ra1, rb1);
-  gemm_sstore<C>(la, lb, vb, ra0, rb0, s0);
-  __syncthreads();
-  gemm_gload<C>(pa, pb, vb, kofs(2), ra0, rb0);
-  int64_t kt = 0;
-  for (; kt + 2 <= nk; kt += 2) {
-    compute(s0);                                     // tile kt
-    gemm_sstore<C>(la, lb, vb, ra1, rb1, s1);        // tile kt + 1
-    __syncthreads();
-    gemm_gload<C>(pa, pb, vb, kofs(kt + 3), ra1, rb1);
-    compute(s1);                                     // tile kt + 1
-    gemm_sstore<C>(la, lb, vb, ra0, rb0, s0);        // tile kt + 2 (past the end: never computed)
-    __syncthreads();
-    gemm_gload<C>(pa, pb, vb, kofs(kt + 4), ra0, rb0);
-  }
-  if (kt < nk) compute(s0);                          // odd number of K tiles
-  __syncthreads();  // the stages may be refilled by a following main loop (output-gate products)
-}
-
-// Tile order for a 1-D grid: workgroups are handed to the 8 XCDs round-robin by id, so id is
-// mapped to a tile such that each XCD gets a contiguous run of tiles (row-major over
-// (M tile, N tile)); consecutive tiles of one XCD share A rows in that XCD's L2.
-__device__ __forceinline__ void xcd_tile_of(int64_t pid, int64_t ntm, int64_t ntn, int64_t& tm, int64_t& tn) {
-  constexpr int64_t kXcd = 8;
-  const int64_t total = ntm * ntn;
-  const int64_t x = pid % kXcd, i = pid / kXcd;
-  const int64_t q = total / kXcd, r = total % kXcd;
-  const int64_t tile = x * q + (x < r ? x : r) + i;
-  // groups of kGroupM M-tile rows with M fastest: the tiles an XCD runs at once cover a few M rows
-  // and N columns, so both operands' K slabs are shared through its L2
-  constexpr int64_t kGroupM = 8;
-  const int64_t g = tile / (kGroupM * ntn);
-  const int64_t first_m = g * kGroupM;
-  const int64_t gsz = ntm - first_m < kGroupM ? ntm - first_m : kGroupM;
-  const int64_t local = tile - g * kGroupM * ntn;
-  tm = first_m + local % gsz;
-  tn = local / gsz;
-}
-__device__ __forceinline__ void xcd_tile(int64_t ntm, int64_t ntn, int64_t& tm, int64_t& tn) {
-  xcd_tile_of(blockIdx.x, ntm, ntn, tm, tn);
-}
-
-// With the weights as the A operand, element r of lane L's accumulator is output row L%16 and
-// output column 4*(L/16) + r of the 16 x 16 tile.
-template <int OUT_DT>
-__device__ __forceinline__ void store4(void* out, int64_t idx, const float (&v)[4], bool vec) {
-  if (vec) {
-    if constexpr (OUT_DT == kBF16) {
-      const uint32_t lo = pack_bf16x2(v[0], v[1]);
-      const uint32_t hi = pack_bf16x2(v[2], v[3]);
-      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + idx) = make_uint2(lo, hi);
-    } else {
-      *reinterpret_cast<float4*>(static_cast<float*>(out) + idx) = make_float4(v[0], v[1], v[2], v[3]);
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) st<OUT_DT>(out, idx + r, v[r]);
-  }
-}
-
-template <int DT>
-__device__ __forceinline__ void load4(const void* p, int64_t idx, bool vec, float (&v)[4]) {
-  if (vec) {
-    if constexpr (DT == kBF16) {
-      const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p) + idx);
-      v[0] = __uint_as_float(w.x << 16);
-      v[1] = __uint_as_float(w.x & 0xffff0000u);
-      v[2] = __uint_as_float(w.y << 16);
-      v[3] = __uint_as_float(w.y & 0xffff0000u);
-    } else {
-      const float4 f = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + idx);
-      v[0] = f.x;
-      v[1] = f.y;
-      v[2] = f.z;
-      v[3] = f.w;
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = ld<DT>(p, idx + r);
-  }
-}
-
-// 4-element vector access at element (m * ld + n) is aligned for every m and every n % 4 == 0.
-template <int DT>
-__device__ __forceinline__ bool vec4_ok(const void* p, int64_t ld) {
-  constexpr int64_t bytes = DT == kBF16 ? 8 : 16;
-  return (reinterpret_cast<uintptr_t>(p) % bytes) == 0 && (ld * (DT == kBF16 ? 2 : 4)) % bytes == 0;
-}
-
-// Two-product epilogues on the rounded products p0 = rnd(v0), p1 = rnd(v1):
-//   output gate  y = rnd(rnd(local + rnd(sigmoid(gate) * p0)) + p1)      (tesm.py:1256-1261)
-//   SwiGLU       h = rnd(rnd(silu(p0)) * p1), silu(x) = x * sigmoid(x)  (mixer_seq_simple.py:63-64)
-template <int EPI, int OUT_DT>
-__device__ __forceinline__ float dual_epi(float p0, float p1, float local, float gate) {
-  if constexpr (EPI == kEpiOutputGate) {
-    const float g = rnd<OUT_DT>(sigmoidf_(gate));
-    return rnd<OUT_DT>(rnd<OUT_DT>(local + rnd<OUT_DT>(g * p0)) + p1);
-  } else {
-    return rnd<OUT_DT>(rnd<OUT_DT>(p0 * sigmoidf_(p0)) * p1);
-  }
-}
-
-// kEpiGates: the region of the 32-column tile that starts at column n (0: stored as is, 1: tanh,
-// 2: biased sigmoid, 3: sigmoid).  act_n0 and act_w are multiples of 32, so a tile lies in one region
-// and the region is uniform over the wave.
-__device__ __forceinline__ int gate_region(const LinearArgs& a, int64_t n) {
-  const int64_t r = n - a.act_n0;
-  return r < 0 ? 0 : r < a.act_w ? 1 : r < 2 * a.act_w ? 2 : r < 3 * a.act_w ? 3 : 0;
-}
-
-// The MIMO gates on four consecutive columns n .. n + 3 of one region (tesm_mimo.py:958-961), each
-// on the product rounded to the output dtype: the float ops a scan would apply to the stored
-// products, so the values it reads are the ones it would have computed.
-template <int DT>
-__device__ __forceinline__ void gate_act4(const LinearArgs& a, int kind, int64_t n, float (&v)[4]) {
-  if (kind == 1) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = rnd<DT>(tanhf_(rnd<DT>(v[r])));
-  } else if (kind == 2) {
-    const int64_t c = n - a.act_n0 - a.act_w;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = rnd<DT>(sigmoidf_(rnd<DT>(rnd<DT>(v[r]) + ld<DT>(a.act_bias, c + r))));
-  } else if (kind == 3) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = rnd<DT>(sigmoidf_(rnd<DT>(v[r])));
-  }
-}
-
 // General epilogue of the 16 x 16 tiles of one wave (tile rows wm*TM.., columns wn*TN..): scale the
 // exact accumulators, optional bias / accumulator dump, or the output gate
 // y = local + sigmoid(gate) * state_proj + ent_proj in the module dtype's op order.
@@ -515,132 +262,6 @@ __device__ __forceinline__ void epilogue16_pre(const LinearArgs& a, const v4i (&
       }
     }
   }
-}
-
-template <int TM, int TN, int EPI, int OUT_DT>
-__device__ __forceinline__ void epilogue16(const LinearArgs& a, const v4i (&acc0)[TM][TN], const v4i (&acc1)[TM][TN],
-                                           int64_t m0, int64_t n0, int wm, int wn, int lane) {
-  const LinearOperand& o0 = a.op[0];
-  const LinearOperand& o1 = a.op[1];
-  const bool vout = vec4_ok<OUT_DT>(a.out, a.ldo);
-  bool vin = false;
-  if constexpr (EPI == kEpiOutputGate) vin = vec4_ok<OUT_DT>(a.local, a.ld_local) && vec4_ok<OUT_DT>(a.gate, a.ld_gate);
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int64_t m = m0 + (wm * TM + i) * 16 + (lane & 15);
-    if (m >= a.M) continue;
-    const float inv0 = 1.0f / o0.s_x[m];
-    const int32_t rs0 = o0.rowsum[m];
-    float inv1 = 0.0f;
-    int32_t rs1 = 0;
-    if constexpr (epi_dual(EPI)) {
-      inv1 = 1.0f / o1.s_x[m];
-      rs1 = o1.rowsum[m];
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int64_t nb = n0 + (wn * TN + j) * 16 + 4 * (lane >> 4);
-      if (nb >= a.N) continue;
-      const bool full = nb + 3 < a.N;
-      float v[4], lo[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if constexpr (EPI == kEpiOutputGate) {
-        if (full) {
-          load4<OUT_DT>(a.local, m * a.ld_local + nb, vin, lo);
-          load4<OUT_DT>(a.gate, m * a.ld_gate + nb, vin, gt);
-        } else {
-          for (int r = 0; r < 4; ++r) {
-            lo[r] = nb + r < a.N ? ld<OUT_DT>(a.local, m * a.ld_local + nb + r) : 0.0f;
-            gt[r] = nb + r < a.N ? ld<OUT_DT>(a.gate, m * a.ld_gate + nb + r) : 0.0f;
-          }
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t n = nb + r;
-        v[r] = 0.0f;
-        if (n >= a.N) continue;
-        const float cw0 = o0.c_w_per_row ? o0.c_w[n] : o0.c_w[0];
-        const int32_t a0 = acc0[i][j][r] - rs0;
-        if (a.acc_dump) a.acc_dump[m * a.N + n] = a0;
-        const float v0 = (static_cast<float>(a0) * inv0) * cw0;
-        if constexpr (EPI == kEpiStore) {
-          v[r] = a.bias ? v0 + ld<OUT_DT>(a.bias, n) : v0;
-        } else {
-          const float cw1 = o1.c_w_per_row ? o1.c_w[n] : o1.c_w[0];
-          const float v1 = rnd<OUT_DT>((static_cast<float>(acc1[i][j][r] - rs1) * inv1) * cw1);
-          v[r] = dual_epi<EPI, OUT_DT>(rnd<OUT_DT>(v0), v1, lo[r], gt[r]);
-        }
-      }
-      if (full) {
-        store4<OUT_DT>(a.out, m * a.ldo + nb, v, vout);
-      } else {
-        for (int r = 0; r < 4 && nb + r < a.N; ++r) st<OUT_DT>(a.out, m * a.ldo + nb + r, v[r]);
-      }
-    }
-  }
-}
-
-template <int WM, int WN, int TM, int TN, int EPI, int OUT_DT>
-__global__ __launch_bounds__(WM* WN * 64) void mfma_kernel(LinearArgs a) {
-  using C = Cfg<WM, WN, TM, TN>;
-  __shared__ __attribute__((aligned(16))) char smem[2 * C::STAGE];
-  int64_t tm, tn;
-  xcd_tile((a.M + C::BM - 1) / C::BM, (a.N + C::BN - 1) / C::BN, tm, tn);
-  const int64_t m0 = tm * C::BM;
-  const int64_t n0 = tn * C::BN;
-  v4i acc0[TM][TN], acc1[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      acc0[i][j] = v4i{0, 0, 0, 0};
-      acc1[i][j] = v4i{0, 0, 0, 0};
-    }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w / WN, wn = w % WN;
-  const LinearOperand& o0 = a.op[0];
-  // plain products (one scalar c_w, no bias, no accumulator dump) take the short epilogue, whose
-  // per-row operands are requested before the main loop
-  const bool plain = EPI == kEpiStore && !o0.c_w_per_row && !a.bias && !a.acc_dump;
-  float sx[TM];
-  int32_t rsum[TM];
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int64_t m = m0 + (wm * TM + i) * 16 + (lane & 15);
-    const int64_t mc = m < a.M ? m : a.M - 1;
-    sx[i] = o0.s_x[mc];
-    rsum[i] = o0.rowsum[mc];
-  }
-  const float cws = o0.c_w[0];
-  mfma_mainloop<C, WN, TM, TN>(a.op[0], a.M, a.N, m0, n0, a.Kp, acc0, smem);
-  if constexpr (epi_dual(EPI)) mfma_mainloop<C, WN, TM, TN>(a.op[1], a.M, a.N, m0, n0, a.Kp, acc1, smem);
-
-  if (plain) {
-    const int nrem = static_cast<int>(std::min<int64_t>(a.N - n0, C::BN));  // columns of this tile
-    const bool vout = vec4_ok<OUT_DT>(a.out, a.ldo);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int64_t m = m0 + (wm * TM + i) * 16 + (lane & 15);
-      if (m >= a.M) continue;
-      const float inv = 1.0f / sx[i];
-      char* orow = static_cast<char*>(a.out) + (m * a.ldo + n0) * (OUT_DT == kBF16 ? 2 : 4);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int nb = (wn * TN + j) * 16 + 4 * (lane >> 4);  // within the tile
-        if (nb >= nrem) continue;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = (static_cast<float>(acc0[i][j][r] - rsum[i]) * inv) * cws;
-        if (vout && nb + 4 <= nrem) {
-          store4<OUT_DT>(orow, nb, v, true);
-        } else {
-          for (int r = 0; r < 4 && nb + r < nrem; ++r) st<OUT_DT>(orow, nb + r, v[r]);
-        }
-      }
-    }
-    return;
-  }
-  epilogue16<TM, TN, EPI, OUT_DT>(a, acc0, acc1, m0, n0, wm, wn, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -859,531 +480,6 @@ __global__ __launch_bounds__(NW * 64) void skinny_fq_kernel(LinearArgs a, FusedQ
   b.op[0].s_x = sc_l - m0;
   b.op[0].rowsum = rs_l - m0;
   skinny_body<NW, TM, TN, kEpiStore, OUT_DT>(b, m0, n0);
-}
-
-// ---------------------------------------------------------------------------
-// GEMM on v_mfma_i32_32x32x32_i8, which on gfx950 delivers about twice the int8 rate of the
-// 16x16x64 form.  Block tile BM x BN (waves WM x WN, each TM x TN tiles of 32 x 32), K tiles of
-// 128 codes = 8 chunks of 16 codes in 4 k-steps.  Weights are the MFMA's A operand: in k-step s,
-// lane L feeds weight column L%32 with chunk 4*(L/32) + s (one packed dword, unpacked in registers)
-// and activation row L%32 with the same chunk (16 bytes); any pairing of chunks to k-steps gives the
-// same sums as long as both operands use it, and this one makes a lane's four weight dwords of a K
-// tile one contiguous 16-byte read.  Accumulator element r of lane L is weight column
-// 8*(r/4) + 4*(L/32) + r%4 and activation row L%32, so every lane stores runs of 4 consecutive
-// outputs.
-//
-// LDS, per stage (bank model measured on the device: 16-byte reads are served 16 lanes per pass over
-// 256 bytes, 16-byte writes 8 lanes per pass over 128 bytes): activations in chunk planes
-// [q][row][16 bytes] with row slot row ^ q, so a fragment read (16 consecutive rows, one chunk) and
-// a staging store (8 chunks of one row) both hit distinct banks; packed weights [col][half][16 bytes]
-// with the halves swapped on odd groups of 8 columns, so a fragment read (16 columns, one half)
-// covers all banks and a staging store (4 columns x 2 halves) 128 contiguous bytes.
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
-
-template <int WM, int WN, int TM, int TN>
-struct Cfg32 {
-  static constexpr int NT = WM * WN * 64;
-  static constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 128;
-  static constexpr int A_BYTES = BM * BK;
-  static constexpr int B_BYTES = BN * BK / 4;
-  static constexpr int STAGE = A_BYTES + B_BYTES;
-  static constexpr int A_CHUNKS = BM * BK / 16;
-  static constexpr int B_CHUNKS = BN * BK / 64;
-  static constexpr int A_PT = (A_CHUNKS + NT - 1) / NT;
-  static constexpr int B_PT = (B_CHUNKS + NT - 1) / NT;
-};
-
-template <int BM>
-__device__ __forceinline__ int a32_off(int row, int q) { return q * BM * 16 + (row ^ q) * 16; }
-__device__ __forceinline__ int b32_off(int col, int h) { return col * 32 + 16 * (h ^ ((col >> 3) & 1)); }
-
-template <class C, int WN, int TM, int TN>
-__device__ __forceinline__ void mfma32_mainloop(const LinearOperand& o, int64_t M, int64_t N, int64_t m0, int64_t n0,
-                                                int64_t Kp, v16i (&acc)[TM][TN], char* smem) {
-  const int t = threadIdx.x;
-  __builtin_assume(t < C::NT);
-  const int lane = t & 63, w = t >> 6;
-  const int wm = w / WN, wn = w % WN;
-  constexpr bool kAllA = (C::A_CHUNKS % C::NT) == 0;
-  constexpr bool kAllB = (C::B_CHUNKS % C::NT) == 0;
-  static_assert(kAllA, "A chunks must divide evenly over the workgroup");
-
-  // rows past M / columns past N read the last valid one and only feed outputs never stored
-  const int8_t* pa[C::A_PT];
-  int la[C::A_PT];
-#pragma unroll
-  for (int p = 0; p < C::A_PT; ++p) {
-    const int c = t + p * C::NT;
-    const int64_t m = m0 + (c >> 3);
-    pa[p] = o.q + (m < M ? m : M - 1) * o.ldq + 16 * (c & 7);
-    la[p] = a32_off<C::BM>(c >> 3, c & 7);
-  }
-  const uint8_t* pb[C::B_PT];
-  int lb[C::B_PT];
-  bool vb[C::B_PT];
-#pragma unroll
-  for (int p = 0; p < C::B_PT; ++p) {
-    const int c = t + p * C::NT;
-    vb[p] = kAllB || c < C::B_CHUNKS;
-    const int64_t n = n0 + (c >> 1);
-    pb[p] = o.w + (n < N ? n : N - 1) * o.ldw + 16 * (c & 1);
-    lb[p] = C::A_BYTES + b32_off(c >> 1, c & 1);
-  }
-  const int64_t nk = Kp / C::BK;
-  auto gload = [&](int64_t kt, v4i (&ra)[C::A_PT], v4i (&rb)[C::B_PT]) {
-    const int64_t k0 = (kt < nk ? kt : nk - 1) * C::BK;
-#pragma unroll
-    for (int p = 0; p < C::A_PT; ++p) ra[p] = *reinterpret_cast<const v4i*>(pa[p] + k0);
-#pragma unroll
-    for (int p = 0; p < C::B_PT; ++p)
-      if (vb[p]) rb[p] = *reinterpret_cast<const v4i*>(pb[p] + k0 / 4);
-  };
-  auto sstore = [&](const v4i (&ra)[C::A_PT], const v4i (&rb)[C::B_PT], char* stage) {
-#pragma unroll
-    for (int p = 0; p < C::A_PT; ++p) *reinterpret_cast<v4i*>(stage + la[p]) = ra[p];
-#pragma unroll
-    for (int p = 0; p < C::B_PT; ++p)
-      if (vb[p]) *reinterpret_cast<v4i*>(stage + lb[p]) = rb[p];
-  };
-  // per-lane fragment offsets: chunk 4*(lane/32) + s of the lane's row / column
-  const int hq = 4 * (lane >> 5);
-  int ar[4][TM];
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
-#pragma unroll
-    for (int i = 0; i < TM; ++i) ar[s][i] = a32_off<C::BM>((wm * TM + i) * 32 + (lane & 31), hq + s);
-  int br[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) br[j] = C::A_BYTES + b32_off((wn * TN + j) * 32 + (lane & 31), lane >> 5);
-  auto compute = [&](const char* cur) {
-    v4i bw[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bw[j] = *reinterpret_cast<const v4i*>(cur + br[j]);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      v4i af[TM];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = *reinterpret_cast<const v4i*>(cur + ar[s][i]);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const v4i bf = unpack_frag(static_cast<uint32_t>(bw[j][s]));
-#pragma unroll
-        for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[i], acc[i][j], 0, 0, 0);
-      }
-    }
-  };
-  // two register sets keep two K tiles of loads in flight beyond the one in LDS
-  v4i ra0[C::A_PT], rb0[C::B_PT], ra1[C::A_PT], rb1[C::B_PT];
-  char* const s0 = smem;
-  char* const s1 = smem + C::STAGE;
-  gload(0, ra0, rb0);
-  gload(1, ra1, rb1);
-  sstore(ra0, rb0, s0);
-  __syncthreads();
-  gload(2, ra0, rb0);
-  int64_t kt = 0;
-  for (; kt + 2 <= nk; kt += 2) {
-    compute(s0);
-    sstore(ra1, rb1, s1);
-    __syncthreads();
-    gload(kt + 3, ra1, rb1);
-    compute(s1);
-    sstore(ra0, rb0, s0);
-    __syncthreads();
-    gload(kt + 4, ra0, rb0);
-  }
-  if (kt < nk) compute(s0);
-  __syncthreads();
-}
-
-// Main loop with direct-to-LDS loads (global_load_lds_dwordx4): NS stages in LDS, no staging
-// registers.  One such instruction moves 64 lanes x 16 bytes into 1 KB of LDS in lane order, so the
-// layouts are chosen through the lanes' global addresses: activation rows in blocks of 8 rows x 8
-// chunks (a row's 8 lanes read one 128-byte line, chunk q of row r lands in slot
-// r*8 + (q ^ ((r/2) % 8))), weights in blocks of 32 columns x 2 halves (half h of column n in slot
-// 2n + (h ^ ((n/8) % 2))); both make the fragment reads (16 lanes: consecutive rows or columns, one
-// chunk) hit 16 distinct 16-byte slots of 256 bytes.  Each wave issues D of these per K tile (with two
-// stages the last blocks may leave some waves one short); the wait for tile kt is "at most (NS - 2) *
-// D outstanding" (loads past the last K tile re-read it, so the count never shrinks), then one
-// barrier, then the refill of the stage the previous tile used.
-template <int BM>
-__device__ __forceinline__ int a32d_off(int row, int q) { return 16 * (row * 8 + (q ^ ((row >> 1) & 7))); }
-__device__ __forceinline__ int b32d_off(int col, int h) { return 16 * (col * 2 + (h ^ ((col >> 3) & 1))); }
-
-__device__ __forceinline__ void lds_dma16(const void* src, char* dst) {
-  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(dst), 16, 0, 0);
-}
-
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding: vmcnt bits [3:0] and
-// [15:14], expcnt [6:4] and lgkmcnt [11:8] left at their maxima)
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt out of range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
-}
-
-template <class C, int WN, int TM, int TN, int NS>
-__device__ __forceinline__ void mfma32d_mainloop(const LinearOperand& o, int64_t M, int64_t N, int64_t m0, int64_t n0,
-                                                 int64_t Kp, v16i (&acc)[TM][TN], char* smem) {
-  constexpr int NW = C::NT / 64;
-  constexpr int NA = C::BM / 8, NB = C::BN / 32;  // 1 KB blocks per K tile
-  // deeper pipelines count each wave's loads in flight, so they need the same number per wave; two
-  // stages wait for all of a wave's loads, so the last blocks may leave some waves one short
-  static_assert(NS == 2 || (NA + NB) % NW == 0, "DMA blocks must divide evenly over the waves");
-  constexpr int D = (NA + NB + NW - 1) / NW;
-  static_assert((NS - 2) * D < 64, "too many loads in flight for vmcnt");
-  const int t = threadIdx.x;
-  __builtin_assume(t < C::NT);
-  const int lane = t & 63, w = t >> 6;
-  const int wm = w / WN, wn = w % WN;
-  // this lane's source of each of the wave's D blocks (rows / columns past M / N read the last one)
-  const char* src[D];
-  int dst[D], adv[D];
-#pragma unroll
-  for (int i = 0; i < D; ++i) {
-    const int blk = w + i * NW < NA + NB ? w + i * NW : NA + NB - 1;  // (blocks past the end are never issued)
-    if (blk < NA) {
-      const int row = blk * 8 + (lane >> 3);
-      const int q = (lane & 7) ^ ((row >> 1) & 7);
-      const int64_t m = m0 + row;
-      src[i] = reinterpret_cast<const char*>(o.q) + (m < M ? m : M - 1) * o.ldq + 16 * q;
-      dst[i] = blk * 1024;
-      adv[i] = C::BK;
-    } else {
-      const int col = (blk - NA) * 32 + (lane >> 1);
-      const int h = (lane & 1) ^ ((col >> 3) & 1);
-      const int64_t n = n0 + col;
-      src[i] = reinterpret_cast<const char*>(o.w) + (n < N ? n : N - 1) * o.ldw + 16 * h;
-      dst[i] = C::A_BYTES + (blk - NA) * 1024;
-      adv[i] = C::BK / 4;
-    }
-  }
-  const int64_t nk = Kp / C::BK;
-  auto issue = [&](int64_t kt) {
-    const int64_t k = kt < nk ? kt : nk - 1;
-    char* stage = smem + static_cast<int>(kt % NS) * C::STAGE;
-#pragma unroll
-    for (int i = 0; i < D; ++i)
-      if ((NA + NB) % NW == 0 || __builtin_amdgcn_readfirstlane(w) + i * NW < NA + NB)  // wave-uniform
-        lds_dma16(src[i] + k * adv[i], stage + dst[i]);
-  };
-  const int hq = 4 * (lane >> 5);
-  int ar[4][TM], br[TN];
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
-#pragma unroll
-    for (int i = 0; i < TM; ++i) ar[s][i] = a32d_off<C::BM>((wm * TM + i) * 32 + (lane & 31), hq + s);
-#pragma unroll
-  for (int j = 0; j < TN; ++j) br[j] = C::A_BYTES + b32d_off((wn * TN + j) * 32 + (lane & 31), lane >> 5);
-  // fragments double-buffered by one k-step: the reads for step s + 1 are issued before the MFMAs
-  // of step s (scheduling barriers keep the compiler from sinking them), so their latency hides
-  // behind TM x TN MFMAs instead of one
-  auto compute = [&](const char* cur) {
-    v4i bw[TN], af[2][TM];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bw[j] = *reinterpret_cast<const v4i*>(cur + br[j]);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) af[0][i] = *reinterpret_cast<const v4i*>(cur + ar[0][i]);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (s < 3) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) af[(s + 1) & 1][i] = *reinterpret_cast<const v4i*>(cur + ar[s + 1][i]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const v4i bf = unpack_frag(static_cast<uint32_t>(bw[j][s]));
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[s & 1][i], acc[i][j], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  __syncthreads();  // the stages may still be read by a previous main loop or epilogue
-#pragma unroll
-  for (int g = 0; g < NS - 1; ++g) issue(g);
-  for (int64_t kt = 0; kt < nk; ++kt) {
-    wait_vmcnt<(NS - 2) * D>();  // this wave's loads of tile kt have landed
-    __builtin_amdgcn_s_barrier();  // ... every wave's, and every wave is done with tile kt - 1
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    issue(kt + NS - 1);           // into the stage tile kt - 1 used
-    compute(smem + static_cast<int>(kt % NS) * C::STAGE);
-  }
-  wait_vmcnt<0>();  // the re-reads past the last tile
-  __syncthreads();
-}
-
-// Plain epilogue staged through LDS.  The accumulator layout gives each lane 4 consecutive outputs
-// of one row, so direct stores cover 32 rows x 16 bytes per instruction; instead each wave writes
-// one 32-row slab of its (already scaled and rounded) outputs into a private LDS buffer and reads
-// it back as 16-byte row-contiguous chunks, so a store instruction covers whole row segments.
-// Output values are the same as the direct path's.  Needs a 16-byte aligned output and row pitch.
-// LDS bytes the staged epilogue of NWV waves needs with JU 32-column tiles per slab.
-template <int NWV, int JU, int OUT_DT>
-constexpr int epi32_bytes() {
-  return NWV * 32 * (JU * 32 * (OUT_DT == kBF16 ? 2 : 4) + 16);
-}
-
-template <int NWV, int TM, int TN, int OUT_DT, int AVAIL, bool GATES>
-__device__ __forceinline__ void epi32_plain_staged(const LinearArgs& a, const v16i (&acc)[TM][TN], const float (&sx)[TM],
-                                                   const int32_t (&rsum)[TM], float cws, int64_t m0, int64_t n0,
-                                                   int wm, int wn, char* smem) {
-  constexpr int ES = OUT_DT == kBF16 ? 2 : 4;
-  constexpr int JU = epi32_bytes<NWV, TN, OUT_DT>() <= AVAIL ? TN : 1;  // 32-col tiles per slab
-  constexpr int RB = JU * 32 * ES;   // bytes of one staged row
-  constexpr int PITCH = RB + 16;     // padded so the column-wise staging stores spread over the banks
-  constexpr int CPR = RB / 16;       // 16-byte chunks per row
-  constexpr int VPC = 16 / ES;       // outputs per chunk
-  static_assert(NWV * 32 * PITCH <= AVAIL, "staging buffers exceed the LDS given");
-  static_assert((32 * CPR) % 64 == 0, "chunks must divide over the wave");
-  const int lane = threadIdx.x & 63;
-  char* wb = smem + (threadIdx.x >> 6) * 32 * PITCH;
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const float inv = 1.0f / sx[i];
-    const int64_t mb = m0 + (wm * TM + i) * 32;
-#pragma unroll
-    for (int jb = 0; jb < TN; jb += JU) {
-      lds_barrier();  // the buffer's previous contents (or the last K tile) are consumed
-#pragma unroll
-      for (int jj = 0; jj < JU; ++jj) {
-        const int64_t nt = n0 + (wn * TN + jb + jj) * 32;  // the 32-column tile's first column
-        const int kind = GATES ? gate_region(a, nt) : 0;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (static_cast<float>(acc[i][jb + jj][4 * g + r] - rsum[i]) * inv) * cws;
-          if constexpr (GATES) gate_act4<OUT_DT>(a, kind, nt + 8 * g + 4 * (lane >> 5), v);
-          char* p = wb + (lane & 31) * PITCH + (jj * 32 + 8 * g + 4 * (lane >> 5)) * ES;
-          if constexpr (OUT_DT == kBF16)
-            *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-          else
-            *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-        }
-      }
-      lds_barrier();
-      const int64_t nb = n0 + (wn * TN + jb) * 32;
-#pragma unroll
-      for (int it = 0; it < 32 * CPR / 64; ++it) {
-        const int idx = it * 64 + lane;
-        const int row = idx / CPR, ch = idx % CPR;
-        const int64_t m = mb + row, n = nb + ch * VPC;
-        if (m >= a.M || n >= a.N) continue;
-        const uint4 d = *reinterpret_cast<const uint4*>(wb + row * PITCH + ch * 16);
-        char* dst = static_cast<char*>(a.out) + (m * a.ldo + n) * ES;
-        if (n + VPC <= a.N) {
-          *reinterpret_cast<uint4*>(dst) = d;
-        } else {
-          const uint32_t wd[4] = {d.x, d.y, d.z, d.w};
-          for (int e = 0; e < a.N - n; ++e) {
-            if constexpr (OUT_DT == kBF16)
-              reinterpret_cast<uint16_t*>(dst)[e] = static_cast<uint16_t>(wd[e >> 1] >> (16 * (e & 1)));
-            else
-              reinterpret_cast<uint32_t*>(dst)[e] = wd[e];
-          }
-        }
-      }
-    }
-  }
-}
-
-// NS == 0: register-staged main loop (two LDS stages); NS >= 2: direct-to-LDS loads into NS stages.
-// One output tile at (m0, n0); smem holds SMEM bytes (at least the tile's stages).
-template <int WM, int WN, int TM, int TN, int EPI, int OUT_DT, int NS, int SMEM>
-__device__ __forceinline__ void mfma32_tile(const LinearArgs& a, int64_t m0, int64_t n0, char* smem) {
-  using C = Cfg32<WM, WN, TM, TN>;
-  static_assert((NS == 0 ? 2 : NS) * C::STAGE <= SMEM, "tile stages exceed the LDS given");
-  v16i acc0[TM][TN], acc1[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      acc0[i][j] = v16i{};
-      acc1[i][j] = v16i{};
-    }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wm = w / WN, wn = w % WN;
-  const LinearOperand& o0 = a.op[0];
-  const LinearOperand& o1 = a.op[1];
-  const bool plain = (EPI == kEpiStore || EPI == kEpiGates) && !o0.c_w_per_row && !a.bias && !a.acc_dump;
-  float sx[TM], sx1[TM];
-  int32_t rsum[TM], rs1[TM];
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int64_t m = m0 + (wm * TM + i) * 32 + (lane & 31);
-    const int64_t mc = m < a.M ? m : a.M - 1;
-    sx[i] = o0.s_x[mc];
-    rsum[i] = o0.rowsum[mc];
-    if constexpr (epi_dual(EPI)) {
-      sx1[i] = o1.s_x[mc];
-      rs1[i] = o1.rowsum[mc];
-    }
-  }
-  const float cws = o0.c_w[0];
-  const float cws1 = epi_dual(EPI) ? o1.c_w[0] : 0.0f;
-  if constexpr (NS == 0) {
-    mfma32_mainloop<C, WN, TM, TN>(a.op[0], a.M, a.N, m0, n0, a.Kp, acc0, smem);
-    if constexpr (epi_dual(EPI)) mfma32_mainloop<C, WN, TM, TN>(a.op[1], a.M, a.N, m0, n0, a.Kp, acc1, smem);
-  } else {
-    mfma32d_mainloop<C, WN, TM, TN, NS>(a.op[0], a.M, a.N, m0, n0, a.Kp, acc0, smem);
-    if constexpr (epi_dual(EPI))
-      mfma32d_mainloop<C, WN, TM, TN, NS>(a.op[1], a.M, a.N, m0, n0, a.Kp, acc1, smem);
-  }
-
-  const bool vout = vec4_ok<OUT_DT>(a.out, a.ldo);
-  // the staged epilogue needs one 32-column slab per wave in the tile's LDS (else the direct stores)
-  if constexpr (epi32_bytes<WM * WN, 1, OUT_DT>() <= SMEM) {
-    if (plain && reinterpret_cast<uintptr_t>(a.out) % 16 == 0 && (a.ldo * (OUT_DT == kBF16 ? 2 : 4)) % 16 == 0) {
-      epi32_plain_staged<WM * WN, TM, TN, OUT_DT, SMEM, EPI == kEpiGates>(a, acc0, sx, rsum, cws, m0, n0, wm, wn,
-                                                                        smem);
-      return;
-    }
-  }
-  if (plain) {
-    const int nrem = static_cast<int>(std::min<int64_t>(a.N - n0, C::BN));
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int64_t m = m0 + (wm * TM + i) * 32 + (lane & 31);
-      if (m >= a.M) continue;
-      const float inv = 1.0f / sx[i];
-      char* orow = static_cast<char*>(a.out) + (m * a.ldo + n0) * (OUT_DT == kBF16 ? 2 : 4);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int kind = EPI == kEpiGates ? gate_region(a, n0 + (wn * TN + j) * 32) : 0;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int nb = (wn * TN + j) * 32 + 8 * g + 4 * (lane >> 5);
-          if (nb >= nrem) continue;
-          float v[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (static_cast<float>(acc0[i][j][4 * g + r] - rsum[i]) * inv) * cws;
-          if constexpr (EPI == kEpiGates) gate_act4<OUT_DT>(a, kind, n0 + nb, v);
-          if (vout && nb + 4 <= nrem) {
-            store4<OUT_DT>(orow, nb, v, true);
-          } else {
-            for (int r = 0; r < 4 && nb + r < nrem; ++r) st<OUT_DT>(orow, nb + r, v[r]);
-          }
-        }
-      }
-    }
-    return;
-  }
-  // Generic epilogue.  The output-gate inputs of one 32 x 32 tile (four groups of four columns per
-  // lane) are requested together in straight-line code (indices clamped into range, raw bits) before
-  // any is used, so the tile waits for memory once instead of once per group; second-operand row
-  // scales and sums and per-tensor weight scales were read before the K loop.
-  const bool vin = EPI == kEpiOutputGate && vec4_ok<OUT_DT>(a.local, a.ld_local) &&
-                   vec4_ok<OUT_DT>(a.gate, a.ld_gate) && a.N % 4 == 0;
-  constexpr int es = OUT_DT == kBF16 ? 2 : 4;
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int64_t m = m0 + (wm * TM + i) * 32 + (lane & 31), mc = m < a.M ? m : a.M - 1;
-    const float inv0 = 1.0f / sx[i];
-    const float inv1 = epi_dual(EPI) ? 1.0f / sx1[i] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      uint32_t lo[4][4], gt[4][4];
-      if constexpr (EPI == kEpiOutputGate) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int64_t nb = n0 + (wn * TN + j) * 32 + 8 * g + 4 * (lane >> 5);
-          if (vin) {  // whole groups of four: a group past N re-reads the last one
-            const int64_t nv = nb < a.N ? nb : a.N - 4;
-            const char* pl = static_cast<const char*>(a.local) + (mc * a.ld_local + nv) * es;
-            const char* pg = static_cast<const char*>(a.gate) + (mc * a.ld_gate + nv) * es;
-#pragma unroll
-            for (int q = 0; q < es / 2; ++q) {  // bf16: one 8-byte load, f32: two
-              const uint2 wl = reinterpret_cast<const uint2*>(pl)[q], wg = reinterpret_cast<const uint2*>(pg)[q];
-              lo[g][2 * q] = wl.x;
-              lo[g][2 * q + 1] = wl.y;
-              gt[g][2 * q] = wg.x;
-              gt[g][2 * q + 1] = wg.y;
-            }
-          } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              const int64_t n = nb + r < a.N ? nb + r : a.N - 1;
-              lo[g][r] = ld_bits<OUT_DT>(a.local, mc * a.ld_local + n);
-              gt[g][r] = ld_bits<OUT_DT>(a.gate, mc * a.ld_gate + n);
-            }
-          }
-        }
-      }
-      if (m >= a.M) continue;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int64_t nb = n0 + (wn * TN + j) * 32 + 8 * g + 4 * (lane >> 5);
-        if (nb >= a.N) continue;
-        float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t n = nb + r;
-          const float cw0 = o0.c_w_per_row ? o0.c_w[n < a.N ? n : a.N - 1] : cws;
-          const int32_t a0 = acc0[i][j][4 * g + r] - rsum[i];
-          if (a.acc_dump && n < a.N) a.acc_dump[m * a.N + n] = a0;
-          const float v0 = (static_cast<float>(a0) * inv0) * cw0;
-          if constexpr (!epi_dual(EPI)) {  // (kEpiGates is always plain)
-            v[r] = a.bias ? v0 + ld<OUT_DT>(a.bias, n < a.N ? n : a.N - 1) : v0;
-          } else {
-            const float cw1 = o1.c_w_per_row ? o1.c_w[n < a.N ? n : a.N - 1] : cws1;
-            const float v1 = rnd<OUT_DT>((static_cast<float>(acc1[i][j][4 * g + r] - rs1[i]) * inv1) * cw1);
-            float lv = 0.0f, gv = 0.0f;
-            if constexpr (EPI == kEpiOutputGate) {
-              if (vin && OUT_DT == kBF16) {
-                const uint32_t wl = lo[g][r >> 1], wg = gt[g][r >> 1];
-                lv = __uint_as_float(r & 1 ? wl & 0xffff0000u : wl << 16);
-                gv = __uint_as_float(r & 1 ? wg & 0xffff0000u : wg << 16);
-              } else {
-                lv = from_bits<OUT_DT>(lo[g][r]);
-                gv = from_bits<OUT_DT>(gt[g][r]);
-              }
-            }
-            v[r] = dual_epi<EPI, OUT_DT>(rnd<OUT_DT>(v0), v1, lv, gv);
-          }
-        }
-        if (nb + 3 < a.N) {
-          store4<OUT_DT>(a.out, m * a.ldo + nb, v, vout);
-        } else {
-          for (int r = 0; r < 4 && nb + r < a.N; ++r) st<OUT_DT>(a.out, m * a.ldo + nb + r, v[r]);
-        }
-      }
-    }
-  }
-}
-
-template <int WM, int WN, int TM, int TN, int EPI, int OUT_DT, int NS = 0>
-__global__ __launch_bounds__(WM* WN * 64) void mfma32_kernel(LinearArgs a) {
-  using C = Cfg32<WM, WN, TM, TN>;
-  constexpr int SMEM = (NS == 0 ? 2 : NS) * C::STAGE;
-  __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  int64_t tm, tn;
-  xcd_tile((a.M + C::BM - 1) / C::BM, (a.N + C::BN - 1) / C::BN, tm, tn);
-  mfma32_tile<WM, WN, TM, TN, EPI, OUT_DT, NS, SMEM>(a, tm * C::BM, tn * C::BN, smem);
-}
-
-// Plain product whose 128x256 tiles would run in more rounds than the CUs hold (the SISO in_proj, 640
-// tiles): columns [0, nA) in 128x256 tiles, two per CU, and the remaining N - nA columns in 128x128
-// tiles launched after them, so the last round runs half-size tiles on more CUs.  Both use two
-// direct-to-LDS stages and eight waves; TMB = 32-row MFMA tiles per wave of a tail tile (2: 128 rows).
-template <int OUT_DT, int TMB, int EPI>
-__global__ __launch_bounds__(512) void mfma32_split_kernel(LinearArgs a, int64_t nA) {
-  using CA = Cfg32<2, 4, 2, 2>;
-  using CB = Cfg32<2, 4, TMB, 1>;
-  constexpr int SMEM = 2 * (CA::STAGE > CB::STAGE ? CA::STAGE : CB::STAGE);
-  __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  const int64_t ntm = (a.M + CA::BM - 1) / CA::BM, ntnA = nA / CA::BN, tilesA = ntm * ntnA;
-  int64_t tm, tn;
-  if (static_cast<int64_t>(blockIdx.x) < tilesA) {
-    xcd_tile_of(blockIdx.x, ntm, ntnA, tm, tn);
-    mfma32_tile<2, 4, 2, 2, EPI, OUT_DT, 2, SMEM>(a, tm * CA::BM, tn * CA::BN, smem);
-  } else {
-    xcd_tile_of(blockIdx.x - tilesA, (a.M + CB::BM - 1) / CB::BM, (a.N - nA + CB::BN - 1) / CB::BN, tm, tn);
-    mfma32_tile<2, 4, TMB, 1, EPI, OUT_DT, 2, SMEM>(a, tm * CB::BM, nA + tn * CB::BN, smem);
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2359,26 +1455,10 @@ __global__ __launch_bounds__(NW * 64) void gate32_kernel(LinearArgs a, RowQuant 
   }
 }
 
-template <int WM, int WN, int TM, int TN, int EPI, int NS = 0>
-int run_mfma32(const LinearArgs& a, hipStream_t st) {
-  using C = Cfg32<WM, WN, TM, TN>;
-  const int64_t tiles = ((a.N + C::BN - 1) / C::BN) * ((a.M + C::BM - 1) / C::BM);
-  TESM_REQUIRE(tiles <= 0x7fffffff, kErrUnsupported, "bitlinear: too many tiles");
-  const unsigned grid = static_cast<unsigned>(tiles);
-  if (a.out_dt == kBF16)
-    mfma32_kernel<WM, WN, TM, TN, EPI, kBF16, NS><<<grid, C::NT, 0, TESM_LOGGED(st, mfma32_kernel<WM, WN, TM, TN, EPI, kBF16, NS>)>>>(a);
-  else
-    mfma32_kernel<WM, WN, TM, TN, EPI, kF32, NS><<<grid, C::NT, 0, TESM_LOGGED(st, mfma32_kernel<WM, WN, TM, TN, EPI, kF32, NS>)>>>(a);
-  return check_launch("bitlinear mfma32");
-}
-
-struct DeviceLimits {
-  int cus = 0;
-  int64_t lds = 0;
-};
-
 // Compute units and LDS bytes per workgroup of the current device (queried once per device).
-inline DeviceLimits device_limits() {
+}  // namespace
+
+DeviceLimits device_limits() {
   static DeviceLimits cache[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return DeviceLimits{};
@@ -2394,6 +1474,8 @@ inline DeviceLimits device_limits() {
   return d;
 }
 
+namespace {
+
 template <int NW, int TM, int TN, int EPI>
 int run_skinny(const LinearArgs& a, hipStream_t st) {
   const int64_t tiles = ((a.M + 16 * TM - 1) / (16 * TM)) * ((a.N + 16 * TN - 1) / (16 * TN));
@@ -2403,19 +1485,6 @@ int run_skinny(const LinearArgs& a, hipStream_t st) {
   else
     skinny_kernel<NW, TM, TN, EPI, kF32><<<static_cast<unsigned>(tiles), NW * 64, 0, TESM_LOGGED(st, skinny_kernel<NW, TM, TN, EPI, kF32>)>>>(a);
   return check_launch("bitlinear skinny");
-}
-
-template <int WM, int WN, int TM, int TN, int EPI>
-int run_mfma(const LinearArgs& a, hipStream_t st) {
-  using C = Cfg<WM, WN, TM, TN>;
-  const int64_t tiles = ((a.N + C::BN - 1) / C::BN) * ((a.M + C::BM - 1) / C::BM);
-  TESM_REQUIRE(tiles <= 0x7fffffff, kErrUnsupported, "bitlinear: too many tiles");
-  const unsigned grid = static_cast<unsigned>(tiles);
-  if (a.out_dt == kBF16)
-    mfma_kernel<WM, WN, TM, TN, EPI, kBF16><<<grid, C::NT, 0, TESM_LOGGED(st, mfma_kernel<WM, WN, TM, TN, EPI, kBF16>)>>>(a);
-  else
-    mfma_kernel<WM, WN, TM, TN, EPI, kF32><<<grid, C::NT, 0, TESM_LOGGED(st, mfma_kernel<WM, WN, TM, TN, EPI, kF32>)>>>(a);
-  return check_launch("bitlinear mfma");
 }
 
 inline bool host_vec4_ok(const void* p, int64_t ld, int dt) {
@@ -2557,19 +1626,6 @@ int check_operand(const LinearOperand& o, int64_t Kp, const char* which) {
 
 }  // namespace
 
-// Two-product epilogues: split-K for decode-size batches, else the 32x32 kernels as for plain products.
-template <int EPI>
-int dispatch_dual(const LinearArgs& a, hipStream_t st) {
-  if (a.M <= 16) return run_skinny<4, 1, 1, EPI>(a, st);
-  if (a.M <= 32) return run_skinny<4, 2, 1, EPI>(a, st);
-  const int64_t tiles256 = ((a.M + 127) / 128) * ((a.N + 255) / 256);
-  // long K on many tiles (the MIMO output gate, K 2 x 8192): two direct-to-LDS stages, 694 us vs 766 us
-  // with three at M 8192
-  if (a.N % 256 == 0 && tiles256 >= 2048 && a.Kp >= 2048) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
-  if (a.N % 256 == 0 && tiles256 >= 128) return run_mfma32<2, 4, 2, 2, EPI>(a, st);
-  return run_mfma32<1, 4, 2, 1, EPI>(a, st);
-}
-
 // Waves of a fused-quantization workgroup (16 waves, four per SIMD, were measured no faster at the
 // decode shapes: the quantization phase is bound by its dependent load / reduction / LDS steps).
 constexpr int kFqNW = 4;
@@ -2645,50 +1701,6 @@ int launch_linear_fq(const LinearArgs& a, const FusedQuantIn& f, hipStream_t st)
   return check_launch("bitlinear skinny (fused quant)");
 }
 
-// Store-epilogue products of more than 32 rows on the 32x32x32 MFMA kernels (EPI kEpiStore or
-// kEpiGates).
-template <int EPI>
-int dispatch_store32(const LinearArgs& a, hipStream_t st) {
-  // 32x32x32 MFMA kernels: 128x256 tiles (8 waves of 64x64) when N fills them and there are
-  // enough of them, 128x128 (4 waves of 64x64) when those still give two workgroups per CU,
-  // else 64x128 (4 waves side by side along N); measured at the layer shapes (in_proj /
-  // out_proj / configs[1] / configs[4])
-  const int64_t tiles256 = ((a.M + 127) / 128) * ((a.N + 255) / 256);
-  const int64_t tiles128 = ((a.M + 127) / 128) * ((a.N + 127) / 128);
-  // long K loops over many tiles: direct-to-LDS loads into two stages (no staging registers);
-  // MIMO in_proj at M 8192: 1048 us vs 1069 us with three stages
-  if (a.N % 256 == 0 && tiles256 >= 2048 && a.Kp >= 2048) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
-  // short K on a few hundred 128x256 tiles (the SISO in_proj: 8192 x 2432 x 768; the LM head: 512 x
-  // 151936 x 768): two direct-to-LDS stages (48 KB; registers allow two workgroups per CU either
-  // way): 23.6 us vs 25.6 us with three stages and 27.6 us for register-staged 128x128 tiles; LM
-  // head 74 us vs 82 us
-  if (tiles256 >= 512 && a.Kp <= 1024) {
-    // more 128x256 tiles than two rounds of the CUs with a narrow remainder (the SISO in_proj: 640
-    // tiles): the columns past two tiles per CU go to 128x128 tiles (the split kernel)
-    const int cus = device_limits().cus;
-    const int64_t ntm = (a.M + 127) / 128;
-    const int64_t ntnA = cus > 0 ? std::min<int64_t>(a.N / 256, (2 * cus) / ntm) : 0;
-    const int64_t nA = ntnA * 256;
-    constexpr int TMB = 2;  // 128-row tail tiles (64-row ones: 26.7 against 26.1 us in the layer)
-    const int64_t ntmB = (a.M + 64 * TMB - 1) / (64 * TMB), ntnB = (a.N - nA + 127) / 128;
-    if (ntnA >= 1 && a.N > nA && a.N - nA <= 512 && ntm * ntnA + ntmB * ntnB <= 0x7fffffff) {
-      const unsigned grid = static_cast<unsigned>(ntm * ntnA + ntmB * ntnB);
-      if (a.out_dt == kBF16)
-        mfma32_split_kernel<kBF16, TMB, EPI><<<grid, 512, 0, TESM_LOGGED(st, mfma32_split_kernel<kBF16, TMB, EPI>)>>>(a, nA);
-      else
-        mfma32_split_kernel<kF32, TMB, EPI><<<grid, 512, 0, TESM_LOGGED(st, mfma32_split_kernel<kF32, TMB, EPI>)>>>(a, nA);
-      return check_launch("bitlinear mfma32 split");
-    }
-    return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
-  }
-  // fewer 128x256 tiles than CUs at short K (the SISO out_proj: 8192 x 768 x 768): 64x128 tiles, two
-  // direct-to-LDS stages: 10.1 us vs 10.7 us for 128x256 tiles
-  if (tiles256 < 256 && a.Kp <= 1024) return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
-  if (a.N % 256 == 0 && tiles256 >= 128) return run_mfma32<2, 4, 2, 2, EPI>(a, st);
-  if (tiles128 >= 512) return run_mfma32<2, 2, 2, 2, EPI>(a, st);
-  return run_mfma32<1, 4, 2, 1, EPI>(a, st);
-}
-
 int launch_linear(const LinearArgs& a, hipStream_t st) {
   TESM_REQUIRE(a.M >= 0 && a.N >= 0, kErrInvalidArg, "bitlinear: negative size");
   TESM_REQUIRE(a.Kp >= kKTile && a.Kp % kKTile == 0, kErrInvalidArg, "bitlinear: Kp must be a positive multiple of 128");
@@ -2703,7 +1715,7 @@ int launch_linear(const LinearArgs& a, hipStream_t st) {
     TESM_REQUIRE(a.M > 32 && !a.bias && !a.acc_dump && !a.op[0].c_w_per_row && a.act_bias && a.act_w > 0 &&
                      a.act_n0 >= 0 && a.act_n0 % 32 == 0 && a.act_w % 32 == 0 && a.act_n0 + 3 * a.act_w <= a.N,
                  kErrUnsupported, "bitlinear gates epilogue: needs M > 32, 32-aligned regions inside N, no bias");
-    return dispatch_store32<kEpiGates>(a, st);
+    return launch_mfma32(a, st);
   }
   if (a.epilogue != kEpiStore) {
     if (int rc = check_operand(a.op[1], a.Kp, "op1")) return rc;
@@ -2723,13 +1735,12 @@ int launch_linear(const LinearArgs& a, hipStream_t st) {
     // tiles to fill the chip (measured at M = 32: N = 768 .. 4096 faster split, N = 34816 staged)
     if (a.M <= 16 && a.N < 16384) return run_skinny<4, 1, 1, kEpiStore>(a, st);
     if (a.M <= 32 && a.N < 16384) return run_skinny<4, 2, 1, kEpiStore>(a, st);
-    // decode-size batches over wide weights (MIMO decode in_proj, 32 x 34816 x 4096): 32x128 tiles on
-    // the 32x32x32 form, 16.5 us vs 19.3 us for 32x64 tiles on the 16x16x64 one
-    if (a.M <= 32) return run_mfma32<1, 4, 1, 1, kEpiStore>(a, st);
-    return dispatch_store32<kEpiStore>(a, st);
+    return launch_mfma32(a, st);
   }
-  if (a.epilogue == kEpiOutputGate) return dispatch_dual<kEpiOutputGate>(a, st);
-  return dispatch_dual<kEpiSwiGLU>(a, st);
+  // two-product epilogues: split-K for decode-size batches, else the 32x32 kernels
+  if (a.M <= 16) return a.epilogue == kEpiOutputGate ? run_skinny<4, 1, 1, kEpiOutputGate>(a, st) : run_skinny<4, 1, 1, kEpiSwiGLU>(a, st);
+  if (a.M <= 32) return a.epilogue == kEpiOutputGate ? run_skinny<4, 2, 1, kEpiOutputGate>(a, st) : run_skinny<4, 2, 1, kEpiSwiGLU>(a, st);
+  return launch_mfma32(a, st);
 }
 
 int launch_gate_out(const LinearArgs& a, const RowQuant& o, const LinearOperand& out_proj, void* out, int64_t ldout,

@@ -1,0 +1,589 @@
+// INT2 x INT8 products of more than 32 rows (and wide ones of fewer) on v_mfma_i32_32x32x32_i8, which on
+// gfx950 delivers about twice the int8 rate of the 16x16x64 form.
+//
+// A workgroup owns BM x BN outputs: WM x WN waves, each TM x TN tiles of 32 x 32.  Weights are the MFMA's A
+// operand: in k-step s (of the 4 of a 128-code K tile) lane L feeds weight column L%32 with chunk 4*(L/32) + s
+// (one packed dword, unpacked in registers) and activation row L%32 with the same 16-code chunk; any pairing
+// of chunks to k-steps gives the same sums as long as both operands use it, and this one makes a lane's four
+// weight dwords of a K tile one 16-byte read.  Accumulator element r of lane L is weight column
+// 8*(r/4) + 4*(L/32) + r%4 and activation row L%32.
+//
+// Pipeline.  K tiles go straight from memory to LDS (global_load_lds_dwordx4, no staging registers) into NS
+// stages.  A fragment's LDS reads are issued one k-step ahead of its MFMAs, across the K tile boundary too: the
+// one barrier of a K tile stands in its middle, where a wave (a) knows its loads of the next tile landed
+// (vmcnt), (b) meets the others, so the next tile may be read from the last k-step on and the previous tile's
+// stage may be refilled.  With the wait at a tile's start instead, and two stages, every tile paid an LDS round
+// trip and the slowest wave's load (2048 x 4096 x 4096: 37.6 -> 34.7 us; 4095 x 3840 x 1024: 28.3 -> 21.0).
+//
+// What bounds it: large products run at 2.1-2.3 POP/s, where the chip's power limit lies for these operands (the
+// library int8 product reaches 2.25 on random codes; the same kernel on all-zero codes is 1.3 times faster; tiles
+// from 128x128 to 256x256, 64x64 to 128x64 per wave and 2 to 4 stages all end within 10 % of each other).  Small
+// ones are bound by the latency of the first tiles and by idle CUs, hence the K groups: KS groups of waves
+// in one workgroup take K tiles g, g + KS, ... into stages of their own, and their exact int32 sums are added in
+// LDS, so a 32 x 64 tile with a quarter of the K loop per group replaces 64 x 128 tiles on a fifth of the CUs
+// (512 x 768 x 3072: 13.7 -> 5.7 us; 512 x 768 x 768: 6.1 -> 4.0).
+//
+// Two-product epilogues: SwiGLU's products share the activations, so one K loop reads them once against both
+// weight tiles (it ran one K loop after the other: 4095 x 2816 x 1024 53.8 us); the output gate's products follow
+// each other in one pipeline.
+//
+// LDS images (bank model measured on the device: 16-byte reads are served 16 lanes per pass over 256 bytes): one
+// load instruction moves 64 lanes x 16 bytes into 1 KB in lane order, so the layouts are chosen through the lanes'
+// global addresses: activation rows in blocks of 8 rows x 8 chunks (chunk q of row r in slot
+// r*8 + (q ^ ((r/2) % 8))), weights in blocks of 32 columns x 2 halves (half h of column n in slot
+// 2n + (h ^ ((n/8) % 2))); both make the fragment reads hit 16 distinct 16-byte slots of 256 bytes.
+#include "linear_dev.h"
+
+namespace tesm {
+
+namespace {
+
+__device__ __forceinline__ int a32_off(int row, int q) { return 16 * (row * 8 + (q ^ ((row >> 1) & 7))); }
+__device__ __forceinline__ int b32_off(int col, int h) { return 16 * (col * 2 + (h ^ ((col >> 3) & 1))); }
+
+template <int WM, int WN, int TM, int TN, int KS, int NS, int EPI, int OUT_DT>
+struct Tile32 {
+  static constexpr bool DUAL = epi_dual(EPI);
+  static constexpr bool SHARE = EPI == kEpiSwiGLU;  // both products read one set of activations
+  static constexpr int NACC = DUAL ? 2 : 1;
+  static constexpr int NWT = SHARE ? 2 : 1;  // weight tiles per K tile
+  static constexpr int NG = WM * WN, NW = NG * KS, NT = NW * 64;
+  static constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 128;
+  static constexpr int A_BYTES = BM * BK, W_BYTES = BN * BK / 4;
+  static constexpr int SUB = A_BYTES + NWT * W_BYTES;  // one group's K tile
+  static constexpr int STAGE = SUB * KS;
+  static constexpr int NA = BM / 8, NB = BN / 32, PER = NA + NWT * NB;  // 1 KB blocks
+  static constexpr int D = (PER * KS + NW - 1) / NW;  // loads per wave and stage (the last block is loaded twice
+                                                      // where they do not divide: the same bytes to the same place)
+  static constexpr int ES = OUT_DT == kBF16 ? 2 : 4;
+  static constexpr int RED = (KS - 1) * NG * NACC * TM * TN * 4096;  // partial sums of the other K groups
+  static constexpr int SLAB = 32 * (TN * 32 * ES + 16);              // a wave's 32 rows x TN column tiles
+  static constexpr int SMEM = std::max(NS * STAGE, RED + NG * SLAB);
+  static_assert(NS >= 3 && (NS - 2) * D < 64, "loads in flight");
+  static_assert(!(EPI == kEpiOutputGate && KS > 1), "the gate's products follow each other in one group");
+};
+
+// acc[p][i][j]: product p, row tile i, column tile j of the wave's group (with KS > 1 a partial sum).
+template <class T, int WN, int TM, int TN, int KS, int NS>
+__device__ __forceinline__ void mfma32_loop(const LinearArgs& a, int64_t m0, int64_t n0, v16i (&acc)[T::NACC][TM][TN],
+                                            char* smem) {
+  const int t = threadIdx.x;
+  __builtin_assume(t < T::NT);
+  const int lane = t & 63, wall = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int kg = wall / T::NG, w = wall % T::NG;
+  const int wm = w / WN, wn = w % WN;
+  constexpr int SEQ = T::DUAL && !T::SHARE ? 2 : 1;  // products one after the other
+  // this lane's source of each of the wave's D blocks (rows past M and columns past N re-read the last one and
+  // feed only outputs that are never stored), and the K group each block belongs to
+  const char* src[SEQ][T::D];
+  int dst[T::D], adv[T::D], grp[T::D];
+#pragma unroll
+  for (int i = 0; i < T::D; ++i) {
+    const int b0 = wall + i * T::NW, blk = b0 < T::PER * KS ? b0 : T::PER * KS - 1;
+    const int g = blk / T::PER, bb = blk % T::PER;
+    grp[i] = g;
+#pragma unroll
+    for (int p = 0; p < SEQ; ++p) {
+      if (bb < T::NA) {
+        const LinearOperand& o = a.op[p];
+        const int row = bb * 8 + (lane >> 3);
+        const int q = (lane & 7) ^ ((row >> 1) & 7);
+        const int64_t m = m0 + row;
+        src[p][i] = reinterpret_cast<const char*>(o.q) + (m < a.M ? m : a.M - 1) * o.ldq + 16 * q;
+      } else {
+        const int wt = (bb - T::NA) / T::NB, cb = (bb - T::NA) % T::NB;
+        const LinearOperand& o = a.op[T::SHARE ? wt : p];
+        const int col = cb * 32 + (lane >> 1);
+        const int h = (lane & 1) ^ ((col >> 3) & 1);
+        const int64_t n = n0 + col;
+        src[p][i] = reinterpret_cast<const char*>(o.w) + (n < a.N ? n : a.N - 1) * o.ldw + 16 * h;
+      }
+    }
+    adv[i] = bb < T::NA ? T::BK : T::BK / 4;
+    dst[i] = g * T::SUB + bb * 1024;  // (A_BYTES and W_BYTES are whole blocks)
+  }
+  const int nk = static_cast<int>(a.Kp / T::BK);
+  const int steps = SEQ == 2 ? 2 * nk : (nk + KS - 1) / KS;
+  auto issue = [&](int kt, int st) {  // (past the last tile: re-reads it, so every wave's count stays the same)
+    char* stage = smem + st * T::STAGE;
+#pragma unroll
+    for (int i = 0; i < T::D; ++i) {
+      if constexpr (SEQ == 2) {
+        const int p = kt >= nk ? 1 : 0;
+        int k = kt - p * nk;
+        k = k < nk ? k : nk - 1;
+        lds_dma16((p ? src[SEQ - 1][i] : src[0][i]) + static_cast<int64_t>(k) * adv[i], stage + dst[i]);
+      } else {
+        int k = kt * KS + grp[i];
+        k = k < nk ? k : nk - 1;
+        lds_dma16(src[0][i] + static_cast<int64_t>(k) * adv[i], stage + dst[i]);
+      }
+    }
+  };
+  const int hq = 4 * (lane >> 5);
+  int ar[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) ar[s] = kg * T::SUB + a32_off(wm * TM * 32 + (lane & 31), hq + s);
+  const int br = kg * T::SUB + T::A_BYTES + b32_off(wn * TN * 32 + (lane & 31), lane >> 5);
+  constexpr int NB = T::NWT * TN;
+  v4i bw[2][NB], af[2][TM];
+  auto read_a = [&](const char* cur, int s, v4i (&f)[TM]) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) f[i] = *reinterpret_cast<const v4i*>(cur + ar[s] + i * 4096);
+  };
+  auto read_b = [&](const char* cur, v4i (&f)[NB]) {
+#pragma unroll
+    for (int p = 0; p < T::NWT; ++p)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        f[p * TN + j] = *reinterpret_cast<const v4i*>(cur + br + p * T::W_BYTES + j * 1024);
+  };
+  auto mma = [&](int prod, const v4i (&b)[NB], const v4i (&f)[TM], int s) {
+#pragma unroll
+    for (int p = 0; p < T::NWT; ++p)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const v4i bf = unpack_frag(static_cast<uint32_t>(b[p * TN + j][s]));
+        v16i(&c)[TM][TN] = acc[T::SHARE ? p : prod];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) c[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, f[i], c[i][j], 0, 0, 0);
+      }
+  };
+  // scheduling barriers keep the compiler from sinking the next fragments' reads behind the MFMAs
+  int st = 0;
+  auto tile = [&](int kt, int prod, v4i (&b)[NB], v4i (&bn)[NB]) {
+    const char* cur = smem + st * T::STAGE;
+    const int nx = st + 1 == NS ? 0 : st + 1, pv = st == 0 ? NS - 1 : st - 1;
+    const char* nxt = smem + nx * T::STAGE;
+    const bool live = KS == 1 || kt * KS + kg < nk;  // (wave-uniform)
+    read_a(cur, 1, af[1]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) mma(prod, b, af[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(cur, 2, af[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) mma(prod, b, af[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    read_a(cur, 3, af[1]);
+    wait_vmcnt<(NS - 3) * T::D>();  // this wave's loads of tile kt + 1 have landed
+    __builtin_amdgcn_s_barrier();   // ... every wave's, and every wave is done with tile kt - 1
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    issue(kt + NS - 1, pv);         // into the stage tile kt - 1 used
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) mma(prod, b, af[0], 2);
+    __builtin_amdgcn_sched_barrier(0);
+    read_b(nxt, bn);
+    read_a(nxt, 0, af[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (live) mma(prod, b, af[1], 3);
+    __builtin_amdgcn_sched_barrier(0);
+    st = nx;
+  };
+#pragma unroll
+  for (int g = 0; g < NS - 1; ++g) issue(g, g);
+  wait_vmcnt<(NS - 2) * T::D>();
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  read_b(smem, bw[0]);
+  read_a(smem, 0, af[0]);
+  if constexpr (SEQ == 2) {
+    int kt = 0;
+    for (; kt + 2 <= nk; kt += 2) {
+      tile(kt, 0, bw[0], bw[1]);
+      tile(kt + 1, 0, bw[1], bw[0]);
+    }
+    if (kt < nk) {  // an odd number of K tiles: the second product starts on the other weight registers
+      tile(kt, 0, bw[0], bw[1]);
+      ++kt;
+      for (; kt + 2 <= steps; kt += 2) {
+        tile(kt, 1, bw[1], bw[0]);
+        tile(kt + 1, 1, bw[0], bw[1]);
+      }
+      if (kt < steps) tile(kt, 1, bw[1], bw[0]);
+    } else {
+      for (; kt + 2 <= steps; kt += 2) {
+        tile(kt, 1, bw[0], bw[1]);
+        tile(kt + 1, 1, bw[1], bw[0]);
+      }
+    }
+  } else {
+    int kt = 0;
+    for (; kt + 2 <= steps; kt += 2) {
+      tile(kt, 0, bw[0], bw[1]);
+      tile(kt + 1, 0, bw[1], bw[0]);
+    }
+    if (kt < steps) tile(kt, 0, bw[0], bw[1]);
+  }
+  wait_vmcnt<0>();  // the re-reads past the last tile: the stages are reused by the epilogue
+  __syncthreads();
+}
+
+// Orders a wave's own LDS accesses (its slab is private: no other wave waits for it).
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
+// A wave's 32 rows x TN column tiles, four consecutive columns per lane and group: written to its LDS slab and
+// read back as 16-byte row-contiguous chunks, so a store instruction covers whole row segments (128 bytes for two
+// bf16 tiles).  v(j, g, out) gives the four values of tile j's group g (columns 8g + 4*(lane/32) ..).
+template <int OUT_DT, int TN, class F>
+__device__ __forceinline__ void store_tiles32(const LinearArgs& a, char* slab, int64_t mb, int64_t nb, F v) {
+  constexpr int ES = OUT_DT == kBF16 ? 2 : 4, RB = TN * 32 * ES, PITCH = RB + 16, CPR = RB / 16, VPC = 16 / ES;
+  const int lane = threadIdx.x & 63;
+  wave_lds_fence();  // the slab's previous contents are consumed
+#pragma unroll
+  for (int j = 0; j < TN; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float x[4];
+      v(j, g, x);
+      char* p = slab + (lane & 31) * PITCH + (32 * j + 8 * g + 4 * (lane >> 5)) * ES;
+      if constexpr (OUT_DT == kBF16)
+        *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]));
+      else
+        *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
+    }
+  wave_lds_fence();
+#pragma unroll
+  for (int it = 0; it < 32 * CPR / 64; ++it) {
+    const int idx = it * 64 + lane, row = idx / CPR, ch = idx % CPR;
+    const int64_t m = mb + row, n = nb + ch * VPC;
+    if (m >= a.M || n >= a.N) continue;
+    const uint4 d = *reinterpret_cast<const uint4*>(slab + row * PITCH + ch * 16);
+    char* dst = static_cast<char*>(a.out) + (m * a.ldo + n) * ES;
+    if (n + VPC <= a.N) {
+      *reinterpret_cast<uint4*>(dst) = d;
+    } else {
+      const uint32_t wd[4] = {d.x, d.y, d.z, d.w};
+      for (int e = 0; e < a.N - n; ++e) {
+        if constexpr (OUT_DT == kBF16)
+          reinterpret_cast<uint16_t*>(dst)[e] = static_cast<uint16_t>(wd[e >> 1] >> (16 * (e & 1)));
+        else
+          reinterpret_cast<uint32_t*>(dst)[e] = wd[e];
+      }
+    }
+  }
+}
+
+// The outputs of one wave (tile rows wm*TM .., columns wn*TN ..).  slab: SLAB bytes of the wave's own.
+template <int TM, int TN, int EPI, int OUT_DT>
+__device__ __forceinline__ void epilogue32(const LinearArgs& a, const v16i (&acc)[epi_dual(EPI) ? 2 : 1][TM][TN],
+                                           int64_t m0, int64_t n0, int wm, int wn, char* slab) {
+  constexpr bool DUAL = epi_dual(EPI);
+  constexpr int es = OUT_DT == kBF16 ? 2 : 4;
+  const int lane = threadIdx.x & 63;
+  const LinearOperand& o0 = a.op[0];
+  const LinearOperand& o1 = a.op[1];
+  float inv0[TM], inv1[TM];
+  int32_t rs0[TM], rs1[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int64_t m = m0 + (wm * TM + i) * 32 + (lane & 31);
+    const int64_t mc = m < a.M ? m : a.M - 1;
+    inv0[i] = o0.s_x[mc];
+    rs0[i] = o0.rowsum[mc];
+    inv1[i] = DUAL ? o1.s_x[mc] : 1.0f;
+    rs1[i] = DUAL ? o1.rowsum[mc] : 0;
+  }
+  const float cws = o0.c_w[0], cws1 = DUAL ? o1.c_w[0] : 0.0f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    inv0[i] = 1.0f / inv0[i];
+    inv1[i] = 1.0f / inv1[i];
+  }
+  const bool a16 = reinterpret_cast<uintptr_t>(a.out) % 16 == 0 && (a.ldo * es) % 16 == 0;
+  const bool tensor = !o0.c_w_per_row && !(DUAL && o1.c_w_per_row) && !a.acc_dump;
+  if (a16 && tensor && EPI != kEpiOutputGate && !a.bias) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int64_t nb = n0 + wn * TN * 32;
+      int kind[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) kind[j] = EPI == kEpiGates ? gate_region(a, nb + 32 * j) : 0;
+      store_tiles32<OUT_DT, TN>(a, slab, m0 + (wm * TM + i) * 32, nb, [&](int j, int g, float (&v)[4]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = (static_cast<float>(acc[0][i][j][4 * g + r] - rs0[i]) * inv0[i]) * cws;
+        if constexpr (EPI == kEpiGates) gate_act4<OUT_DT>(a, kind[j], nb + 32 * j + 8 * g + 4 * (lane >> 5), v);
+        if constexpr (DUAL) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float v1 = (static_cast<float>(acc[DUAL ? 1 : 0][i][j][4 * g + r] - rs1[i]) * inv1[i]) * cws1;
+            v[r] = dual_epi<EPI, OUT_DT>(rnd<OUT_DT>(v[r]), rnd<OUT_DT>(v1), 0.0f, 0.0f);
+          }
+        }
+      });
+    }
+    return;
+  }
+  // General form: per-row weight scales, bias, accumulator dump, unaligned outputs, and the output gate.  The
+  // gate's inputs of one 32 x 32 tile (four groups of four columns per lane) are requested together in
+  // straight-line code (indices clamped into range, raw bits) before any is used, so the tile waits for
+  // memory once instead of once per group.
+  const bool vout = vec4_ok<OUT_DT>(a.out, a.ldo);
+  const bool vin = EPI == kEpiOutputGate && vec4_ok<OUT_DT>(a.local, a.ld_local) &&
+                   vec4_ok<OUT_DT>(a.gate, a.ld_gate) && a.N % 4 == 0;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int64_t m = m0 + (wm * TM + i) * 32 + (lane & 31), mc = m < a.M ? m : a.M - 1;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      uint32_t lo[4][4], gt[4][4];
+      if constexpr (EPI == kEpiOutputGate) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int64_t nb = n0 + (wn * TN + j) * 32 + 8 * g + 4 * (lane >> 5);
+          if (vin) {  // whole groups of four: a group past N re-reads the last one
+            const int64_t nv = nb < a.N ? nb : a.N - 4;
+            const char* pl = static_cast<const char*>(a.local) + (mc * a.ld_local + nv) * es;
+            const char* pg = static_cast<const char*>(a.gate) + (mc * a.ld_gate + nv) * es;
+#pragma unroll
+            for (int q = 0; q < es / 2; ++q) {  // bf16: one 8-byte load, f32: two
+              const uint2 wl = reinterpret_cast<const uint2*>(pl)[q], wg = reinterpret_cast<const uint2*>(pg)[q];
+              lo[g][2 * q] = wl.x;
+              lo[g][2 * q + 1] = wl.y;
+              gt[g][2 * q] = wg.x;
+              gt[g][2 * q + 1] = wg.y;
+            }
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int64_t n = nb + r < a.N ? nb + r : a.N - 1;
+              lo[g][r] = ld_bits<OUT_DT>(a.local, mc * a.ld_local + n);
+              gt[g][r] = ld_bits<OUT_DT>(a.gate, mc * a.ld_gate + n);
+            }
+          }
+        }
+      }
+      if (m >= a.M) continue;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int64_t nb = n0 + (wn * TN + j) * 32 + 8 * g + 4 * (lane >> 5);
+        if (nb >= a.N) continue;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int64_t n = nb + r, nc = n < a.N ? n : a.N - 1;
+          const float cw0 = o0.c_w_per_row ? o0.c_w[nc] : cws;
+          const int32_t a0 = acc[0][i][j][4 * g + r] - rs0[i];
+          if (a.acc_dump && n < a.N) a.acc_dump[m * a.N + n] = a0;
+          const float v0 = (static_cast<float>(a0) * inv0[i]) * cw0;
+          if constexpr (!DUAL) {
+            v[r] = a.bias ? v0 + ld<OUT_DT>(a.bias, nc) : v0;
+          } else {
+            const float cw1 = o1.c_w_per_row ? o1.c_w[nc] : cws1;
+            const float v1 = rnd<OUT_DT>((static_cast<float>(acc[1][i][j][4 * g + r] - rs1[i]) * inv1[i]) * cw1);
+            float lv = 0.0f, gv = 0.0f;
+            if constexpr (EPI == kEpiOutputGate) {
+              if (vin && OUT_DT == kBF16) {
+                const uint32_t wl = lo[g][r >> 1], wg = gt[g][r >> 1];
+                lv = __uint_as_float(r & 1 ? wl & 0xffff0000u : wl << 16);
+                gv = __uint_as_float(r & 1 ? wg & 0xffff0000u : wg << 16);
+              } else {
+                lv = from_bits<OUT_DT>(lo[g][r]);
+                gv = from_bits<OUT_DT>(gt[g][r]);
+              }
+            }
+            v[r] = dual_epi<EPI, OUT_DT>(rnd<OUT_DT>(v0), v1, lv, gv);
+          }
+        }
+        if constexpr (EPI == kEpiGates) gate_act4<OUT_DT>(a, gate_region(a, n0 + (wn * TN + j) * 32), nb, v);
+        if (nb + 3 < a.N) {
+          store4<OUT_DT>(a.out, m * a.ldo + nb, v, vout);
+        } else {
+          for (int r = 0; r < 4 && nb + r < a.N; ++r) st<OUT_DT>(a.out, m * a.ldo + nb + r, v[r]);
+        }
+      }
+    }
+  }
+}
+
+// One output tile at (m0, n0); smem holds at least the tile's SMEM bytes.
+template <int WM, int WN, int TM, int TN, int KS, int NS, int EPI, int OUT_DT>
+__device__ __forceinline__ void mfma32_tile(const LinearArgs& a, int64_t m0, int64_t n0, char* smem) {
+  using T = Tile32<WM, WN, TM, TN, KS, NS, EPI, OUT_DT>;
+  v16i acc[T::NACC][TM][TN];
+#pragma unroll
+  for (int p = 0; p < T::NACC; ++p)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[p][i][j] = v16i{};
+  mfma32_loop<T, WN, TM, TN, KS, NS>(a, m0, n0, acc, smem);
+  const int lane = threadIdx.x & 63, wall = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int kg = wall / T::NG, w = wall % T::NG;
+  if constexpr (KS > 1) {  // the other groups' partial sums, added by group 0 (integers: any order is exact)
+    constexpr int TQ = T::NACC * TM * TN * 4;
+    v4i* red = reinterpret_cast<v4i*>(smem);
+    if (kg > 0) {
+#pragma unroll
+      for (int q = 0; q < TQ; ++q) {
+        const v16i& c = acc[q / (4 * TM * TN)][q / (4 * TN) % TM][q / 4 % TN];
+        red[(((kg - 1) * T::NG + w) * TQ + q) * 64 + lane] =
+            v4i{c[4 * (q % 4)], c[4 * (q % 4) + 1], c[4 * (q % 4) + 2], c[4 * (q % 4) + 3]};
+      }
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int h = 0; h < KS - 1; ++h)
+#pragma unroll
+      for (int q = 0; q < TQ; ++q) {
+        v16i& c = acc[q / (4 * TM * TN)][q / (4 * TN) % TM][q / 4 % TN];
+        const v4i v = red[((h * T::NG + w) * TQ + q) * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[4 * (q % 4) + r] += v[r];
+      }
+  }
+  epilogue32<TM, TN, EPI, OUT_DT>(a, acc, m0, n0, w / WN, w % WN, smem + T::RED + w * T::SLAB);
+}
+
+// One group of WM x WN waves per tile.  ORD: the tile order, 4 (ORD 0) or 8 (ORD 2) M tiles per group of the
+// XCD-aware walk: the fewer for grids of about one round, whose XCDs then share weights across fewer rows
+// (2048 x 4096 x 4096: 34.7 us with 4, 38.1 with 8), the more for grids of many rounds (8192 x 34816 x 4096:
+// 1016 us with 8, 1054 with 4).
+template <int WM, int WN, int TM, int TN, int EPI, int OUT_DT, int ORD>
+__global__ __launch_bounds__(WM* WN * 64, WM * WN >= 8 && EPI != kEpiOutputGate ? 4 : 1) void mfma32_kernel(LinearArgs a) {
+  using T = Tile32<WM, WN, TM, TN, 1, 3, EPI, OUT_DT>;
+  __shared__ __attribute__((aligned(16))) char smem[T::SMEM];
+  int64_t tm, tn;
+  xcd_tile_of<ORD == 0 ? 4 : 8>(blockIdx.x, (a.M + T::BM - 1) / T::BM, (a.N + T::BN - 1) / T::BN, tm, tn);
+  mfma32_tile<WM, WN, TM, TN, 1, 3, EPI, OUT_DT>(a, tm * T::BM, tn * T::BN, smem);
+}
+
+// KS groups of WM x WN waves per tile, each with K tiles of its own.
+template <int WM, int WN, int TM, int TN, int KS, int NS, int EPI, int OUT_DT>
+__global__ __launch_bounds__(WM* WN* KS * 64) void mfma32k_kernel(LinearArgs a) {
+  using T = Tile32<WM, WN, TM, TN, KS, NS, EPI, OUT_DT>;
+  __shared__ __attribute__((aligned(16))) char smem[T::SMEM];
+  int64_t tm, tn;
+  xcd_tile_of<4>(blockIdx.x, (a.M + T::BM - 1) / T::BM, (a.N + T::BN - 1) / T::BN, tm, tn);
+  mfma32_tile<WM, WN, TM, TN, KS, NS, EPI, OUT_DT>(a, tm * T::BM, tn * T::BN, smem);
+}
+
+// Plain product whose 128x256 tiles would run in more rounds than the CUs hold (the SISO in_proj, 640
+// tiles): columns [0, nA) in 128x256 tiles, two per CU, and the remaining N - nA columns in 128x128
+// tiles launched after them, so the last round runs half-size tiles on more CUs.
+template <int OUT_DT, int TMB, int EPI>
+__global__ __launch_bounds__(512, 4) void mfma32_split_kernel(LinearArgs a, int64_t nA) {
+  using A = Tile32<2, 4, 2, 2, 1, 3, EPI, OUT_DT>;
+  using B = Tile32<2, 4, TMB, 1, 1, 3, EPI, OUT_DT>;
+  __shared__ __attribute__((aligned(16))) char smem[A::SMEM > B::SMEM ? A::SMEM : B::SMEM];
+  const int64_t ntm = (a.M + A::BM - 1) / A::BM, ntnA = nA / A::BN, tilesA = ntm * ntnA;
+  int64_t tm, tn;
+  if (static_cast<int64_t>(blockIdx.x) < tilesA) {
+    xcd_tile_of<8>(blockIdx.x, ntm, ntnA, tm, tn);
+    mfma32_tile<2, 4, 2, 2, 1, 3, EPI, OUT_DT>(a, tm * A::BM, tn * A::BN, smem);
+  } else {
+    xcd_tile_of<8>(blockIdx.x - tilesA, (a.M + B::BM - 1) / B::BM, (a.N - nA + B::BN - 1) / B::BN, tm, tn);
+    mfma32_tile<2, 4, TMB, 1, 1, 3, EPI, OUT_DT>(a, tm * B::BM, nA + tn * B::BN, smem);
+  }
+}
+
+template <int WM, int WN, int TM, int TN, int EPI, int ORD>
+int run_mfma32(const LinearArgs& a, hipStream_t st) {
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, NT = WM * WN * 64;
+  const int64_t tiles = ((a.N + BN - 1) / BN) * ((a.M + BM - 1) / BM);
+  TESM_REQUIRE(tiles <= 0x7fffffff, kErrUnsupported, "bitlinear: too many tiles");
+  const unsigned grid = static_cast<unsigned>(tiles);
+  if (a.out_dt == kBF16)
+    mfma32_kernel<WM, WN, TM, TN, EPI, kBF16, ORD><<<grid, NT, 0, TESM_LOGGED(st, mfma32_kernel<WM, WN, TM, TN, EPI, kBF16, ORD>)>>>(a);
+  else
+    mfma32_kernel<WM, WN, TM, TN, EPI, kF32, ORD><<<grid, NT, 0, TESM_LOGGED(st, mfma32_kernel<WM, WN, TM, TN, EPI, kF32, ORD>)>>>(a);
+  return check_launch("bitlinear mfma32");
+}
+
+template <int WM, int WN, int TM, int TN, int KS, int NS, int EPI>
+int run_mfma32k(const LinearArgs& a, hipStream_t st) {
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, NT = WM * WN * KS * 64;
+  const int64_t tiles = ((a.N + BN - 1) / BN) * ((a.M + BM - 1) / BM);
+  TESM_REQUIRE(tiles <= 0x7fffffff, kErrUnsupported, "bitlinear: too many tiles");
+  const unsigned grid = static_cast<unsigned>(tiles);
+  if (a.out_dt == kBF16)
+    mfma32k_kernel<WM, WN, TM, TN, KS, NS, EPI, kBF16><<<grid, NT, 0, TESM_LOGGED(st, mfma32k_kernel<WM, WN, TM, TN, KS, NS, EPI, kBF16>)>>>(a);
+  else
+    mfma32k_kernel<WM, WN, TM, TN, KS, NS, EPI, kF32><<<grid, NT, 0, TESM_LOGGED(st, mfma32k_kernel<WM, WN, TM, TN, KS, NS, EPI, kF32>)>>>(a);
+  return check_launch("bitlinear mfma32 (K groups)");
+}
+
+#ifdef MFMA32_SWEEP
+#include "sweep.inc"
+#endif
+
+// Tile sizes by grid.  Times in us on one box, bf16 outputs unless noted; "before" is the two-stage, one-group form.
+//   * 128x256 tiles (8 waves of 64x64, two workgroups per CU) when they give every CU one: 2048 x 4096 x 4096 36.2
+//     (64x256 tiles 40), 4095 x 3744 x 1024 22.0 (64x128: 26.3).  Grids past two rounds walk 8 M tiles per group.
+//   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
+//     kernel: 24.6 against 26.1 for 128x256 tiles throughout.
+//   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU: 8192 x 768 x 768 10.6 (128x256: 10.9),
+//     4095 x 1024 x 2816 15.4 (before 21.5), 1000 x 4096 x 4096 21.2 (before 28.3).  A K loop of at most
+//     three tiles stays on this shape too: such calls are launch-bound (16384 x 256 x 256 5.9, best 5.7; 512 x 96 x
+//     384 5.4, best 4.2), and it keeps short products to one instantiation.
+//   * 32x128 tiles when those do, at short K: 512 x 2944 x 768 4.9 (64x128: 5.8), 666 x 2944 x 768 f32 6.1 (7.1).
+//   * else K groups on 32x64 tiles: two (512 x 768 x 768 4.2, before 5.3; 32 x 34816 x 4096 12.3, before 14.0), or
+//     four when K is long and two would leave CUs idle (512 x 768 x 3072 5.7, before 11.8; 200 x 4096 x 11008 18.2,
+//     two groups 21.1).
+template <int EPI>
+int dispatch_store32(const LinearArgs& a, hipStream_t st) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+  const int64_t cus = std::max(device_limits().cus, 1);
+  const int64_t big = tiles(128, 256);
+  if (big >= 2 * cus && a.Kp <= 1024) {
+    const int64_t ntm = (a.M + 127) / 128, ntnA = std::min<int64_t>(a.N / 256, (2 * cus) / ntm), nA = ntnA * 256;
+    if (ntnA >= 1 && a.N > nA && a.N - nA <= 512) {
+      const int64_t grid = ntm * ntnA + ntm * ((a.N - nA + 127) / 128);
+      TESM_REQUIRE(grid <= 0x7fffffff, kErrUnsupported, "bitlinear: too many tiles");
+      if (a.out_dt == kBF16)
+        mfma32_split_kernel<kBF16, 2, EPI><<<static_cast<unsigned>(grid), 512, 0, TESM_LOGGED(st, mfma32_split_kernel<kBF16, 2, EPI>)>>>(a, nA);
+      else
+        mfma32_split_kernel<kF32, 2, EPI><<<static_cast<unsigned>(grid), 512, 0, TESM_LOGGED(st, mfma32_split_kernel<kF32, 2, EPI>)>>>(a, nA);
+      return check_launch("bitlinear mfma32 split");
+    }
+  }
+  if (a.Kp > 3 * kKTile) {
+    if (big >= 2 * cus) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
+    if (big >= cus) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
+    if (tiles(64, 128) < 2 * cus) {
+      if (a.Kp <= 1024 && tiles(32, 128) >= cus) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
+      if (a.Kp >= 2048 && tiles(32, 64) < 2 * cus) return run_mfma32k<1, 2, 1, 1, 4, 3, EPI>(a, st);
+      return run_mfma32k<1, 2, 1, 1, 2, 3, EPI>(a, st);
+    }
+  }
+  return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
+}
+
+// The output gate (two accumulator sets, so one 128x256 workgroup per CU): 4096 x 4096 x 2 x 2048 115 (before 118);
+// 64x128 tiles of eight waves when they give every CU one: 4095 x 1024 x 2 x 512 16.2 (before 28.6); else 32x64
+// tiles of two waves: 512 x 768 x 2 x 384 7.6 (before 12.0), 64 x 4096 x 2 x 8192 36.3 (before 51.4).
+int dispatch_gate32(const LinearArgs& a, hipStream_t st) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+  const int64_t cus = std::max(device_limits().cus, 1), big = tiles(128, 256);
+  if (big >= 8 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 2>(a, st);
+  if (big >= 2 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 0>(a, st);
+  if (tiles(64, 128) >= cus) return run_mfma32<2, 4, 1, 1, kEpiOutputGate, 0>(a, st);
+  return run_mfma32<1, 2, 1, 1, kEpiOutputGate, 0>(a, st);
+}
+
+// SwiGLU over 128 + 128 columns when those tiles give two workgroups per CU (4095 x 2 x 2816 x 1024 35.2, before 53.8;
+// one per CU is enough at long K: 200 x 2 x 16384 x 4096 34.5, before 58), else over 64 + 64 (512 x 2 x 3072 x 768
+// 7.6, before 12.5).
+int dispatch_swiglu32(const LinearArgs& a, hipStream_t st) {
+  const int64_t cus = std::max(device_limits().cus, 1), big = ((a.M + 127) / 128) * ((a.N + 127) / 128);
+  if (big >= 2 * cus || (big >= cus && a.Kp >= 2048)) return run_mfma32<2, 4, 2, 1, kEpiSwiGLU, 2>(a, st);
+  return run_mfma32<2, 2, 1, 1, kEpiSwiGLU, 0>(a, st);
+}
+
+#ifdef MFMA32_SWEEP
+#include "sweep.inc"
+#endif
+
+}  // namespace
+
+int launch_mfma32(const LinearArgs& a, hipStream_t st) {
+#ifdef MFMA32_SWEEP
+  if (const int rc = sweep_run(a, st); rc >= 0) return rc;
+#endif
+  if (a.epilogue == kEpiGates) return dispatch_store32<kEpiGates>(a, st);
+  if (a.epilogue == kEpiStore) return dispatch_store32<kEpiStore>(a, st);
+  if (a.epilogue == kEpiOutputGate) return dispatch_gate32(a, st);
+  return dispatch_swiglu32(a, st);
+}
+
+}  // namespace tesm
