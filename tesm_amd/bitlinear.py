@@ -52,6 +52,25 @@ class PackedWeight:
         self.packed, self.s_w, self.c_w, self.N, self.K = packed, s_w, c_w, N, K
 
 
+def packed_weights(lins, dt, n: int):
+    """The first n layers' current packed weights; every layer's weight must be of dtype ``dt``, as F.linear
+    requires of its operands."""
+    for p in lins:
+        wdt = p._parameters["weight"].dtype
+        if wdt != dt:
+            raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {wdt}")
+    return [p.packed_weight() for p in lins[:n]]
+
+
+def same_packs(keep, packs) -> bool:
+    """Whether a plan that holds ``keep`` (its packed weights first) was built on these packed weights.  The plan
+    keeps them alive, so one of them is the same object only if it is the same weight."""
+    for a, b in zip(keep, packs):
+        if a is not b:
+            return False
+    return True
+
+
 class BitLinear(nn.Module):
     def __init__(self, in_features, out_features, bias=False, bit_eps=1e-5, bit_threshold=0.5, kernel_backend="hip",
                  kernel_mode="fast", device=None, dtype=None):
@@ -199,11 +218,12 @@ class BitLinear(nn.Module):
             # F.linear in the reference raises for mixed operand dtypes
             raise RuntimeError(f"expected both operands to have the same dtype, got {x.dtype} and {self.weight.dtype}")
         pw = self.packed_weight()
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, self.in_features)
+        K = self.in_features
+        flat = x.dim() == 2 and x.shape[1] == K
         # quantized_input + _project_quantized (tesm.py:206-209, 287-290) in one C-ABI call
-        out = hip_ops.bitlinear_fwd(x2, pw.packed, pw.c_w, self.out_features, self.bit_eps, bias=self.bias)
-        return out.reshape(*lead, self.out_features)
+        out = hip_ops.bitlinear_fwd(x if flat else x.reshape(-1, K), pw.packed, pw.c_w, self.out_features, self.bit_eps,
+                                    bias=self.bias)
+        return out if flat else out.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self):
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

@@ -40,7 +40,8 @@ class RMSNorm(nn.Module):
         ``(y or None, s in residual_dtype or None, codes or None)`` where ``codes = (q, s_x, rowsum)``
         are y's per-token int8 codes in the product layout (computed when ``codes_eps`` is given)."""
         _check(x, "RMSNorm")
-        dt = self.weight.dtype
+        w = self._parameters["weight"]
+        dt = w.dtype
         if x.dtype != dt:
             raise RuntimeError(f"RMSNorm: input is {x.dtype} but the weight is {dt}")
         D = x.shape[-1]
@@ -66,7 +67,6 @@ class RMSNorm(nn.Module):
             res_out = torch.empty((M, D), dtype=residual_dtype, device=dev)
             desc.residual_out, desc.residual_out_dt, desc.ld_res_out = (res_out.data_ptr(),
                                                                         hip_ops.dt_code(residual_dtype), D)
-        w = self.weight.detach()
         desc.weight = w.data_ptr()
         y = None
         if want_y:
@@ -82,9 +82,7 @@ class RMSNorm(nn.Module):
                                                                      float(codes_eps))
             codes = (q, s, rs)
         hip_ops.require_device(x2, r2, w, res_out, y, *(codes or ()))
-        with torch.cuda.device(dev):
-            _lib.check(_lib.load().tesm_hip_add_rmsnorm(ctypes.byref(desc),
-                                                         ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)))
+        hip_ops.on_device(dev.index, _lib.load().tesm_hip_add_rmsnorm, ctypes.byref(desc), hip_ops.raw_stream(dev.index))
         return (y.reshape(*lead, D) if y is not None else None,
                 res_out.reshape(*lead, D) if res_out is not None else None, codes)
 

@@ -48,16 +48,34 @@ def _rows(x: torch.Tensor) -> torch.Tensor:
 def require_device(*ts):
     """Every tensor handed to a kernel must live on one ROCm device: a host pointer would be
     dereferenced by the GPU."""
-    dev = None
+    first, dev = None, -1
     for t in ts:
         if t is None:
             continue
-        if not t.is_cuda:
+        d = t.get_device()  # the index, -1 on the host: cheaper per call than building and comparing devices
+        if d < 0 or not t.is_cuda:
             raise RuntimeError(f"hip backend ops need tensors on a ROCm device, got one on {t.device}")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"hip backend ops need all tensors on one device, got {dev} and {t.device}")
+        if first is None:
+            first, dev = t, d
+        elif d != dev:
+            raise RuntimeError(f"hip backend ops need all tensors on one device, got {first.device} and {t.device}")
+
+
+def raw_stream(index: int) -> int:
+    """The raw handle of device ``index``'s current stream (``torch.cuda.current_stream(..).cuda_stream``
+    without building a Stream object, which costs over a microsecond per call)."""
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+def on_device(index: int, fn, *args) -> None:
+    """``fn(*args)`` with device ``index`` current (switched only if it is not already), its return code checked."""
+    if torch._C._cuda_getDevice() == index:
+        rc = fn(*args)
+    else:
+        with torch.cuda.device(index):
+            rc = fn(*args)
+    if rc:
+        _lib.check(rc)
 
 
 def kpad(K: int) -> int:
@@ -149,6 +167,11 @@ def bitlinear(q, s_x, rowsum, packed, c_w, N: int, K: int, out_dtype: torch.dtyp
     return (out, acc) if acc_dump else out
 
 
+@functools.lru_cache(maxsize=256)
+def _bitlinear_ws_bytes(M: int, K: int) -> int:
+    return int(_lib.load().tesm_hip_bitlinear_fwd_ws_bytes(M, K))
+
+
 def bitlinear_fwd(x, packed, c_w, N: int, eps: float = 1e-5, bias=None, c_w_per_row: bool = False,
                   fuse: bool = True, out: Optional[torch.Tensor] = None):
     """BitLinear forward from raw activations x (M, K): codes + product in one C-ABI call (fused
@@ -156,17 +179,19 @@ def bitlinear_fwd(x, packed, c_w, N: int, eps: float = 1e-5, bias=None, c_w_per_
     lib = _lib.load()
     x = _rows(x)
     M, K = x.shape
+    dev = x.device
     if out is None:
-        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        out = torch.empty((M, N), dtype=x.dtype, device=dev)
     require_device(x, packed, c_w, bias, out)
-    nbytes = int(lib.tesm_hip_bitlinear_fwd_ws_bytes(M, K))
+    nbytes = _bitlinear_ws_bytes(M, K)
     from .tesm import workspace
-    ws = workspace(x.device, nbytes)
-    with torch.cuda.device(x.device):
-        _lib.check(lib.tesm_hip_bitlinear_fwd(_p(x), dt_code(x.dtype), x.stride(0), eps, _p(packed), packed.stride(0),
-                                              _p(c_w), int(c_w_per_row), _p(bias), M, N, K, _p(out),
-                                              dt_code(out.dtype), out.stride(0), int(fuse), _p(ws), nbytes,
-                                              _stream(x)))
+    raw = raw_stream(dev.index)
+    ws = workspace(dev, nbytes, raw=raw)
+    # (pointers as plain integers: the signatures convert them, a c_void_p object per argument would cost more)
+    on_device(dev.index, lib.tesm_hip_bitlinear_fwd, x.data_ptr(), dt_code(x.dtype), x.stride(0), eps,
+              packed.data_ptr(), packed.stride(0), c_w.data_ptr(), int(c_w_per_row),
+              bias.data_ptr() if bias is not None else None, M, N, K, out.data_ptr(), dt_code(out.dtype),
+              out.stride(0), int(fuse), ws.data_ptr(), nbytes, raw)
     return out
 
 

@@ -22,7 +22,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, backend_error, check_hip_call
+from .bitlinear import BitLinear, backend_error, check_hip_call, packed_weights, same_packs
 from .block import Block, RMSNorm
 from .config import TESMConfig
 from .tesm import TESM_SISO, workspace
@@ -50,18 +50,38 @@ class FeedForward(nn.Module):
         self.down_proj = BitLinear(config.d_intermediate, config.d_model, **bl)
         self.dropout = nn.Dropout(config.dropout)
 
-    def _run(self, dt, lead, M, dev, x2=None, codes=None):
-        for p in (self.gate_proj, self.up_proj, self.down_proj):
+    def __getstate__(self):  # the plan holds device addresses: a copied or loaded module builds its own
+        return {k: v for k, v in self.__dict__.items() if k != "_plan"}
+
+    def _ffn_plan(self, dt):
+        """The descriptor's fields that depend on the weights alone, rebuilt when one changes (the packed weights'
+        rule, tesm.py:226-236); a call copies it."""
+        mods = self._modules
+        lins = (mods["gate_proj"], mods["up_proj"], mods["down_proj"])
+        for p in lins:
             if p.bias is not None:
                 raise backend_error(p.kernel_backend, "FeedForward", "BitLinear bias is not supported here")
-            if p.weight.dtype != dt:
-                raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
-        d_model, d_inter = self.gate_proj.in_features, self.gate_proj.out_features
-        y = torch.empty((M, d_model), dtype=dt, device=dev)
+        packs = packed_weights(lins, dt, 3)
+        key = (dt, lins[0].bit_eps)
+        plan = self.__dict__.get("_plan")
+        if plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
+            return plan[1]
         desc = _lib.Ffn()
         desc.dt = hip_ops.dt_code(dt)
-        desc.M, desc.d_model, desc.d_inter = M, d_model, d_inter
-        desc.bit_eps = float(self.gate_proj.bit_eps)
+        desc.d_model, desc.d_inter = lins[0].in_features, lins[0].out_features
+        desc.bit_eps = float(lins[0].bit_eps)
+        desc.gate_proj = lins[0].linear_desc()
+        desc.up_proj = lins[1].linear_desc()
+        desc.down_proj = lins[2].linear_desc()
+        self.__dict__["_plan"] = (key, (desc, packs))
+        return desc, packs
+
+    def _run(self, dt, lead, M, dev, x2=None, codes=None):
+        plan, keep = self._ffn_plan(dt)
+        desc = _lib.Ffn.from_buffer_copy(plan)
+        d_model = desc.d_model
+        y = torch.empty((M, d_model), dtype=dt, device=dev)
+        desc.M = M
         if codes is not None:
             q, s, rs = codes
             desc.x_codes, desc.ldq_x, desc.x_scale, desc.x_rowsum = q.data_ptr(), q.stride(0), s.data_ptr(), rs.data_ptr()
@@ -69,17 +89,13 @@ class FeedForward(nn.Module):
         else:
             desc.x, desc.ld_x = x2.data_ptr(), x2.stride(0)
             hip_ops.require_device(x2, y)
-        desc.gate_proj = self.gate_proj.linear_desc()
-        desc.up_proj = self.up_proj.linear_desc()
-        desc.down_proj = self.down_proj.linear_desc()
         desc.y, desc.ld_y = y.data_ptr(), d_model
         lib = _lib.load()
-        nbytes = int(lib.tesm_hip_ffn_ws_bytes(ctypes.byref(desc)))
-        stream = torch.cuda.current_stream(dev)
-        with torch.cuda.device(dev):
-            ws = workspace(dev, nbytes, stream)
-            _lib.check(lib.tesm_hip_ffn_forward(ctypes.byref(desc), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
-                                                ctypes.c_void_p(stream.cuda_stream)))
+        ref = ctypes.byref(desc)
+        nbytes = int(lib.tesm_hip_ffn_ws_bytes(ref))
+        raw = hip_ops.raw_stream(dev.index)
+        ws = workspace(dev, nbytes, raw=raw)
+        hip_ops.on_device(dev.index, lib.tesm_hip_ffn_forward, ref, ws.data_ptr(), ws.numel(), raw)
         return y.reshape(*lead, d_model)
 
     def forward(self, x):

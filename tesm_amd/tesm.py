@@ -20,15 +20,10 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, backend_error, check_hip_call
+from .bitlinear import BitLinear, backend_error, check_hip_call, packed_weights, same_packs
+from .hip_ops import on_device, raw_stream
 
 _WORKSPACES = {}
-
-
-def raw_stream(index: int) -> int:
-    """The raw handle of device ``index``'s current stream (``torch.cuda.current_stream(..).cuda_stream``
-    without building a Stream object, which costs over a microsecond on the per-token decode path)."""
-    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def workspace(device: torch.device, nbytes: int, stream=None, raw=None) -> torch.Tensor:
@@ -116,6 +111,12 @@ class TESM_SISO(nn.Module):
         self._rope = {}
         self._bias_cache = None
 
+    # descriptor plans hold device addresses (of tensors they keep alive): a copied or loaded module builds its own
+    _PLANS = ("_prefill_plan", "_decode_plan", "_mimo_plan", "_mimo_decode_plan")
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in self._PLANS}
+
     # -- cached device constants ---------------------------------------------------
     def rope_table(self, L: int, dtype: torch.dtype, device: torch.device, pos_offset: int = 0) -> torch.Tensor:
         key = (dtype, device, pos_offset)
@@ -174,25 +175,72 @@ class TESM_SISO(nn.Module):
             if cache is None or "state" not in cache:
                 cache = None
         y, states, h_final = self._prefill(u, cross_layer_state, prev_state, cache)
-        self._last_cross_layer_state = states
-        self._last_scan_state_f64 = h_final
-        self.last_entanglement_map = None
-        self.last_entanglement_stats = None
+        # plain attributes, set without nn.Module.__setattr__'s microsecond each (as in the decode step)
+        self.__dict__.update(_last_cross_layer_state=states, _last_scan_state_f64=h_final, last_entanglement_map=None)
+        if self.last_entanglement_stats is not None:
+            self.last_entanglement_stats = None
         return y, h_final
+
+    def _layer_plan(self, dt, dev, cross):
+        """The prefill descriptor's fields that depend on the module alone: sizes, thresholds, packed weights and
+        biases.  Rebuilt when a weight, a bias or an option changes (the packed weights' own rule,
+        tesm.py:226-236); a call copies it and fills in its lengths, tensors and outputs."""
+        mods, params = self._modules, self._parameters
+        lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"], mods["cross_layer_q_proj"])
+        glob = self.entanglement_window <= 0
+        biases = (params["decay_bias"],) + ((params["global_rel_pos_embed"], params["global_rel_pos_scale"],
+                                            params["global_rel_pos_bias"]) if glob else
+                                           (params["local_entanglement_bias"],))
+        packs = packed_weights(lins, dt, 4 + int(cross))
+        key = (dt, dev, cross, self.entanglement_window, self.state_scan_chunk_size, self.entanglement_threshold,
+               float(self.entanglement_scale), lins[0].bit_eps, self.d_model, self.d_state, self.ent_rank,
+               tuple((b._version, b.data_ptr(), b.dtype) for b in biases))
+        plan = self.__dict__.get("_prefill_plan")
+        if plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
+            return plan[1]
+        decay_bias = self._decay_bias_dt(dt)
+        local_bias = None if glob else self._local_bias_f32(dt)
+        gparams = self._global_params_f32(dt) if glob else ()
+        hip_ops.require_device(decay_bias, local_bias, *gparams)
+        if decay_bias.device != dev:
+            raise RuntimeError(f"hip backend ops need all tensors on one device, got {dev} and {decay_bias.device}")
+        desc = _lib.SisoLayer()
+        desc.dt = hip_ops.dt_code(dt)
+        desc.d_model, desc.d_state, desc.ent_rank = self.d_model, self.d_state, self.ent_rank
+        desc.window, desc.chunk_size = max(self.entanglement_window, 0), self.state_scan_chunk_size
+        desc.bit_eps = self.in_proj.bit_eps
+        desc.thr = hip_ops.round_dtype(self.entanglement_threshold, dt)
+        desc.ent_scale = float(self.entanglement_scale)
+        desc.in_proj = self.in_proj.linear_desc()
+        desc.state_proj = self.state_proj.linear_desc()
+        desc.ent_proj = self.ent_proj.linear_desc()
+        desc.out_proj = self.out_proj.linear_desc()
+        if cross:
+            desc.cross_q_proj = self.cross_layer_q_proj.linear_desc()
+        desc.decay_bias = decay_bias.data_ptr()
+        if glob:
+            emb, scale, bias = gparams
+            desc.global_embed, desc.global_dim = emb.data_ptr(), emb.numel()
+            desc.global_scale, desc.global_bias = scale.data_ptr(), bias.data_ptr()
+        else:
+            desc.local_bias = local_bias.data_ptr()
+        keep = packs + [decay_bias, local_bias, gparams]
+        self.__dict__["_prefill_plan"] = (key, (desc, keep))
+        return desc, keep
 
     def _prefill(self, u, cross_layer_state, prev_state, cache=None):
         lib = _lib.load()
         dt = u.dtype
         B, L, dm = u.shape
-        D, R = self.d_state, self.ent_rank
+        D = self.d_state
         u = u.contiguous()
         dev = u.device
+        # a copy of the plan's descriptor per call, so calls of several threads do not share one
+        plan, keep = self._layer_plan(dt, dev, cross_layer_state is not None)
+        desc = _lib.SisoLayer.from_buffer_copy(plan)
         y = torch.empty((B, L, dm), dtype=dt, device=dev)
         states = torch.empty((B, L, D), dtype=dt, device=dev)
         h_final = torch.empty((B, D), dtype=torch.float64, device=dev)
-        for p in (self.in_proj, self.state_proj, self.ent_proj, self.out_proj, self.cross_layer_q_proj):
-            if p.weight.dtype != dt:
-                raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
         cs = None
         if cross_layer_state is not None:
             cs = cross_layer_state
@@ -200,36 +248,15 @@ class TESM_SISO(nn.Module):
                 cs = cs.unsqueeze(1).expand(B, L, D)
             cs = cs.to(dt).contiguous()
         h0 = prev_state.to(device=dev, dtype=torch.float64).contiguous() if prev_state is not None else None
-        decay_bias = self._decay_bias_dt(dt)
-        glob = self.entanglement_window <= 0
-        local_bias = None if glob else self._local_bias_f32(dt)
-        gparams = self._global_params_f32(dt) if glob else None
         rope = self.rope_table(L, dt, dev)
-        hip_ops.require_device(u, cs, h0, decay_bias, local_bias, rope, y, states, h_final,
-                               *(gparams if gparams is not None else ()))
-        desc = _lib.SisoLayer()
-        desc.dt = hip_ops.dt_code(dt)
-        desc.B, desc.L, desc.d_model, desc.d_state, desc.ent_rank = B, L, dm, D, R
-        desc.window, desc.chunk_size = max(self.entanglement_window, 0), self.state_scan_chunk_size
-        desc.bit_eps = self.in_proj.bit_eps
-        desc.thr = hip_ops.round_dtype(self.entanglement_threshold, dt)
-        desc.ent_scale = float(self.entanglement_scale)
+        hip_ops.require_device(u, cs, h0, rope, y, states, h_final)
+        desc.B, desc.L = B, L
         desc.u = u.data_ptr()
-        desc.in_proj = self.in_proj.linear_desc()
-        desc.state_proj = self.state_proj.linear_desc()
-        desc.ent_proj = self.ent_proj.linear_desc()
-        desc.out_proj = self.out_proj.linear_desc()
         if cs is not None:
-            desc.cross_q_proj = self.cross_layer_q_proj.linear_desc()
             desc.cross_state = cs.data_ptr()
-        desc.decay_bias = decay_bias.data_ptr()
-        desc.local_bias = local_bias.data_ptr() if local_bias is not None else None
-        if gparams is not None:
-            emb, scale, bias = gparams
-            desc.global_embed, desc.global_dim = emb.data_ptr(), emb.numel()
-            desc.global_scale, desc.global_bias = scale.data_ptr(), bias.data_ptr()
         desc.rope = rope.data_ptr()
-        desc.h0 = h0.data_ptr() if h0 is not None else None
+        if h0 is not None:
+            desc.h0 = h0.data_ptr()
         desc.y = y.data_ptr()
         desc.states = states.data_ptr()
         desc.h_final = h_final.data_ptr()
@@ -239,11 +266,11 @@ class TESM_SISO(nn.Module):
             desc.k_cache, desc.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
             desc.cache_dt = hip_ops.dt_code(k_cache.dtype)
             desc.cache_window = k_cache.shape[1]
-        nbytes = int(lib.tesm_hip_siso_prefill_ws_bytes(ctypes.byref(desc)))
-        with torch.cuda.device(dev):
-            ws = workspace(dev, nbytes)
-            _lib.check(lib.tesm_hip_siso_prefill(ctypes.byref(desc), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
-                                                 ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)))
+        ref = ctypes.byref(desc)
+        nbytes = int(lib.tesm_hip_siso_prefill_ws_bytes(ref))
+        raw = raw_stream(dev.index)
+        ws = workspace(dev, nbytes, raw=raw)
+        on_device(dev.index, lib.tesm_hip_siso_prefill, ref, ws.data_ptr(), ws.numel(), raw)
         if cache is not None:  # tesm.py:1240-1252
             cache["state"] = h_final.clone()
             cache["seq_pos"] = L

@@ -22,7 +22,8 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, check_hip_call
+from .bitlinear import BitLinear, check_hip_call, packed_weights, same_packs
+from .hip_ops import on_device, raw_stream
 from .tesm import TESM_SISO, workspace
 
 
@@ -120,6 +121,51 @@ class TESMMIMO_Optimized(TESM_SISO):
             self._coef_cache = (key, coef, x0sq)
         return self._coef_cache[1], self._coef_cache[2]
 
+    def _mimo_layer_plan(self, dt, dev):
+        """The prefill descriptor's fields that depend on the module alone (see TESM_SISO._layer_plan)."""
+        mods, params = self._modules, self._parameters
+        lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"])
+        glob = self.entanglement_window <= 0
+        biases = (params["decay_bias"], params["mimo_x"], params["mimo_o"]) + (
+            (params["global_rel_pos_embed"], params["global_rel_pos_scale"], params["global_rel_pos_bias"]) if glob else
+            (params["local_entanglement_bias"],))
+        packs = packed_weights(lins, dt, 4)
+        key = (dt, dev, self.entanglement_window, self.entanglement_threshold, float(self.entanglement_scale),
+               lins[0].bit_eps, self.d_model, self.d_state, self.n_heads, self.ent_rank,
+               tuple((b._version, b.data_ptr(), b.dtype) for b in biases))
+        plan = self.__dict__.get("_mimo_plan")
+        if plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
+            return plan[1]
+        decay_bias = self._decay_bias_dt(dt).contiguous()
+        local_bias = None if glob else self._local_bias_f32(dt)
+        gparams = self._global_params_f32(dt) if glob else ()
+        coef, x0sq = self._mimo_coef(dt)
+        hip_ops.require_device(decay_bias, local_bias, coef, x0sq, *gparams)
+        if decay_bias.device != dev:
+            raise RuntimeError(f"hip backend ops need all tensors on one device, got {dev} and {decay_bias.device}")
+        desc = _lib.MimoLayer()
+        desc.dt = hip_ops.dt_code(dt)
+        desc.d_model, desc.d_state, desc.n_heads = self.d_model, self.d_state, self.n_heads
+        desc.ent_rank, desc.window = self.ent_rank, max(self.entanglement_window, 0)
+        desc.bit_eps = self.in_proj.bit_eps
+        desc.thr = hip_ops.round_dtype(self.entanglement_threshold, dt)
+        desc.ent_scale = float(self.entanglement_scale)
+        desc.in_proj = self.in_proj.linear_desc()
+        desc.state_proj = self.state_proj.linear_desc()
+        desc.ent_proj = self.ent_proj.linear_desc()
+        desc.out_proj = self.out_proj.linear_desc()
+        desc.decay_bias = decay_bias.data_ptr()
+        if glob:
+            emb, scale, bias = gparams
+            desc.global_embed, desc.global_dim = emb.data_ptr(), emb.numel()
+            desc.global_scale, desc.global_bias = scale.data_ptr(), bias.data_ptr()
+        else:
+            desc.local_bias = local_bias.data_ptr()
+        desc.mimo_coef, desc.mimo_x0sq = coef.data_ptr(), x0sq.data_ptr()
+        keep = packs + [decay_bias, local_bias, gparams, coef, x0sq]
+        self.__dict__["_mimo_plan"] = (key, (desc, keep))
+        return desc, keep
+
     # -- forward ---------------------------------------------------------------------
     def forward(self, u, inference_params=None, cross_layer_state=None, prev_state=None, **kwargs):
         """Prefill forward (tesm_mimo.py:914-1062); returns ``(y, rank-0 final state float64)``.
@@ -138,44 +184,21 @@ class TESMMIMO_Optimized(TESM_SISO):
             if cache is None or "state" not in cache:
                 cache = None
         dt = u.dtype
-        H, D, R = self.n_heads, self.d_state, self.ent_rank
+        H, D = self.n_heads, self.d_state
         dev = u.device
-        for p in (self.in_proj, self.state_proj, self.ent_proj, self.out_proj):
-            if p.weight.dtype != dt:
-                raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
         u = u.contiguous()
+        # a copy of the plan's descriptor per call, so calls of several threads do not share one
+        plan, keep = self._mimo_layer_plan(dt, dev)
+        desc = _lib.MimoLayer.from_buffer_copy(plan)
         y = torch.empty((B, L, dm), dtype=dt, device=dev)
         h_final = torch.empty((B, H, D), dtype=torch.float64, device=dev)
         last = torch.empty((B, H, D), dtype=torch.float32, device=dev)
-        decay_bias = self._decay_bias_dt(dt).contiguous()
-        glob = self.entanglement_window <= 0
-        local_bias = None if glob else self._local_bias_f32(dt)
-        gparams = self._global_params_f32(dt) if glob else None
         rope = self.rope_table(L, dt, dev)
-        coef, x0sq = self._mimo_coef(dt)
-        hip_ops.require_device(u, decay_bias, local_bias, rope, coef, x0sq, y, h_final, last,
-                               *(gparams if gparams is not None else ()))
+        hip_ops.require_device(u, rope, y, h_final, last)
         lib = _lib.load()
-        desc = _lib.MimoLayer()
-        desc.dt = hip_ops.dt_code(dt)
-        desc.B, desc.L, desc.d_model, desc.d_state, desc.n_heads = B, L, dm, D, H
-        desc.ent_rank, desc.window = R, max(self.entanglement_window, 0)
-        desc.bit_eps = self.in_proj.bit_eps
-        desc.thr = hip_ops.round_dtype(self.entanglement_threshold, dt)
-        desc.ent_scale = float(self.entanglement_scale)
+        desc.B, desc.L = B, L
         desc.u = u.data_ptr()
-        desc.in_proj = self.in_proj.linear_desc()
-        desc.state_proj = self.state_proj.linear_desc()
-        desc.ent_proj = self.ent_proj.linear_desc()
-        desc.out_proj = self.out_proj.linear_desc()
-        desc.decay_bias = decay_bias.data_ptr()
-        desc.local_bias = local_bias.data_ptr() if local_bias is not None else None
-        if gparams is not None:
-            emb, scale, bias = gparams
-            desc.global_embed, desc.global_dim = emb.data_ptr(), emb.numel()
-            desc.global_scale, desc.global_bias = scale.data_ptr(), bias.data_ptr()
         desc.rope = rope.data_ptr()
-        desc.mimo_coef, desc.mimo_x0sq = coef.data_ptr(), x0sq.data_ptr()
         desc.y = y.data_ptr()
         desc.h_final = h_final.data_ptr()
         desc.last_state = last.data_ptr()
@@ -187,19 +210,18 @@ class TESMMIMO_Optimized(TESM_SISO):
             desc.k_cache, desc.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
             desc.cache_dt = hip_ops.dt_code(k_cache.dtype)
             desc.cache_window = k_cache.shape[1]
-        nbytes = int(lib.tesm_hip_mimo_prefill_ws_bytes(ctypes.byref(desc)))
-        with torch.cuda.device(dev):
-            ws = workspace(dev, nbytes)
-            _lib.check(lib.tesm_hip_mimo_prefill(ctypes.byref(desc), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
-                                                 ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)))
+        ref = ctypes.byref(desc)
+        nbytes = int(lib.tesm_hip_mimo_prefill_ws_bytes(ref))
+        raw = raw_stream(dev.index)
+        ws = workspace(dev, nbytes, raw=raw)
+        on_device(dev.index, lib.tesm_hip_mimo_prefill, ref, ws.data_ptr(), ws.numel(), raw)
         if cache is not None:  # tesm_mimo.py:1022-1037
             cache["state"] = h_final.clone()
             cache["seq_pos"] = L
             cache["ent_k_cache"], cache["ent_v_cache"] = k_cache, v_cache
             cache["cache_idx"] = 0
-        self._last_cross_layer_state = last
-        self._last_scan_state_f64 = h_final
-        self.last_entanglement_map = None
+        # plain attributes, set without nn.Module.__setattr__'s microsecond each (as in the SISO layer)
+        self.__dict__.update(_last_cross_layer_state=last, _last_scan_state_f64=h_final, last_entanglement_map=None)
         flat = stern.reshape(-1)  # tesm_mimo.py:506-519
         total = float(flat.numel())
         key = (total, dev)
@@ -331,18 +353,13 @@ class TESMMIMO_Optimized(TESM_SISO):
         desc.k_cache, desc.v_cache = kc.data_ptr(), vc.data_ptr()
         desc.y = y.data_ptr()
         desc.new_state = new.data_ptr()
-        stream = torch.cuda.current_stream(dev)
-        with torch.cuda.device(dev):
-            ws = workspace(dev, nbytes, stream)
-            rc = lib.tesm_hip_mimo_decode(ctypes.byref(desc), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
-                                          ctypes.c_void_p(stream.cuda_stream))
-        _lib.check(rc)
+        raw = raw_stream(dev.index)
+        ws = workspace(dev, nbytes, raw=raw)
+        on_device(dev.index, lib.tesm_hip_mimo_decode, ctypes.byref(desc), ws.data_ptr(), ws.numel(), raw)
         cache["cache_idx"] = (slot + 1) % W
         cache["state"] = state_out
         cache["seq_pos"] = pos + 1
-        self._last_cross_layer_state = new
-        self._last_scan_state_f64 = state_out
-        self.last_entanglement_map = None
+        self.__dict__.update(_last_cross_layer_state=new, _last_scan_state_f64=state_out, last_entanglement_map=None)
         return y, state_out
 
     def _mimo_cache_buffers(self, cache, B, L, dev):

@@ -1,0 +1,120 @@
+"""The layers' descriptor plans (fields kept from call to call): every change a user can make to a module between
+two calls reaches the next call, a copied or reloaded module does not use another's plan, and calls from several
+threads on streams of their own do not disturb each other."""
+import copy
+import io
+import threading
+
+import pytest
+import torch
+
+from hip_helpers import DEV, need_gpu
+from tesm_amd import FeedForward, TESM_SISO, TESMConfig, TESMMIMO_Optimized
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _gpu():
+    need_gpu()
+
+
+def _make(kind, dtype=torch.float32, seed=0):
+    torch.manual_seed(seed)
+    if kind == "ffn":
+        m = FeedForward(TESMConfig(d_model=64, d_intermediate=128))
+    elif kind == "mimo":
+        m = TESMMIMO_Optimized(d_model=64, d_state=32, n_heads=2, ent_rank=8, entanglement_window=8,
+                               entanglement_threshold=0.08, max_seq_len=64)
+    else:
+        m = TESM_SISO(d_model=64, d_state=32, ent_rank=8, entanglement_window=8 if kind == "siso" else 0,
+                      entanglement_threshold=0.08, max_seq_len=64)
+    return m.to(DEV).to(dtype).eval()
+
+
+def _out(m, u):
+    with torch.no_grad():
+        out = m(u)
+    return out[0] if isinstance(out, tuple) else out
+
+
+def _u(dtype=torch.float32, L=40, seed=1):
+    return torch.randn(2, L, 64, generator=torch.Generator().manual_seed(seed)).to(dtype).to(DEV)
+
+
+KINDS = ["siso", "global", "mimo", "ffn"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_weight_and_option_changes_reach_the_next_call(kind):
+    """Each change is compared with a module that never had a plan."""
+    m, u = _make(kind), _u()
+    _out(m, u)
+    other = _make(kind, seed=5)
+    first = "gate_proj" if kind == "ffn" else "in_proj"
+    edits = [lambda x: getattr(x, first).weight.data.mul_(-1.0).add_(0.01),        # in place through .data + version
+             lambda x: setattr(x, first, copy.deepcopy(getattr(other, first))),       # a replaced submodule
+             lambda x: getattr(x, first).__setattr__("weight", torch.nn.Parameter(getattr(other, first).weight * 0.5))]
+    if kind != "ffn":
+        edits += [lambda x: x.decay_bias.add_(0.5), lambda x: setattr(x, "entanglement_threshold", 0.3)]
+    for i, edit in enumerate(edits):
+        with torch.no_grad():
+            edit(m)
+            if i == 0:
+                getattr(m, first).weight.add_(0.0)  # bump the version the packed cache follows
+        fresh = _make(kind)
+        fresh.load_state_dict(m.state_dict())
+        if kind != "ffn":
+            fresh.entanglement_threshold = m.entanglement_threshold
+        assert torch.equal(_out(m, u), _out(fresh, u)), (kind, i)
+        assert torch.equal(_out(m, _u(L=17, seed=9)), _out(fresh, _u(L=17, seed=9))), (kind, i)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_copied_and_reloaded_modules(kind):
+    m, u = _make(kind), _u()
+    want = _out(m, u)
+    twin = copy.deepcopy(m)
+    buf = io.BytesIO()
+    torch.save(m, buf)
+    buf.seek(0)
+    loaded = torch.load(buf, weights_only=False)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.zero_()
+    del m
+    for x in (twin, loaded):
+        assert torch.equal(_out(x, u), want)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_dtype_mismatch_still_refused(kind):
+    m = _make(kind)
+    _out(m, _u())
+    with pytest.raises(RuntimeError, match="same dtype"):
+        _out(m, _u(torch.bfloat16))
+
+
+def test_threads_on_their_own_streams():
+    m = _make("siso")
+    us = [_u(L=8 + 7 * i, seed=20 + i) for i in range(4)]
+    want = [_out(m, u) for u in us]
+    torch.cuda.synchronize()
+    got, errors = [None] * 4, []
+
+    def work(i):
+        try:
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                for _ in range(20):
+                    got[i] = _out(m, us[i])
+            s.synchronize()
+        except Exception as e:  # noqa: BLE001 - reported below
+            errors.append(e)
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join(60) for t in ts]
+    assert not errors
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
