@@ -1701,6 +1701,15 @@ int launch_linear_fq(const LinearArgs& a, const FusedQuantIn& f, hipStream_t st)
   return check_launch("bitlinear skinny (fused quant)");
 }
 
+// The 32x32x32 kernels address a tile's rows (up to 128 of codes, 256 of weights) with 32-bit offsets; longer rows
+// take the split-K kernel, which walks any number of 32-row tiles.
+static bool tiles32_ok(const LinearArgs& a) {
+  const int np = epi_dual(a.epilogue) ? 2 : 1;
+  for (int p = 0; p < np; ++p)
+    if (a.op[p].ldq >= (int64_t(1) << 24) || a.op[p].ldw >= (int64_t(1) << 23)) return false;
+  return true;
+}
+
 int launch_linear(const LinearArgs& a, hipStream_t st) {
   TESM_REQUIRE(a.M >= 0 && a.N >= 0, kErrInvalidArg, "bitlinear: negative size");
   TESM_REQUIRE(a.Kp >= kKTile && a.Kp % kKTile == 0, kErrInvalidArg, "bitlinear: Kp must be a positive multiple of 128");
@@ -1715,6 +1724,7 @@ int launch_linear(const LinearArgs& a, hipStream_t st) {
     TESM_REQUIRE(a.M > 32 && !a.bias && !a.acc_dump && !a.op[0].c_w_per_row && a.act_bias && a.act_w > 0 &&
                      a.act_n0 >= 0 && a.act_n0 % 32 == 0 && a.act_w % 32 == 0 && a.act_n0 + 3 * a.act_w <= a.N,
                  kErrUnsupported, "bitlinear gates epilogue: needs M > 32, 32-aligned regions inside N, no bias");
+    TESM_REQUIRE(tiles32_ok(a), kErrUnsupported, "bitlinear gates epilogue: code rows too long");
     return launch_mfma32(a, st);
   }
   if (a.epilogue != kEpiStore) {
@@ -1734,12 +1744,12 @@ int launch_linear(const LinearArgs& a, hipStream_t st) {
     // decode-size batches: the split-K kernel while the LDS-staged one would have too few 64-column
     // tiles to fill the chip (measured at M = 32: N = 768 .. 4096 faster split, N = 34816 staged)
     if (a.M <= 16 && a.N < 16384) return run_skinny<4, 1, 1, kEpiStore>(a, st);
-    if (a.M <= 32 && a.N < 16384) return run_skinny<4, 2, 1, kEpiStore>(a, st);
+    if ((a.M <= 32 && a.N < 16384) || !tiles32_ok(a)) return run_skinny<4, 2, 1, kEpiStore>(a, st);
     return launch_mfma32(a, st);
   }
   // two-product epilogues: split-K for decode-size batches, else the 32x32 kernels
   if (a.M <= 16) return a.epilogue == kEpiOutputGate ? run_skinny<4, 1, 1, kEpiOutputGate>(a, st) : run_skinny<4, 1, 1, kEpiSwiGLU>(a, st);
-  if (a.M <= 32) return a.epilogue == kEpiOutputGate ? run_skinny<4, 2, 1, kEpiOutputGate>(a, st) : run_skinny<4, 2, 1, kEpiSwiGLU>(a, st);
+  if (a.M <= 32 || !tiles32_ok(a)) return a.epilogue == kEpiOutputGate ? run_skinny<4, 2, 1, kEpiOutputGate>(a, st) : run_skinny<4, 2, 1, kEpiSwiGLU>(a, st);
   return launch_mfma32(a, st);
 }
 

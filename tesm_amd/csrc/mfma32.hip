@@ -8,16 +8,17 @@
 // weight dwords of a K tile one 16-byte read.  Accumulator element r of lane L is weight column
 // 8*(r/4) + 4*(L/32) + r%4 and activation row L%32.
 //
-// Pipeline.  K tiles go straight from memory to LDS (global_load_lds_dwordx4, no staging registers) into NS
-// stages.  A fragment's LDS reads are issued one k-step ahead of its MFMAs, across the K tile boundary too: the
+// Pipeline.  K tiles go straight from memory to LDS (16-byte buffer loads with the LDS destination, no staging
+// registers) into NS stages.  A fragment's LDS reads are issued one k-step ahead of its MFMAs, across the K tile boundary too: the
 // one barrier of a K tile stands in its middle, where a wave (a) knows its loads of the next tile landed
 // (vmcnt), (b) meets the others, so the next tile may be read from the last k-step on and the previous tile's
 // stage may be refilled.  With the wait at a tile's start instead, and two stages, every tile paid an LDS round
-// trip and the slowest wave's load (2048 x 4096 x 4096: 37.6 -> 34.7 us; 4095 x 3840 x 1024: 28.3 -> 21.0).
+// trip and the slowest wave's load (2048 x 4096 x 4096: 37.6 -> 35 us; 4095 x 3744 x 1024: 28.3 -> 21.2).
 //
 // What bounds it: large products run at 2.1-2.3 POP/s, where the chip's power limit lies for these operands (the
 // library int8 product reaches 2.25 on random codes; the same kernel on all-zero codes is 1.3 times faster; tiles
-// from 128x128 to 256x256, 64x64 to 128x64 per wave and 2 to 4 stages all end within 10 % of each other).  Small
+// from 128x128 to 256x256, 64x64 to 128x64 per wave and 2 to 4 stages all end within 10 % of each other):
+// 8192 x 34816 x 4096 1055 us, 4096 x 14848 x 4096 231 (the two-stage loop 1111 and 262).  Small
 // ones are bound by the latency of the first tiles and by idle CUs, hence the K groups: KS groups of waves
 // in one workgroup take K tiles g, g + KS, ... into stages of their own, and their exact int32 sums are added in
 // LDS, so a 32 x 64 tile with a quarter of the K loop per group replaces 64 x 128 tiles on a fifth of the CUs
@@ -37,6 +38,17 @@
 namespace tesm {
 
 namespace {
+
+// Loads to LDS through a buffer resource rather than global_load_lds: the compiler counts that instruction as one
+// that may also touch LDS out of order, and waits for every outstanding LDS read (lgkmcnt(0)) wherever one is
+// needed while such a load is in flight, which undoes the fragment prefetch (4096 x 14848 x 4096: 242 us, 231 with
+// buffer loads; 8192 x 34816 x 4096: 1108, 1056).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffffu, 0x00027000);
+}
+__device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t buf, char* dst, uint32_t off, int koff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (__attribute__((address_space(3))) void*)(dst), 16, off, koff, 0, 0);
+}
 
 __device__ __forceinline__ int a32_off(int row, int q) { return 16 * (row * 8 + (q ^ ((row >> 1) & 7))); }
 __device__ __forceinline__ int b32_off(int col, int h) { return 16 * (col * 2 + (h ^ ((col >> 3) & 1))); }
@@ -60,7 +72,6 @@ struct Tile32 {
   static constexpr int SLAB = 32 * (TN * 32 * ES + 16);              // a wave's 32 rows x TN column tiles
   static constexpr int SMEM = std::max(NS * STAGE, RED + NG * SLAB);
   static_assert(NS >= 3 && (NS - 2) * D < 64, "loads in flight");
-  static_assert(!(EPI == kEpiOutputGate && KS > 1), "the gate's products follow each other in one group");
 };
 
 // acc[p][i][j]: product p, row tile i, column tile j of the wave's group (with KS > 1 a partial sum).
@@ -73,52 +84,51 @@ __device__ __forceinline__ void mfma32_loop(const LinearArgs& a, int64_t m0, int
   const int kg = wall / T::NG, w = wall % T::NG;
   const int wm = w / WN, wn = w % WN;
   constexpr int SEQ = T::DUAL && !T::SHARE ? 2 : 1;  // products one after the other
-  // this lane's source of each of the wave's D blocks (rows past M and columns past N re-read the last one and
-  // feed only outputs that are never stored), and the K group each block belongs to
-  const char* src[SEQ][T::D];
+  // Each of the wave's D blocks: its buffer (the tile's rows of an operand, so offsets fit 32 bits), the lane's
+  // offset in it (rows past M and columns past N re-read the last one and feed only outputs that are never stored),
+  // and its K group.  The K position is the scalar offset, so a load costs no address arithmetic.
+  __amdgpu_buffer_rsrc_t buf[SEQ][T::D];
+  uint32_t off[SEQ][T::D];
   int dst[T::D], adv[T::D], grp[T::D];
 #pragma unroll
   for (int i = 0; i < T::D; ++i) {
     const int b0 = wall + i * T::NW, blk = b0 < T::PER * KS ? b0 : T::PER * KS - 1;
     const int g = blk / T::PER, bb = blk % T::PER;
-    grp[i] = g;
+    const bool is_q = bb < T::NA;
+    const int wt = T::SHARE && bb >= T::NA + T::NB ? 1 : 0, cb = (bb - T::NA) % T::NB;
+    const int row = is_q ? bb * 8 + (lane >> 3) : cb * 32 + (lane >> 1);  // row of the tile, or column
+    const int chunk = is_q ? (lane & 7) ^ ((row >> 1) & 7) : (lane & 1) ^ ((row >> 3) & 1);
+    const int64_t last = is_q ? a.M - 1 - m0 : a.N - 1 - n0;
 #pragma unroll
     for (int p = 0; p < SEQ; ++p) {
-      if (bb < T::NA) {
-        const LinearOperand& o = a.op[p];
-        const int row = bb * 8 + (lane >> 3);
-        const int q = (lane & 7) ^ ((row >> 1) & 7);
-        const int64_t m = m0 + row;
-        src[p][i] = reinterpret_cast<const char*>(o.q) + (m < a.M ? m : a.M - 1) * o.ldq + 16 * q;
-      } else {
-        const int wt = (bb - T::NA) / T::NB, cb = (bb - T::NA) % T::NB;
-        const LinearOperand& o = a.op[T::SHARE ? wt : p];
-        const int col = cb * 32 + (lane >> 1);
-        const int h = (lane & 1) ^ ((col >> 3) & 1);
-        const int64_t n = n0 + col;
-        src[p][i] = reinterpret_cast<const char*>(o.w) + (n < a.N ? n : a.N - 1) * o.ldw + 16 * h;
-      }
+      const LinearOperand& o = a.op[p];
+      const LinearOperand& ow = a.op[T::SHARE ? wt : p];
+      const char* base = is_q ? reinterpret_cast<const char*>(o.q) + m0 * o.ldq
+                              : reinterpret_cast<const char*>(ow.w) + n0 * ow.ldw;
+      buf[p][i] = tile_buffer(base);
+      off[p][i] = static_cast<uint32_t>((row < last ? row : last) * (is_q ? o.ldq : ow.ldw)) + 16 * chunk;
     }
-    adv[i] = bb < T::NA ? T::BK : T::BK / 4;
+    grp[i] = g;
+    adv[i] = is_q ? T::BK : T::BK / 4;
     dst[i] = g * T::SUB + bb * 1024;  // (A_BYTES and W_BYTES are whole blocks)
   }
   const int nk = static_cast<int>(a.Kp / T::BK);
-  const int steps = SEQ == 2 ? 2 * nk : (nk + KS - 1) / KS;
-  auto issue = [&](int kt, int st) {  // (past the last tile: re-reads it, so every wave's count stays the same)
-    char* stage = smem + st * T::STAGE;
+  const int ns = (nk + KS - 1) / KS;  // steps of one product: a K tile per group
+  const int steps = SEQ * ns;
+  auto issue_p = [&](int kt, char* stage, const __amdgpu_buffer_rsrc_t (&bf)[T::D], const uint32_t (&of)[T::D]) {
 #pragma unroll
     for (int i = 0; i < T::D; ++i) {
-      if constexpr (SEQ == 2) {
-        const int p = kt >= nk ? 1 : 0;
-        int k = kt - p * nk;
-        k = k < nk ? k : nk - 1;
-        lds_dma16((p ? src[SEQ - 1][i] : src[0][i]) + static_cast<int64_t>(k) * adv[i], stage + dst[i]);
-      } else {
-        int k = kt * KS + grp[i];
-        k = k < nk ? k : nk - 1;
-        lds_dma16(src[0][i] + static_cast<int64_t>(k) * adv[i], stage + dst[i]);
-      }
+      int k = kt * KS + grp[i];
+      k = k < nk ? k : nk - 1;  // (past the last tile: re-reads it, so every wave's count stays the same)
+      lds_dma16(bf[i], stage + dst[i], of[i], k * adv[i]);
     }
+  };
+  auto issue = [&](int kt, int st) {
+    char* stage = smem + st * T::STAGE;
+    if (SEQ == 2 && kt >= ns)
+      issue_p(kt - ns, stage, buf[SEQ - 1], off[SEQ - 1]);
+    else
+      issue_p(kt, stage, buf[0], off[0]);
   };
   const int hq = 4 * (lane >> 5);
   int ar[4];
@@ -155,7 +165,7 @@ __device__ __forceinline__ void mfma32_loop(const LinearArgs& a, int64_t m0, int
     const char* cur = smem + st * T::STAGE;
     const int nx = st + 1 == NS ? 0 : st + 1, pv = st == 0 ? NS - 1 : st - 1;
     const char* nxt = smem + nx * T::STAGE;
-    const bool live = KS == 1 || kt * KS + kg < nk;  // (wave-uniform)
+    const bool live = KS == 1 || (kt - prod * ns) * KS + kg < nk;  // (wave-uniform)
     read_a(cur, 1, af[1]);
     __builtin_amdgcn_sched_barrier(0);
     if (live) mma(prod, b, af[0], 0);
@@ -167,7 +177,7 @@ __device__ __forceinline__ void mfma32_loop(const LinearArgs& a, int64_t m0, int
     read_a(cur, 3, af[1]);
     wait_vmcnt<(NS - 3) * T::D>();  // this wave's loads of tile kt + 1 have landed
     __builtin_amdgcn_s_barrier();   // ... every wave's, and every wave is done with tile kt - 1
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    asm volatile("" ::: "memory");  // (orders the compiler only: an acquire fence would wait for the reads above)
     issue(kt + NS - 1, pv);         // into the stage tile kt - 1 used
     __builtin_amdgcn_sched_barrier(0);
     if (live) mma(prod, b, af[0], 2);
@@ -188,11 +198,11 @@ __device__ __forceinline__ void mfma32_loop(const LinearArgs& a, int64_t m0, int
   read_a(smem, 0, af[0]);
   if constexpr (SEQ == 2) {
     int kt = 0;
-    for (; kt + 2 <= nk; kt += 2) {
+    for (; kt + 2 <= ns; kt += 2) {
       tile(kt, 0, bw[0], bw[1]);
       tile(kt + 1, 0, bw[1], bw[0]);
     }
-    if (kt < nk) {  // an odd number of K tiles: the second product starts on the other weight registers
+    if (kt < ns) {  // an odd number of steps: the second product starts on the other weight registers
       tile(kt, 0, bw[0], bw[1]);
       ++kt;
       for (; kt + 2 <= steps; kt += 2) {
@@ -503,15 +513,11 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
   return check_launch("bitlinear mfma32 (K groups)");
 }
 
-#ifdef MFMA32_SWEEP
-#include "sweep.inc"
-#endif
-
 // Tile sizes by grid.  Times in us on one box, bf16 outputs unless noted; "before" is the two-stage, one-group form.
 //   * 128x256 tiles (8 waves of 64x64, two workgroups per CU) when they give every CU one: 2048 x 4096 x 4096 36.2
-//     (64x256 tiles 40), 4095 x 3744 x 1024 22.0 (64x128: 26.3).  Grids past two rounds walk 8 M tiles per group.
+//     (64x256 tiles 40), 4095 x 3744 x 1024 21.2 (64x128: 26.3).  Grids past two rounds walk 8 M tiles per group.
 //   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
-//     kernel: 24.6 against 26.1 for 128x256 tiles throughout.
+//     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
 //   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU: 8192 x 768 x 768 10.6 (128x256: 10.9),
 //     4095 x 1024 x 2816 15.4 (before 21.5), 1000 x 4096 x 4096 21.2 (before 28.3).  A K loop of at most
 //     three tiles stays on this shape too: such calls are launch-bound (16384 x 256 x 256 5.9, best 5.7; 512 x 96 x
@@ -551,13 +557,16 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
 
 // The output gate (two accumulator sets, so one 128x256 workgroup per CU): 4096 x 4096 x 2 x 2048 115 (before 118);
 // 64x128 tiles of eight waves when they give every CU one: 4095 x 1024 x 2 x 512 16.2 (before 28.6); else 32x64
-// tiles of two waves: 512 x 768 x 2 x 384 7.6 (before 12.0), 64 x 4096 x 2 x 8192 36.3 (before 51.4).
+// tiles of two waves: 512 x 768 x 2 x 384 7.6 (before 12.0); at long K with CUs left over, eight K groups on 32x32
+// tiles or four on 32x64: 64 x 4096 x 2 x 8192 24.9 (before 51.4), 100 rows 33.9.
 int dispatch_gate32(const LinearArgs& a, hipStream_t st) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
   const int64_t cus = std::max(device_limits().cus, 1), big = tiles(128, 256);
   if (big >= 8 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 2>(a, st);
   if (big >= 2 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 0>(a, st);
   if (tiles(64, 128) >= cus) return run_mfma32<2, 4, 1, 1, kEpiOutputGate, 0>(a, st);
+  if (a.Kp >= 4096 && tiles(32, 64) < cus) return run_mfma32k<1, 1, 1, 1, 8, 3, kEpiOutputGate>(a, st);
+  if (a.Kp >= 4096 && tiles(32, 64) < 2 * cus) return run_mfma32k<1, 2, 1, 1, 4, 3, kEpiOutputGate>(a, st);
   return run_mfma32<1, 2, 1, 1, kEpiOutputGate, 0>(a, st);
 }
 
@@ -570,16 +579,9 @@ int dispatch_swiglu32(const LinearArgs& a, hipStream_t st) {
   return run_mfma32<2, 2, 1, 1, kEpiSwiGLU, 0>(a, st);
 }
 
-#ifdef MFMA32_SWEEP
-#include "sweep.inc"
-#endif
-
 }  // namespace
 
 int launch_mfma32(const LinearArgs& a, hipStream_t st) {
-#ifdef MFMA32_SWEEP
-  if (const int rc = sweep_run(a, st); rc >= 0) return rc;
-#endif
   if (a.epilogue == kEpiGates) return dispatch_store32<kEpiGates>(a, st);
   if (a.epilogue == kEpiStore) return dispatch_store32<kEpiStore>(a, st);
   if (a.epilogue == kEpiOutputGate) return dispatch_gate32(a, st);
