@@ -1065,9 +1065,6 @@ int tesm_hip_siso_prefill(const tesm_hip_siso_layer* pp, void* ws, int64_t ws_by
   ea.eps = p.bit_eps;
   if (tapping) ea.tern = tp.tern;
   if (p.window == 0) {  // global causal entanglement (tesm.py:963-1063), then the same quantizations
-    if ((rc = launch_global_bias_table(dt, 2 * p.L, p.global_embed, p.global_dim, p.global_scale, p.global_bias,
-                                       s.g_table, st)))
-      return rc;
     GlobalArgs ga;
     ga.dt = dt;
     ga.mimo = 0;
@@ -1097,11 +1094,35 @@ int tesm_hip_siso_prefill(const tesm_hip_siso_layer* pp, void* ws, int64_t ws_by
     ga.states_t = s.g_st;
     ga.qr = s.g_qr;
     ga.kr = s.g_kr;
-    if ((rc = launch_global_ent(ga, st))) return rc;
+    ga.embed = p.global_embed;
+    ga.P = p.global_dim;
+    ga.rel_scale = p.global_scale;
+    ga.rel_bias = p.global_bias;
+    const bool one_pass = global_mfma_ok(ga), quantized = global_mfma_quantizes(ga);
+    if (one_pass) {
+      ga.tap_tern = tapping && tp.tern;
+      if (quantized) {
+        ga.q_te = s.xe.q;
+        ga.s_te = s.xe.s;
+        ga.rs_te = s.xe.rs;
+        ga.q_c = s.xc.q;
+        ga.s_c = s.xc.s;
+        ga.rs_c = s.xc.rs;
+        ga.ldq = s.xe.ldq;
+        ga.eps = p.bit_eps;
+        if (!tapping) ga.e_tanh = ga.c_out = nullptr;  // only the codes are needed
+      }
+      if ((rc = launch_global_mfma(ga, st))) return rc;
+    } else {
+      if ((rc = launch_global_bias_table(dt, 2 * p.L, p.global_embed, p.global_dim, p.global_scale, p.global_bias,
+                                         s.g_table, st)))
+        return rc;
+      if ((rc = launch_global_ent(ga, st))) return rc;
+    }
     if (tapping && (rc = tap_copy(tp.tern, s.g_tern, M * global_tern_pitch(p.L), st))) return rc;
     if (tapping && (rc = tap_copy(tp.te, s.e_tanh, M * D * es, st))) return rc;
     if (tapping && (rc = tap_copy(tp.c, s.c_mix, M * D * es, st))) return rc;
-    if ((rc = quant_te_c(s.e_tanh, s.c_mix, dt, M, D, p.bit_eps, s.xe, s.xc, st))) return rc;
+    if (!quantized && (rc = quant_te_c(s.e_tanh, s.c_mix, dt, M, D, p.bit_eps, s.xe, s.xc, st))) return rc;
   } else if (s.fuse_ent) {
     ea.q_te = s.xe.q;
     ea.s_te = s.xe.s;

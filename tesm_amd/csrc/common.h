@@ -295,6 +295,14 @@ __device__ __forceinline__ uint4 group_codes(const float (&v)[16], float sc, int
   return out;
 }
 
+// A 16-code group from natural order to layout 1 (byte 4s + j holds code 4j + s): a 4 x 4 byte transpose.
+__device__ __forceinline__ uint4 natural_to_layout1(uint4 n) {
+  const uint32_t a0 = __builtin_amdgcn_perm(n.y, n.x, 0x05010400u), a1 = __builtin_amdgcn_perm(n.w, n.z, 0x05010400u);
+  const uint32_t b0 = __builtin_amdgcn_perm(n.y, n.x, 0x07030602u), b1 = __builtin_amdgcn_perm(n.w, n.z, 0x07030602u);
+  return make_uint4(__builtin_amdgcn_perm(a1, a0, 0x05040100u), __builtin_amdgcn_perm(a1, a0, 0x07060302u),
+                    __builtin_amdgcn_perm(b1, b0, 0x05040100u), __builtin_amdgcn_perm(b1, b0, 0x07060302u));
+}
+
 // ---------------------------------------------------------------------------
 // wave64 reductions
 // ---------------------------------------------------------------------------

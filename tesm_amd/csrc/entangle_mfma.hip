@@ -365,16 +365,8 @@ __global__ __launch_bounds__(kMmNT) void ent_mfma_kernel(EntArgs e, int weff, Mm
   for (int i = tid; i < 2 * kMmTP * ngq; i += kMmNT) {
     const int g = i % ngq, row = i / ngq, pp = row & (kMmTP - 1), q = row >> 4;
     if (t0 + pp >= L) continue;
-    uint4 o = make_uint4(0, 0, 0, 0);
-    if (g < groups) {  // natural order -> layout 1 (byte 4s + j holds code 4j + s): a 4 x 4 byte transpose
-      const uint4 n = *reinterpret_cast<const uint4*>(code + row * cp + 4 * g);
-      const uint32_t a0 = __builtin_amdgcn_perm(n.y, n.x, 0x05010400u), a1 = __builtin_amdgcn_perm(n.w, n.z, 0x05010400u);
-      const uint32_t b0 = __builtin_amdgcn_perm(n.y, n.x, 0x07030602u), b1 = __builtin_amdgcn_perm(n.w, n.z, 0x07030602u);
-      o.x = __builtin_amdgcn_perm(a1, a0, 0x05040100u);
-      o.y = __builtin_amdgcn_perm(a1, a0, 0x07060302u);
-      o.z = __builtin_amdgcn_perm(b1, b0, 0x05040100u);
-      o.w = __builtin_amdgcn_perm(b1, b0, 0x07060302u);
-    }
+    const uint4 o = g < groups ? natural_to_layout1(*reinterpret_cast<const uint4*>(code + row * cp + 4 * g))
+                               : make_uint4(0, 0, 0, 0);
     reinterpret_cast<uint4*>((q == 0 ? e.q_te : e.q_c) + (b * L + t0 + pp) * e.ldq)[g] = o;
   }
   if (wv == 0 && q4 < 2 && t < L) {  // lanes 0-15: tanh(E)'s scale and code sum, lanes 16-31: C's

@@ -44,11 +44,62 @@ struct GlobalArgs {
   uint16_t* states_t = nullptr;  // workspace (B, H*D, ldt) bf16 states transposed (bf16 SISO layers only)
   float* qr = nullptr;           // workspace (B, L, H*R) RoPE'd queries (+ cross-layer bias)
   float* kr = nullptr;           // workspace (B, L, H*R) RoPE'd keys
+  // the one-pass kernel (global_mfma.hip): the bias parameters (it fills the table itself), whether to leave the
+  // decisions in tern, and the int8 codes of tanh(E) and C (layout 1), formed in place where q_te is set and
+  // global_mfma_quantizes; e_tanh and c_out may then be null
+  const float* embed = nullptr;
+  int64_t P = 0;
+  const float* rel_scale = nullptr;
+  const float* rel_bias = nullptr;
+  bool tap_tern = false;
+  int8_t* q_te = nullptr;
+  float* s_te = nullptr;
+  int32_t* rs_te = nullptr;
+  int8_t* q_c = nullptr;
+  float* s_c = nullptr;
+  int32_t* rs_c = nullptr;
+  int64_t ldq = 0;
+  float eps = 1e-5f;
 };
+
+__device__ __forceinline__ int64_t round_up64(int64_t v) { return (v + 63) & ~int64_t(63); }
+
+// One entry of the bias table per eight lanes (lane `e & 7` of entry `e >> 3`, each over every eighth frequency; the
+// partial sums meet by shuffles).
+template <int DT>
+__device__ __forceinline__ void global_bias_entry(int64_t e, int64_t n, const float* embed, int64_t P,
+                                                  const float* scale, const float* bias, float* table) {
+  const int64_t r = e >> 3;
+  const int part = static_cast<int>(e & 7);
+  const float rel = rnd<DT>(static_cast<float>(r < n ? r : 0));
+  constexpr float kPi = 3.14159265358979323846f;
+  float ssum = 0.0f, csum = 0.0f;
+  for (int64_t p = part; p < P; p += 8) {
+    const float fr = rnd<DT>(rnd<DT>(static_cast<float>(p + 1) * kPi) / 1000.0f);
+    const float ang = rnd<DT>(rel * fr);
+    const float em = embed[p];
+    ssum += rnd<DT>(rnd<DT>(sinf(ang)) * em);
+    csum += rnd<DT>(rnd<DT>(cosf(ang)) * em);
+  }
+#pragma unroll
+  for (int o = 4; o > 0; o >>= 1) {
+    ssum += __shfl_xor(ssum, o);
+    csum += __shfl_xor(csum, o);
+  }
+  if (r >= n || part != 0) return;
+  const float b = rnd<DT>(rnd<DT>(ssum) + rnd<DT>(csum));
+  table[r] = rnd<DT>(rnd<DT>(b * scale[0]) + bias[0]);
+}
 
 int64_t global_tern_pitch(int64_t L);
 // bytes of the transposed-states workspace (zero where the states are float32)
 int64_t global_states_t_bytes(int dt, int mimo, int64_t B, int64_t L, int64_t C);
+int check_global(const GlobalArgs& a);  // sizes and inputs, as both paths need them
 int launch_global_ent(const GlobalArgs& a, hipStream_t st);
+
+// Scores, decisions and mix in one pass over the keys: the layers it takes, whether it also quantizes, its launch.
+bool global_mfma_ok(const GlobalArgs& a);
+bool global_mfma_quantizes(const GlobalArgs& a);
+int launch_global_mfma(const GlobalArgs& a, hipStream_t st);
 
 }  // namespace tesm

@@ -15,6 +15,9 @@
 // epilogue is the layer's post-processing (SISO: E = S + scale (A - S), tanh(E), E - S; MIMO: the
 // rank merge tanh(A c), (A - S) c).
 //
+// These kernels serve float32 and MIMO layers and the bf16 single-head shapes that global_mfma_ok leaves out; the
+// others take scores, decisions and mix in one kernel (global_mfma.hip).
+//
 // MFMA 32x32 lane layout used throughout: lane L supplies row L % 32 of A and column L % 32 of B, its
 // k values in an order shared by both operands (so any assignment of the contraction index to
 // (L / 32, element) that is the same for A and B is a valid product); accumulator element r of lane L
@@ -60,27 +63,7 @@ __device__ __forceinline__ float tern_f(uint32_t w, int s) {
 template <int DT>
 __global__ __launch_bounds__(256) void global_bias_table_kernel(int64_t n, const float* embed, int64_t P,
                                                                 const float* scale, const float* bias, float* table) {
-  // eight lanes per entry, each over every eighth frequency; the partial sums meet by shuffles
-  const int64_t r = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) >> 3;
-  const int part = threadIdx.x & 7;
-  const float rel = rnd<DT>(static_cast<float>(r < n ? r : 0));
-  constexpr float kPi = 3.14159265358979323846f;
-  float ssum = 0.0f, csum = 0.0f;
-  for (int64_t p = part; p < P; p += 8) {
-    const float fr = rnd<DT>(rnd<DT>(static_cast<float>(p + 1) * kPi) / 1000.0f);
-    const float ang = rnd<DT>(rel * fr);
-    const float e = embed[p];
-    ssum += rnd<DT>(rnd<DT>(sinf(ang)) * e);
-    csum += rnd<DT>(rnd<DT>(cosf(ang)) * e);
-  }
-#pragma unroll
-  for (int o = 4; o > 0; o >>= 1) {
-    ssum += __shfl_xor(ssum, o);
-    csum += __shfl_xor(csum, o);
-  }
-  if (r >= n || part != 0) return;
-  const float b = rnd<DT>(rnd<DT>(ssum) + rnd<DT>(csum));
-  table[r] = rnd<DT>(rnd<DT>(b * scale[0]) + bias[0]);
+  global_bias_entry<DT>(static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, n, embed, P, scale, bias, table);
 }
 
 // RoPE'd queries (+ cross-layer bias) and keys, once: qr / kr (b, t, c) at [(b*L + t)*RQ + c], RQ = H*R,
@@ -384,26 +367,34 @@ int64_t global_states_t_bytes(int dt, int mimo, int64_t B, int64_t L, int64_t C)
   return dt == kBF16 && !mimo ? B * C * global_tern_pitch(L) * 2 : 0;
 }
 
-int launch_global_ent(const GlobalArgs& a, hipStream_t st) {
+int check_global(const GlobalArgs& a) {
   TESM_REQUIRE(a.dt == kF32 || a.dt == kBF16, kErrInvalidArg, "global ent: dtype must be 0 or 1");
   TESM_REQUIRE(a.B >= 0 && a.L >= 0 && a.H >= 1 && a.R >= 2 && a.R % 2 == 0 && a.D >= 1, kErrInvalidArg,
                "global ent: bad sizes (need an even ent_rank)");
   if (a.B == 0 || a.L == 0) return kOk;
-  TESM_REQUIRE(a.q && a.k && a.rope && a.table && a.S && a.e_tanh && a.c_out && a.tern && a.count, kErrInvalidArg,
+  TESM_REQUIRE(a.q && a.k && a.rope && a.table && a.S && a.tern && a.count, kErrInvalidArg,
                "global ent: null pointer");
   TESM_REQUIRE(!a.mimo || a.coef, kErrInvalidArg, "global ent: MIMO needs the merge factors");
   TESM_REQUIRE(!a.mimo || !a.q_add, kErrInvalidArg, "global ent: MIMO has no cross-layer query");
   const bool bf16_states = a.dt == kBF16 && !a.mimo;  // SISO states are in the layer dtype, MIMO's float32
   TESM_REQUIRE(!bf16_states || a.states_t, kErrInvalidArg, "global ent: null transposed-states workspace");
+  const int64_t nqb = (a.L + kGB - 1) / kGB, nqm = (a.L + kMQ - 1) / kMQ, ncb = (a.H * a.D + kMC - 1) / kMC;
+  TESM_REQUIRE(nqb * (nqb + 1) / 2 <= 0x7fffffff && a.B <= 65535 && nqm * ncb * a.B <= 0x7fffffff, kErrUnsupported,
+               "global ent: too large");
+  TESM_REQUIRE(2 * a.L < (int64_t(1) << 24), kErrUnsupported, "global ent: sequence too long for the bias table");
+  TESM_REQUIRE(a.qr && a.kr, kErrInvalidArg, "global ent: null RoPE workspace");
+  return kOk;
+}
+
+int launch_global_ent(const GlobalArgs& a, hipStream_t st) {
+  const int rc = check_global(a);
+  if (rc || a.B == 0 || a.L == 0) return rc;
+  TESM_REQUIRE(a.e_tanh && a.c_out, kErrInvalidArg, "global ent: null outputs");
   const int64_t C = a.H * a.D;
   const int64_t ldt = global_tern_pitch(a.L);
   const int64_t nqb = (a.L + kGB - 1) / kGB;
   const int64_t ntiles = nqb * (nqb + 1) / 2;
   const int64_t nqm = (a.L + kMQ - 1) / kMQ, ncb = (C + kMC - 1) / kMC;
-  TESM_REQUIRE(ntiles <= 0x7fffffff && a.B <= 65535 && nqm * ncb * a.B <= 0x7fffffff, kErrUnsupported,
-               "global ent: too large");
-  TESM_REQUIRE(2 * a.L < (int64_t(1) << 24), kErrUnsupported, "global ent: sequence too long for the bias table");
-  TESM_REQUIRE(a.qr && a.kr, kErrInvalidArg, "global ent: null RoPE workspace");
   const int64_t nrope = std::max(a.B * a.L * a.H * (a.R / 2), a.B * a.L);
   const unsigned nbr = static_cast<unsigned>((nrope + 255) / 256);
   const dim3 gs(static_cast<unsigned>(ntiles), 1, static_cast<unsigned>(a.B));
