@@ -515,15 +515,21 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 
 // Tile sizes by grid.  Times in us on one box, bf16 outputs unless noted; "before" is the two-stage, one-group form.
 //   * 128x256 tiles (8 waves of 64x64, two workgroups per CU) when they give every CU one: 2048 x 4096 x 4096 36.2
-//     (64x256 tiles 40), 4095 x 3744 x 1024 21.2 (64x128: 26.3).  Grids past two rounds walk 8 M tiles per group.
+//     (64x256 tiles 40), 4095 x 3744 x 1024 21.2 (64x128: 26.3); past short K already when they give three CUs in four
+//     one: 1500 x 4096 x 11008 72.4 (64x128: 79.2), 520 x 11008 x 4096 30.5 (35.2), and 400 x 11008 x 4096, below
+//     that, 26.9 against 26.0.  Grids past two rounds walk 8 M tiles per group, past short K those past one (3000 x 4096 x
+//     4096 54.5, by fours 59.2), and at K above 4096 all (1500 x 4096 x 11008 f32 77.0, by fours 85.9).
 //   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
 //     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
-//   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU: 8192 x 768 x 768 10.6 (128x256: 10.9),
-//     4095 x 1024 x 2816 15.4 (before 21.5), 1000 x 4096 x 4096 21.2 (before 28.3).  A K loop of at most
+//   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU, past short K one: 8192 x 768 x 768 10.6
+//     (128x256: 10.9), 4095 x 1024 x 2816 15.4 (before 21.5), 1000 x 4096 x 4096 21.2 (before 28.3), 666 x 4096 x 11008
+//     41.0 (two K groups on 32x64: 50.6), 200 x 11008 x 4096 16.7 (20.7).  A K loop of at most
 //     three tiles stays on this shape too: such calls are launch-bound (16384 x 256 x 256 5.9, best 5.7; 512 x 96 x
 //     384 5.4, best 4.2), and it keeps short products to one instantiation.
 //   * 32x128 tiles when those do, at short K: 512 x 2944 x 768 4.9 (64x128: 5.8), 666 x 2944 x 768 f32 6.1 (7.1).
-//   * else K groups on 32x64 tiles: two (512 x 768 x 768 4.2, before 5.3; 32 x 34816 x 4096 12.3, before 14.0), or
+//   * else K groups: two on 32x128 tiles past short K when those give three workgroups per two CUs (400 x 4096 x 11008
+//     30.1, on 32x64 tiles 35.4; 300 rows 28.8 against 25.0), or on 32x64 tiles two (512 x 768 x 768 4.2, before 5.3;
+//     32 x 34816 x 4096 12.3, before 14.0), or
 //     four when K is long and two would leave CUs idle (512 x 768 x 3072 5.7, before 11.8; 200 x 4096 x 11008 18.2,
 //     two groups 21.1).
 template <int EPI>
@@ -544,11 +550,14 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
     }
   }
   if (a.Kp > 3 * kKTile) {
-    if (big >= 2 * cus) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
-    if (big >= cus) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
-    if (tiles(64, 128) < 2 * cus) {
-      if (a.Kp <= 1024 && tiles(32, 128) >= cus) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
+    const bool wide = big >= cus || (4 * big >= 3 * cus && a.Kp > 1024 && a.M > 64);
+    if (big >= 2 * cus || (wide && (a.Kp > 4096 || (big > cus && a.Kp > 1024)))) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
+    if (wide) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
+    const int64_t mid = tiles(64, 128);
+    if (mid < 2 * cus && a.Kp <= 1024 && tiles(32, 128) >= cus) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
+    if (mid < cus || a.M <= 32) {
       if (a.Kp >= 2048 && tiles(32, 64) < 2 * cus) return run_mfma32k<1, 2, 1, 1, 4, 3, EPI>(a, st);
+      if (a.Kp > 1024 && 2 * tiles(32, 128) >= 3 * cus) return run_mfma32k<1, 4, 1, 1, 2, 3, EPI>(a, st);
       return run_mfma32k<1, 2, 1, 1, 2, 3, EPI>(a, st);
     }
   }

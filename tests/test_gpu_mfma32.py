@@ -33,6 +33,9 @@ STORE = [(33, 65, 128, "mfma32_kernel<1,4,2,1,"), (129, 96, 384, "mfma32_kernel<
          (97, 70, 640, "mfma32k_kernel<1,2,1,1,2,3,"), (40, 300, 513, "mfma32k_kernel<1,2,1,1,2,3,"),
          (17, 16385, 500, "mfma32k_kernel<1,2,1,1,2,3,"), (17, 40001, 500, "mfma32_kernel<1,4,1,1,"), (513, 2944, 768, "mfma32_kernel<1,4,1,1,"),
          (2049, 2500, 700, "mfma32_kernel<1,4,2,1,"), (1025, 8200, 513, "mfma32_kernel<2,4,2,2,"),
+         (1500, 4090, 1100, "mfma32_kernel<2,4,2,2,"), (520, 4090, 1100, "mfma32_kernel<1,4,2,1,"),
+         (410, 4090, 1100, "mfma32k_kernel<1,4,1,1,2,3,"), (300, 4090, 1100, "mfma32k_kernel<1,2,1,1,2,3,"),
+         (32, 40001, 1100, "mfma32k_kernel<1,2,1,1,2,3,"),
          (2100, 8200, 1100, "mfma32_kernel<2,4,2,2,"), (8190, 2401, 520, "mfma32_split_kernel<")]
 
 
