@@ -1091,10 +1091,10 @@ __global__ __launch_bounds__(512) void ent_fused2_kernel(EntArgs a, int64_t weff
 // ---------------------------------------------------------------------------
 // Fused SISO kernel, third form: the window mix in registers, for the shapes whose state halo does not
 // fit ent_fused2_kernel's LDS (D 384-512 with window 32; D 384 with rank 96).  A workgroup owns (batch
-// row b, 2 TS positions) and all D channels (D % 64 == 0, D <= 512); thread (s, ch) owns channel ch of
-// the TS positions of half s.  A position's window mix reads its own channel's states only, so the thread
-// loads the W - 1 + 16 states of its channel it needs (as raw bits, all in flight at once, straight
-// from the state tensor) and forms its 16 window sums from registers, the window weights being the
+// row b, HV halves of TS positions) and all D channels (D % 64 == 0, D <= 512); thread (s, ch) owns channel ch
+// of the TS positions of half s.  A position's window mix reads its own channel's states only, so the thread
+// loads the W - 1 + TS states of its channel it needs (as raw bits, all in flight at once, straight
+// from the state tensor) and forms its TS window sums from registers, the window weights being the
 // same for all 64 lanes of a wave (broadcast LDS reads).  The weights come from one (position, window
 // slot) pair per thread over RoPE'd q / k rows staged in LDS; tanh(E) and C are staged in LDS and
 // quantized with one 16-channel group per thread.  Every value is the same sequence of float
@@ -1126,11 +1126,12 @@ __host__ __device__ inline RegLds reg_lds(int64_t D, int64_t R, int64_t W, int w
 }
 
 // WM: window slots of the mix (16 or 32; a window W < WM is right-aligned, the first WM - W slots
-// weigh zero).  KI: key staging items per thread in the first round (queries: 2).
-template <int DT, int WM, int KI, int NTM, int TS>
-__global__ __launch_bounds__(NTM, 1) void ent_reg_kernel(EntArgs e, int64_t weff, RegLds f) {
+// weigh zero).  KI: key staging items per thread in the first round (queries: 2).  HV: halves per workgroup.  MW: waves
+// per SIMD that the registers must leave room for.
+template <int DT, int WM, int KI, int NTM, int TS, int HV, int MW>
+__global__ __launch_bounds__(NTM, MW) void ent_reg_kernel(EntArgs e, int64_t weff, RegLds f) {
   using T = typename Elem<DT>::T;
-  constexpr int TP = 2 * TS, NX = WM - 1 + TS;
+  constexpr int TP = HV * TS, NX = WM - 1 + TS;
   extern __shared__ __attribute__((aligned(16))) char lds_rg[];
   float* kr = reinterpret_cast<float*>(lds_rg + f.kr);
   float* qr = reinterpret_cast<float*>(lds_rg + f.qr);
@@ -1138,8 +1139,8 @@ __global__ __launch_bounds__(NTM, 1) void ent_reg_kernel(EntArgs e, int64_t weff
   T* stg = reinterpret_cast<T*>(lds_rg + f.stg);
   const int tid = threadIdx.x;
   const int D = static_cast<int>(e.D), W = static_cast<int>(weff), half = static_cast<int>(e.R / 2);
-  const int krs = static_cast<int>(f.krs), NT = 2 * D;
-  const int s = __builtin_amdgcn_readfirstlane(tid / D);  // D % 64 == 0: uniform per wave
+  const int krs = static_cast<int>(f.krs), NT = HV * D;
+  const int s = HV == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / D);  // D % 64 == 0: uniform per wave
   const int ch = tid - s * D;
   const int64_t L = e.L, b = blockIdx.y;
   const int64_t t0 = static_cast<int64_t>(blockIdx.x) * TP, ts = t0 + s * TS;
@@ -1466,35 +1467,46 @@ int launch_rope_table(float2* tab, int64_t L, int64_t R, int64_t pos_offset, dou
 
 static int64_t eff_window(const EntArgs& a) { return a.mimo ? a.W : std::min(a.W, a.L); }
 
-constexpr int kRegTS = 8;  // positions per thread of the register-mix kernel (16 per workgroup)
+constexpr int kRegTS = 8;  // positions per thread of the register-mix kernel
 
-template <int DT, int WM, int KI>
+template <int DT, int WM, int KI, int HV>
 static void launch_reg_k(const EntArgs& a, int64_t weff, const RegLds& f, hipStream_t st) {
   constexpr int TS = kRegTS;
-  dim3 grid(static_cast<unsigned>((a.L + 2 * TS - 1) / (2 * TS)), static_cast<unsigned>(a.B));
-  const unsigned nt = static_cast<unsigned>(2 * a.D);  // the register cap follows nt
-  if (nt > 768)
-    ent_reg_kernel<DT, WM, KI, 1024, TS><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 1024, TS>)>>>(a, weff, f);
-  else if (nt > 512)
-    ent_reg_kernel<DT, WM, KI, 768, TS><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 768, TS>)>>>(a, weff, f);
+  dim3 grid(static_cast<unsigned>((a.L + HV * TS - 1) / (HV * TS)), static_cast<unsigned>(a.B));
+  const unsigned nt = static_cast<unsigned>(HV * a.D);  // (D > 256: one half of at most 512 threads, two per CU)
+  if constexpr (HV == 1)
+    ent_reg_kernel<DT, WM, KI, 512, TS, 1, 4><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 512, TS, 1, 4>)>>>(a, weff, f);
   else
-    ent_reg_kernel<DT, WM, KI, 512, TS><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 512, TS>)>>>(a, weff, f);
+    ent_reg_kernel<DT, WM, KI, 512, TS, 2, 1><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 512, TS, 2, 1>)>>>(a, weff, f);
 }
 
+template <int DT, int HV>
+static void run_reg_hv(const EntArgs& a, int64_t weff, hipStream_t st) {
+  const int wm = weff <= 16 ? 16 : 32;
+  const RegLds f = reg_lds(a.D, a.R, weff, wm, DT == kBF16 ? 2 : 4, HV * kRegTS);
+  const int64_t ki = ((HV * kRegTS + weff - 1) * (a.R / 2) + HV * a.D - 1) / (HV * a.D);  // first-round key items
+  if (wm == 16) {
+    if (ki <= 2) launch_reg_k<DT, 16, 2, HV>(a, weff, f, st);
+    else if (ki == 3) launch_reg_k<DT, 16, 3, HV>(a, weff, f, st);
+    else launch_reg_k<DT, 16, 4, HV>(a, weff, f, st);
+  } else {
+    if (ki <= 2) launch_reg_k<DT, 32, 2, HV>(a, weff, f, st);
+    else if (ki == 3) launch_reg_k<DT, 32, 3, HV>(a, weff, f, st);
+    else launch_reg_k<DT, 32, 4, HV>(a, weff, f, st);
+  }
+}
+
+// Rows of more than 256 channels take one half per workgroup: 8 positions, at most 512 threads, two workgroups per CU
+// (with both halves 1024 threads take a CU, so a grid just past the CUs runs two full rounds, and nothing overlaps the
+// loads).  3 x 1365 tokens, D 512, rank 80, bf16 25.4 us against 32.7; 4 x 8192 115 against 127, 1 x 200 15.1 against
+// 19.6, 3 x 1365 f32 27.0 against 33.6; only a grid of exactly one round of both halves is no faster (1 x 4096 22.9
+// against 21.8).  Narrower rows keep both (1 x 4096, D 256, rank 64, f32 14.0; one half 15.0).
 template <int DT>
 static int run_reg(const EntArgs& a, int64_t weff, hipStream_t st) {
-  const int wm = weff <= 16 ? 16 : 32;
-  const RegLds f = reg_lds(a.D, a.R, weff, wm, DT == kBF16 ? 2 : 4, 2 * kRegTS);
-  const int64_t ki = ((2 * kRegTS + weff - 1) * (a.R / 2) + 2 * a.D - 1) / (2 * a.D);  // first-round key items
-  if (wm == 16) {
-    if (ki <= 2) launch_reg_k<DT, 16, 2>(a, weff, f, st);
-    else if (ki == 3) launch_reg_k<DT, 16, 3>(a, weff, f, st);
-    else launch_reg_k<DT, 16, 4>(a, weff, f, st);
-  } else {
-    if (ki <= 2) launch_reg_k<DT, 32, 2>(a, weff, f, st);
-    else if (ki == 3) launch_reg_k<DT, 32, 3>(a, weff, f, st);
-    else launch_reg_k<DT, 32, 4>(a, weff, f, st);
-  }
+  if (a.D > 256)
+    run_reg_hv<DT, 1>(a, weff, st);
+  else
+    run_reg_hv<DT, 2>(a, weff, st);
   return check_launch("entanglement fused (window mix in registers)");
 }
 
