@@ -42,12 +42,124 @@ constexpr int kMixLD = 4;            // float4 state loads per thread per block:
 // channel block plus its W - 1 row halo are staged per block, and the next block's states are loaded
 // into registers while the current one is mixed and stored.  Each thread owns 2 positions x 4 channels
 // and walks the window keeping the 2 state rows it needs in registers, so every 8 multiply-adds cost
-// one state and one weight read.  Sums run over w in increasing order.  WT is W when it is a
-// compile-time case (index math by shifts), else 0.
+// one state and one weight read.  Sums run over w in increasing order.  WT: 64 for mix64, else 0.
+//
+// W = 64 with whole 16-byte rows (the largest window, and the large preset's) takes mix64 below: here a thread reads 24
+// bytes of LDS per 8 multiply-adds, three bytes each where two keep up with the vector units.
+constexpr int kM64C = 128;                           // channels per block
+constexpr int kM64Rows = kMixTP + 64;                // state rows per block (the last one is not used)
+constexpr int kM64CB = 4;                            // channel blocks per workgroup
+constexpr size_t kM64Lds = (kM64Rows * kM64C + 64 * kMixTP) * sizeof(float);
+static_assert(2 * kM64Lds <= 160 * 1024, "two workgroups per CU");
+
+// The general form's plan at W = 64 with 8 positions x 4 channels per thread: the 8 state rows a slot needs stay in
+// registers and move up by one, so a slot's 32 multiply-adds cost one state and two weight reads of 16 bytes (half the
+// general form's LDS traffic), and the last slot's rows are the positions' own states.  States go straight to LDS; two
+// workgroups per CU overlap one's loads with the other's sums.  Each sum runs over the window in increasing order, as
+// in the general form (same bits).  32768 positions x 8192 channels: 886 us, before 1017, with the next block's states
+// held in registers instead 951; the vector units alone need 440 us for these 17 G multiply-adds, and weights as scalar
+// operands (16 positions x 1 channel per lane) took 1560, the scalar cache being too small for 20 waves' weights.
+template <int DT>
+__device__ __forceinline__ void mix64(const MimoMixArgs& a, float* lds) {
+  float* srow = lds;                         // [kM64Rows][kM64C]
+  float* wtT = lds + kM64Rows * kM64C;       // [64][kMixTP]
+  const int64_t b = blockIdx.z / a.H, h = blockIdx.z - b * a.H;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.y) * kMixTP;
+  const int D = static_cast<int>(a.D), nblk = (D + kM64C - 1) / kM64C;
+  const int cb0 = static_cast<int>(blockIdx.x) * kM64CB, cb1 = cb0 + kM64CB < nblk ? cb0 + kM64CB : nblk;
+  const int tid = threadIdx.x;
+  const int64_t C = a.H * a.D, tlo = t0 - 63;
+  const int nvalid = static_cast<int>(a.L - t0 < kMixTP ? a.L - t0 : kMixTP);
+  const float* Sh = a.S + b * a.L * C + h * a.D;
+  // Straight to LDS, two rows per instruction.  Rows before the sequence re-read row 0 (their weights are 0, and row 0
+  // is in those positions' windows), rows past it and channels past D feed only outputs that are dropped.
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  auto stage = [&](int cb) {
+    const int dc = cb * kM64C + 4 * (lane & 31);
+    const float* src = Sh + (dc < D ? dc : 0);
+#pragma unroll
+    for (int k = 0; k < kM64Rows / 8; ++k) {
+      const int r = 2 * (wv + 4 * k);
+      const int64_t t = tlo + r + (lane >> 5), tc = t < 0 ? 0 : (t < a.L ? t : a.L - 1);
+      __builtin_amdgcn_global_load_lds(src + tc * C, (__attribute__((address_space(3))) void*)(srow + r * kM64C), 16, 0, 0);
+    }
+  };
+  stage(cb0);
+  const float* wb = a.wts + ((b * a.L + t0) * a.H + h) * 64;
+  const int64_t wrow = a.H * 64;
+  for (int i = tid; i < kMixTP * 64; i += 256) {
+    const int p = i & (kMixTP - 1), w = i / kMixTP;  // (reads by position: the stores go to consecutive words)
+    wtT[w * kMixTP + p] = p < nvalid ? wb[p * wrow + w] : 0.0f;
+  }
+  __syncthreads();
+  const int p0 = 8 * (tid >> 5), c0 = 4 * (tid & 31);
+  const float* sp = srow + p0 * kM64C + c0;
+  for (int cb = cb0; cb < cb1; ++cb) {
+    float acc[8][4];
+    float4 s[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+      s[i] = *reinterpret_cast<const float4*>(sp + i * kM64C);
+    }
+#pragma unroll 1
+    for (int w0 = 0; w0 < 64; w0 += 8) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {  // slot w0 + u: position i's row is s[(i + u) % 8]
+        const float4 wa = *reinterpret_cast<const float4*>(wtT + (w0 + u) * kMixTP + p0);
+        const float4 wc = *reinterpret_cast<const float4*>(wtT + (w0 + u) * kMixTP + p0 + 4);
+        const float wv[8] = {wa.x, wa.y, wa.z, wa.w, wc.x, wc.y, wc.z, wc.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float4 x = s[(i + u) & 7];
+          acc[i][0] = __builtin_fmaf(wv[i], x.x, acc[i][0]);
+          acc[i][1] = __builtin_fmaf(wv[i], x.y, acc[i][1]);
+          acc[i][2] = __builtin_fmaf(wv[i], x.z, acc[i][2]);
+          acc[i][3] = __builtin_fmaf(wv[i], x.w, acc[i][3]);
+        }
+        // the row the window's move brings in; after the last slot position 0's own row stays in s[7]
+        if (u < 7 || w0 < 56) s[u] = *reinterpret_cast<const float4*>(sp + (w0 + u + 8) * kM64C);
+      }
+    }
+    const int d = cb * kM64C + c0;
+    if (d < D) {
+      float cf[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cf[j] = a.coef[h * a.D + d + j];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (p0 + i >= nvalid) break;
+        const float4 own = s[(i + 7) & 7];  // slot 63
+        const float sv[4] = {own.x, own.y, own.z, own.w};
+        float te[4], cc[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float e = sv[j] + a.ent_scale * (acc[i][j] - sv[j]);
+          te[j] = tanhf_(e * cf[j]);
+          cc[j] = (e - sv[j]) * cf[j];
+        }
+        const int64_t o = (b * a.L + t0 + p0 + i) * C + h * a.D + d;
+        st4<DT>(a.te, o, te);
+        st4<DT>(a.cc, o, cc);
+      }
+    }
+    __syncthreads();  // every thread is done with this block's states
+    if (cb + 1 < cb1) {
+      stage(cb + 1);
+      __syncthreads();
+    }
+  }
+}
+
 template <int DT, bool VEC, int WT>
-__global__ __launch_bounds__(256) void mimo_mix_kernel(MimoMixArgs a) {
+__global__ __launch_bounds__(256, WT == 64 ? 2 : 1) void mimo_mix_kernel(MimoMixArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds_mimo[];
-  const int W = WT > 0 ? WT : static_cast<int>(a.W);
+  if constexpr (WT == 64) {
+    mix64<DT>(a, lds_mimo);
+    return;
+  }
+  const int W = static_cast<int>(a.W);
   const int rows = kMixTP + W - 1;
   float* srow = lds_mimo;                  // [rows][kMixSP]
   float* wtT = lds_mimo + rows * kMixSP;   // [W][kMixWP]
@@ -317,12 +429,15 @@ int launch_mimo_mix(const MimoMixArgs& a, hipStream_t st) {
   const bool vec = a.D % 4 == 0 && (a.H * a.D) % 4 == 0 && reinterpret_cast<uintptr_t>(a.S) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(a.te) % (a.dt == kBF16 ? 8 : 16) == 0 &&
                    reinterpret_cast<uintptr_t>(a.cc) % (a.dt == kBF16 ? 8 : 16) == 0;
+  const bool m64 = vec && a.W == 64 && a.D < (int64_t(1) << 30);
+  const int64_t nb64 = (a.D + kM64C - 1) / kM64C;
+  const dim3 g64(static_cast<unsigned>((nb64 + kM64CB - 1) / kM64CB), grid.y, grid.z);
   if (a.dt == kBF16) {
-    if (vec && a.W == 64) mimo_mix_kernel<kBF16, true, 64><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kBF16, true, 64>)>>>(a);
+    if (m64) mimo_mix_kernel<kBF16, true, 64><<<g64, 256, kM64Lds, TESM_LOGGED(st, mimo_mix_kernel<kBF16, true, 64>)>>>(a);
     else if (vec) mimo_mix_kernel<kBF16, true, 0><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kBF16, true, 0>)>>>(a);
     else mimo_mix_kernel<kBF16, false, 0><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kBF16, false, 0>)>>>(a);
   } else {
-    if (vec && a.W == 64) mimo_mix_kernel<kF32, true, 64><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kF32, true, 64>)>>>(a);
+    if (m64) mimo_mix_kernel<kF32, true, 64><<<g64, 256, kM64Lds, TESM_LOGGED(st, mimo_mix_kernel<kF32, true, 64>)>>>(a);
     else if (vec) mimo_mix_kernel<kF32, true, 0><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kF32, true, 0>)>>>(a);
     else mimo_mix_kernel<kF32, false, 0><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kF32, false, 0>)>>>(a);
   }
