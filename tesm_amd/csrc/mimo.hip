@@ -81,7 +81,8 @@ __device__ __forceinline__ void mix64(const MimoMixArgs& a, float* lds) {
     for (int k = 0; k < kM64Rows / 8; ++k) {
       const int r = 2 * (wv + 4 * k);
       const int64_t t = tlo + r + (lane >> 5), tc = t < 0 ? 0 : (t < a.L ? t : a.L - 1);
-      __builtin_amdgcn_global_load_lds(src + tc * C, (__attribute__((address_space(3))) void*)(srow + r * kM64C), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(src + tc * C, (__attribute__((address_space(3))) void*)(srow + r * kM64C), 16, 0,
+                                       0);
     }
   };
   stage(cb0);
@@ -287,10 +288,10 @@ __global__ __launch_bounds__(256) void mimo_final_kernel(const float* S, const f
 }
 
 // One workgroup of 16 waves per batch row.  A wave takes up to 64 scores at a time: its lanes form their products side
-// by side (rows of q and k read contiguously) into the wave's slab of LDS, a slice of at most kStSL of a score's products
-// at once, then one lane per score adds its slice in natural order.  Bound by the latency of those two phases.  With one
-// thread per score (256 threads, each walking its own rows of q and k) 1 x 256 scores of 256 products took 101 us, now
-// 58.
+// by side (rows of q and k read contiguously) into the wave's slab of LDS, a slice of at most kStSL of a score's
+// products at once, then one lane per score adds its slice in natural order.  Bound by the latency of those two phases.
+// With one thread per score (256 threads, each walking its own rows of q and k) 1 x 256 scores of 256 products took
+// 101 us, now 58.
 constexpr int kStNW = 16;               // waves
 constexpr int kStSL = 256;              // products of a score per slice
 constexpr int kStSlab = 2048;           // products per wave and slice
@@ -392,7 +393,8 @@ int launch_mimo_stats(const MimoStatsArgs& a, hipStream_t st) {
                "mimo stats: need 1 <= W <= S <= L");
   TESM_REQUIRE(a.R >= 2 && a.R % 2 == 0 && a.H >= 1, kErrInvalidArg, "mimo stats: need an even R");
   TESM_REQUIRE((a.S - a.W + 1) * a.H * a.W <= 0x7fffffff, kErrUnsupported, "mimo stats: too many scores");
-  TESM_REQUIRE(a.H * a.R <= 0x7fffffff && (!a.global || a.S <= 0x7fff), kErrUnsupported, "mimo stats: too many products");
+  TESM_REQUIRE(a.H * a.R <= 0x7fffffff && (!a.global || a.S <= 0x7fff), kErrUnsupported,
+               "mimo stats: too many products");
   constexpr size_t lds = kStNW * kStPitch * sizeof(float);
   if (a.dt == kBF16)
     mimo_stats_kernel<kBF16><<<static_cast<unsigned>(a.B), 64 * kStNW, lds, TESM_LOGGED(st, mimo_stats_kernel<kBF16>)>>>(a);
