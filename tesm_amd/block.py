@@ -16,7 +16,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import backend_error
+from .bitlinear import backend_error, param
 
 
 def _check(t: torch.Tensor, what: str) -> None:
@@ -40,7 +40,7 @@ class RMSNorm(nn.Module):
         ``(y or None, s in residual_dtype or None, codes or None)`` where ``codes = (q, s_x, rowsum)``
         are y's per-token int8 codes in the product layout (computed when ``codes_eps`` is given)."""
         _check(x, "RMSNorm")
-        w = self._parameters["weight"]
+        w = param(self, "weight")
         dt = w.dtype
         if x.dtype != dt:
             raise RuntimeError(f"RMSNorm: input is {x.dtype} but the weight is {dt}")

@@ -20,7 +20,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, backend_error, check_hip_call, packed_weights, same_packs
+from .bitlinear import BitLinear, backend_error, check_hip_call, packed_weights, param, same_packs
 from .hip_ops import on_device, raw_stream
 
 _WORKSPACES = {}
@@ -185,12 +185,11 @@ class TESM_SISO(nn.Module):
         """The prefill descriptor's fields that depend on the module alone: sizes, thresholds, packed weights and
         biases.  Rebuilt when a weight, a bias or an option changes (the packed weights' own rule,
         tesm.py:226-236); a call copies it and fills in its lengths, tensors and outputs."""
-        mods, params = self._modules, self._parameters
+        mods = self._modules
         lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"], mods["cross_layer_q_proj"])
         glob = self.entanglement_window <= 0
-        biases = (params["decay_bias"],) + ((params["global_rel_pos_embed"], params["global_rel_pos_scale"],
-                                            params["global_rel_pos_bias"]) if glob else
-                                           (params["local_entanglement_bias"],))
+        names = ("global_rel_pos_embed", "global_rel_pos_scale", "global_rel_pos_bias") if glob else ("local_entanglement_bias",)
+        biases = [param(self, n) for n in ("decay_bias",) + names]
         packs = packed_weights(lins, dt, 4 + int(cross))
         key = (dt, dev, cross, self.entanglement_window, self.state_scan_chunk_size, self.entanglement_threshold,
                float(self.entanglement_scale), lins[0].bit_eps, self.d_model, self.d_state, self.ent_rank,
@@ -224,7 +223,7 @@ class TESM_SISO(nn.Module):
             desc.global_scale, desc.global_bias = scale.data_ptr(), bias.data_ptr()
         else:
             desc.local_bias = local_bias.data_ptr()
-        keep = packs + [decay_bias, local_bias, gparams]
+        keep = packs + [decay_bias, local_bias, gparams, biases]  # (biases: none of the key's addresses is reused)
         self.__dict__["_prefill_plan"] = (key, (desc, keep))
         return desc, keep
 

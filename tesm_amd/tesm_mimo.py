@@ -22,7 +22,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, check_hip_call, packed_weights, same_packs
+from .bitlinear import BitLinear, check_hip_call, packed_weights, param, same_packs
 from .hip_ops import on_device, raw_stream
 from .tesm import TESM_SISO, workspace
 
@@ -123,12 +123,11 @@ class TESMMIMO_Optimized(TESM_SISO):
 
     def _mimo_layer_plan(self, dt, dev):
         """The prefill descriptor's fields that depend on the module alone (see TESM_SISO._layer_plan)."""
-        mods, params = self._modules, self._parameters
+        mods = self._modules
         lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"])
         glob = self.entanglement_window <= 0
-        biases = (params["decay_bias"], params["mimo_x"], params["mimo_o"]) + (
-            (params["global_rel_pos_embed"], params["global_rel_pos_scale"], params["global_rel_pos_bias"]) if glob else
-            (params["local_entanglement_bias"],))
+        names = ("global_rel_pos_embed", "global_rel_pos_scale", "global_rel_pos_bias") if glob else ("local_entanglement_bias",)
+        biases = [param(self, n) for n in ("decay_bias", "mimo_x", "mimo_o") + names]
         packs = packed_weights(lins, dt, 4)
         key = (dt, dev, self.entanglement_window, self.entanglement_threshold, float(self.entanglement_scale),
                lins[0].bit_eps, self.d_model, self.d_state, self.n_heads, self.ent_rank,
@@ -162,7 +161,7 @@ class TESMMIMO_Optimized(TESM_SISO):
         else:
             desc.local_bias = local_bias.data_ptr()
         desc.mimo_coef, desc.mimo_x0sq = coef.data_ptr(), x0sq.data_ptr()
-        keep = packs + [decay_bias, local_bias, gparams, coef, x0sq]
+        keep = packs + [decay_bias, local_bias, gparams, coef, x0sq, biases]
         self.__dict__["_mimo_plan"] = (key, (desc, keep))
         return desc, keep
 

@@ -7,9 +7,10 @@ import threading
 
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 from hip_helpers import DEV, need_gpu
-from tesm_amd import FeedForward, TESM_SISO, TESMConfig, TESMMIMO_Optimized
+from tesm_amd import FeedForward, RMSNorm, TESM_SISO, TESMConfig, TESMMIMO_Optimized
 
 pytestmark = pytest.mark.gpu
 
@@ -93,6 +94,34 @@ def test_dtype_mismatch_still_refused(kind):
     _out(m, _u())
     with pytest.raises(RuntimeError, match="same dtype"):
         _out(m, _u(torch.bfloat16))
+
+
+class _Scale(torch.nn.Module):
+    factor = 2.0
+
+    def forward(self, x):
+        return x * self.factor
+
+
+@pytest.mark.parametrize("kind", ["siso", "global", "mimo"])
+def test_parametrized_decay_bias(kind):
+    """A parameter that a parametrization computes anew for every access, and its later changes, reach the call."""
+    m, plain, u = _make(kind), _make(kind), _u()
+    rule = _Scale()
+    torch.nn.utils.parametrize.register_parametrization(m, "decay_bias", rule)
+    for factor in (2.0, -1.0, 0.5):
+        rule.factor = factor
+        with torch.no_grad():
+            plain.decay_bias.copy_(m.parametrizations.decay_bias.original * factor)
+        assert torch.equal(_out(m, u), _out(plain, u)), factor
+
+
+def test_parametrized_norm_weight():
+    m, plain, u = RMSNorm(64).to(DEV).eval(), RMSNorm(64).to(DEV).eval(), _u()
+    torch.nn.utils.parametrize.register_parametrization(m, "weight", _Scale())
+    with torch.no_grad():
+        plain.weight.mul_(2.0)
+    assert torch.equal(_out(m, u), _out(plain, u))
 
 
 def test_threads_on_their_own_streams():
