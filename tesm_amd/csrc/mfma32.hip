@@ -517,8 +517,11 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //   * 128x256 tiles (8 waves of 64x64, two workgroups per CU) when they give every CU one: 2048 x 4096 x 4096 36.2
 //     (64x256 tiles 40), 4095 x 3744 x 1024 21.2 (64x128: 26.3); past short K already when they give three CUs in four
 //     one: 1500 x 4096 x 11008 72.4 (64x128: 79.2), 520 x 11008 x 4096 30.5 (35.2), and 400 x 11008 x 4096, below
-//     that, 26.9 against 26.0.  Grids past two rounds walk 8 M tiles per group, past short K those past one (3000 x 4096 x
-//     4096 54.5, by fours 59.2), and at K above 4096 all (1500 x 4096 x 11008 f32 77.0, by fours 85.9).
+//     that, 26.9 against 26.0; above K 4096 from five CUs in eight (with the quantization: 1400 x 4096 x 11008 78.2,
+//     64x128 84.3; 1200 77.5, 78.6; 1100 no difference).  Grids past two rounds walk 8 M tiles per group, past short K
+//     those past one (3000 x 4096 x 4096 54.5, by fours 59.2), at K above 4096 all (1500 x 4096 x 11008 f32 77.0, by
+//     fours 85.9), and with five M tiles (513 x 11008 x 4096 with the quantization 36.0, by fours 36.6; seven or
+//     eight M tiles of 8192 columns 37.0-40.0, by fours 36.6-39.3).
 //   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
 //     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
 //   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU, past short K one: 8192 x 768 x 768 10.6
@@ -526,7 +529,10 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //     41.0 (two K groups on 32x64: 50.6), 200 x 11008 x 4096 16.7 (20.7).  A K loop of at most
 //     three tiles stays on this shape too: such calls are launch-bound (16384 x 256 x 256 5.9, best 5.7; 512 x 96 x
 //     384 5.4, best 4.2), and it keeps short products to one instantiation.
-//   * 32x128 tiles when those do, at short K: 512 x 2944 x 768 4.9 (64x128: 5.8), 666 x 2944 x 768 f32 6.1 (7.1).
+//   * 32x128 tiles when those do, at short K and up to three 64x128 tiles per two CUs (two per CU where those would be
+//     half empty): 512 x 2944 x 768 4.9 (64x128: 5.8), 666 x 2944 x 768 f32 6.1 (7.1); with the quantization
+//     1300 x 2432 x 768 f32 12.4 (11.8), 1600 13.2 (12.8), 4095 x 768 x 768 12.1 (11.6).  Around the line it also
+//     depends on the remainders: 3500 x 1000 x 768 16.5 (17.0), 1100 x 2816 x 1024 11.7 (12.1).
 //   * else K groups: two on 32x128 tiles past short K when those give three workgroups per two CUs (400 x 4096 x 11008
 //     30.1, on 32x64 tiles 35.4; 300 rows 28.8 against 25.0), or on 32x64 tiles two (512 x 768 x 768 4.2, before 5.3;
 //     32 x 34816 x 4096 12.3, before 14.0), or
@@ -550,11 +556,13 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
     }
   }
   if (a.Kp > 3 * kKTile) {
-    const bool wide = big >= cus || (4 * big >= 3 * cus && a.Kp > 1024 && a.M > 64);
-    if (big >= 2 * cus || (wide && (a.Kp > 4096 || (big > cus && a.Kp > 1024)))) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
+    const bool most = a.Kp > 4096 ? 8 * big >= 5 * cus : 4 * big >= 3 * cus;
+    const bool wide = big >= cus || (most && a.Kp > 1024 && a.M > 64);
+    const bool five = a.M > 512 && a.M <= 640;  // M tiles: groups of four would leave one by itself
+    if (big >= 2 * cus || (wide && (a.Kp > 4096 || ((big > cus || five) && a.Kp > 1024)))) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
     if (wide) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
     const int64_t mid = tiles(64, 128);
-    if (mid < 2 * cus && a.Kp <= 1024 && tiles(32, 128) >= cus) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
+    if (2 * mid < (a.M <= 32 ? 4 : 3) * cus && a.Kp <= 1024 && tiles(32, 128) >= cus) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
     if (mid < cus || a.M <= 32) {
       if (a.Kp >= 2048 && tiles(32, 64) < 2 * cus) return run_mfma32k<1, 2, 1, 1, 4, 3, EPI>(a, st);
       if (a.Kp > 1024 && 2 * tiles(32, 128) >= 3 * cus) return run_mfma32k<1, 4, 1, 1, 2, 3, EPI>(a, st);

@@ -36,6 +36,8 @@ STORE = [(33, 65, 128, "mfma32_kernel<1,4,2,1,"), (129, 96, 384, "mfma32_kernel<
          (1500, 4090, 1100, "mfma32_kernel<2,4,2,2,"), (520, 4090, 1100, "mfma32_kernel<1,4,2,1,"),
          (410, 4090, 1100, "mfma32k_kernel<1,4,1,1,2,3,"), (300, 4090, 1100, "mfma32k_kernel<1,2,1,1,2,3,"),
          (32, 40001, 1100, "mfma32k_kernel<1,2,1,1,2,3,"),
+         (1300, 2432, 700, "mfma32_kernel<1,4,2,1,"), (1281, 4090, 4100, "mfma32_kernel<2,4,2,2,"),
+         (513, 10900, 1100, "mfma32_kernel<2,4,2,2,"),
          (2100, 8200, 1100, "mfma32_kernel<2,4,2,2,"), (8190, 2401, 520, "mfma32_split_kernel<")]
 
 
