@@ -59,6 +59,19 @@ def param(module, name: str):
     return getattr(module, name) if p is None else p
 
 
+def stamped(module, names):
+    """The parameters ``names`` and what changes when one of them does: each one's version, address and dtype.  The
+    stamp is None, and nothing made from them may be kept for a later call, where one is an inference tensor (such a
+    tensor keeps no version: a parametrization's value, or a new parameter, under torch.inference_mode)."""
+    ts = [param(module, n) for n in names]
+    try:
+        return ts, [(t._version, t.data_ptr(), t.dtype) for t in ts]
+    except RuntimeError:
+        if any(t.is_inference() for t in ts):
+            return ts, None
+        raise
+
+
 def packed_weights(lins, dt, n: int):
     """The first n layers' current packed weights; every layer's weight must be of dtype ``dt``, as F.linear
     requires of its operands."""

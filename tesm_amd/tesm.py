@@ -20,7 +20,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, backend_error, check_hip_call, packed_weights, param, same_packs
+from .bitlinear import BitLinear, backend_error, check_hip_call, packed_weights, same_packs, stamped
 from .hip_ops import on_device, raw_stream
 
 _WORKSPACES = {}
@@ -39,6 +39,10 @@ def workspace(device: torch.device, nbytes: int, stream=None, raw=None) -> torch
         buf = torch.empty((max(nbytes, 256),), dtype=torch.uint8, device=device)
         _WORKSPACES[key] = buf
     return buf
+
+
+def _rounded_f32(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    return t.detach().to(dtype).to(torch.float32).contiguous()
 
 
 class TESM_SISO(nn.Module):
@@ -127,35 +131,34 @@ class TESM_SISO(nn.Module):
             self._rope[key] = tab
         return tab
 
-    def _local_bias_f32(self, dtype: torch.dtype) -> torch.Tensor:
+    def _derived(self, slot, ts, stamp, dtype, make):
+        """``make(ts)``, values made from parameters for the layer dtype, kept in ``slot`` while the parameters'
+        ``stamp`` (see ``stamped``) stays the same."""
+        held = self.__dict__.get(slot)
+        if stamp is None or held is None or held[0] != (stamp, dtype):
+            with torch.no_grad():
+                held = ((stamp, dtype), make(ts))
+            if stamp is not None:
+                self.__dict__[slot] = held
+        return held[1]
+
+    def _local_bias_f32(self, dtype: torch.dtype, ts, stamp) -> torch.Tensor:
         """``local_entanglement_bias`` rounded to the layer dtype (tesm.py:925), as float32.
 
         The kernels use its last ``min(W, L)`` entries, as the reference does."""
-        p = self.local_entanglement_bias
-        key = (p._version, p.data_ptr(), dtype)
-        if self._bias_cache is None or self._bias_cache[0] != key:
-            with torch.no_grad():
-                v = p.detach().to(dtype).to(torch.float32).contiguous()
-            self._bias_cache = (key, v)
-        return self._bias_cache[1]
+        return self._derived("_bias_cache", ts, stamp, dtype, lambda ts: _rounded_f32(ts[0], dtype))
 
-    def _global_params_f32(self, dtype):
+    def _global_params_f32(self, dtype, ts, stamp):
         """global_rel_pos_embed / _scale / _bias rounded to the layer dtype (tesm.py:980-982), as float32."""
-        ps = (self.global_rel_pos_embed, self.global_rel_pos_scale, self.global_rel_pos_bias)
-        key = tuple((p._version, p.data_ptr()) for p in ps) + (dtype,)
-        cached = self.__dict__.get("_global_cache")
-        if cached is None or cached[0] != key:
-            with torch.no_grad():
-                vals = tuple(p.detach().to(dtype).to(torch.float32).contiguous() for p in ps)
-            self.__dict__["_global_cache"] = (key, vals)
-        return self.__dict__["_global_cache"][1]
+        return self._derived("_global_cache", ts, stamp, dtype, lambda ts: tuple(_rounded_f32(t, dtype) for t in ts))
 
-    def _decay_bias_dt(self, dtype):
-        if self.decay_bias.dtype != dtype:
+    @staticmethod
+    def _decay_bias_dt(dtype, decay_bias):
+        if decay_bias.dtype != dtype:
             raise RuntimeError(
-                f"decay_bias is {self.decay_bias.dtype} but activations are {dtype}: convert the whole module with "
+                f"decay_bias is {decay_bias.dtype} but activations are {dtype}: convert the whole module with "
                 f"module.to({dtype}) (building with dtype= leaves decay_bias float32)")
-        return self.decay_bias.detach()
+        return decay_bias.detach()
 
     # -- forward ---------------------------------------------------------------------
     def forward(self, u, inference_params=None, cross_layer_state=None, prev_state=None, **kwargs):
@@ -189,17 +192,16 @@ class TESM_SISO(nn.Module):
         lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"], mods["cross_layer_q_proj"])
         glob = self.entanglement_window <= 0
         names = ("global_rel_pos_embed", "global_rel_pos_scale", "global_rel_pos_bias") if glob else ("local_entanglement_bias",)
-        biases = [param(self, n) for n in ("decay_bias",) + names]
+        biases, stamp = stamped(self, ("decay_bias",) + names)
         packs = packed_weights(lins, dt, 4 + int(cross))
         key = (dt, dev, cross, self.entanglement_window, self.state_scan_chunk_size, self.entanglement_threshold,
-               float(self.entanglement_scale), lins[0].bit_eps, self.d_model, self.d_state, self.ent_rank,
-               tuple((b._version, b.data_ptr(), b.dtype) for b in biases))
+               float(self.entanglement_scale), lins[0].bit_eps, self.d_model, self.d_state, self.ent_rank, stamp)
         plan = self.__dict__.get("_prefill_plan")
-        if plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
+        if stamp is not None and plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
             return plan[1]
-        decay_bias = self._decay_bias_dt(dt)
-        local_bias = None if glob else self._local_bias_f32(dt)
-        gparams = self._global_params_f32(dt) if glob else ()
+        decay_bias = self._decay_bias_dt(dt, biases[0])
+        local_bias = None if glob else self._local_bias_f32(dt, biases[1:], stamp and stamp[1:])
+        gparams = self._global_params_f32(dt, biases[1:], stamp and stamp[1:]) if glob else ()
         hip_ops.require_device(decay_bias, local_bias, *gparams)
         if decay_bias.device != dev:
             raise RuntimeError(f"hip backend ops need all tensors on one device, got {dev} and {decay_bias.device}")
@@ -224,7 +226,8 @@ class TESM_SISO(nn.Module):
         else:
             desc.local_bias = local_bias.data_ptr()
         keep = packs + [decay_bias, local_bias, gparams, biases]  # (biases: none of the key's addresses is reused)
-        self.__dict__["_prefill_plan"] = (key, (desc, keep))
+        if stamp is not None:
+            self.__dict__["_prefill_plan"] = (key, (desc, keep))
         return desc, keep
 
     def _prefill(self, u, cross_layer_state, prev_state, cache=None):
@@ -342,9 +345,9 @@ class TESM_SISO(nn.Module):
         for p in lins:
             if p.weight.dtype != dt:
                 raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
-        decay_bias = self._decay_bias_dt(dt)
+        decay_bias = self._decay_bias_dt(dt, self.decay_bias)
         if lb is not None:
-            local_bias = self._local_bias_f32(dt)
+            local_bias = self._local_bias_f32(dt, *stamped(self, ("local_entanglement_bias",)))
         else:
             # global layers decode over their one-slot ring with no bias (tesm.py:633, 1355-1357);
             # adding 0 to a score leaves it unchanged

@@ -22,7 +22,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, hip_ops
-from .bitlinear import BitLinear, check_hip_call, packed_weights, param, same_packs
+from .bitlinear import BitLinear, check_hip_call, packed_weights, same_packs, stamped
 from .hip_ops import on_device, raw_stream
 from .tesm import TESM_SISO, workspace
 
@@ -101,25 +101,26 @@ class TESMMIMO_Optimized(TESM_SISO):
         return tern, counts
 
     # -- cached device constants ---------------------------------------------------
-    def _mimo_coef(self, dtype):
-        """(coef, x0sq), each (n_heads, d_state) float32, recomputed when mimo_x / mimo_o change."""
-        x, o = self.mimo_x, self.mimo_o
+    def _mimo_coef(self, dtype, ts, stamp):
+        """(coef, x0sq), each (n_heads, d_state) float32, recomputed when mimo_x / mimo_o (``ts``) change."""
+        x, o = ts
         if x.dtype != dtype or o.dtype != dtype:
             raise RuntimeError(f"mimo_x / mimo_o are {x.dtype} but activations are {dtype}: convert the whole module "
                                f"with module.to({dtype})")
-        key = (x._version, x.data_ptr(), o._version, o.data_ptr(), dtype)
-        if self._coef_cache is None or self._coef_cache[0] != key:
-            H, Rm, D = x.shape
-            coef = torch.empty(H, D, dtype=torch.float32, device=x.device)
-            x0sq = torch.empty(H, D, dtype=torch.float32, device=x.device)
-            xc, oc = x.detach().contiguous(), o.detach().contiguous()
-            hip_ops.require_device(xc, oc, coef, x0sq)
-            lib = _lib.load()
-            _lib.check(lib.tesm_hip_mimo_coef(xc.data_ptr(), oc.data_ptr(), hip_ops.dt_code(dtype), H, Rm, D,
-                                              coef.data_ptr(), x0sq.data_ptr(),
-                                              ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)))
-            self._coef_cache = (key, coef, x0sq)
-        return self._coef_cache[1], self._coef_cache[2]
+        return self._derived("_coef_cache", ts, stamp, dtype, self._make_coef)
+
+    @staticmethod
+    def _make_coef(ts):
+        x, o = ts
+        H, Rm, D = x.shape
+        coef = torch.empty(H, D, dtype=torch.float32, device=x.device)
+        x0sq = torch.empty(H, D, dtype=torch.float32, device=x.device)
+        xc, oc = x.detach().contiguous(), o.detach().contiguous()
+        hip_ops.require_device(xc, oc, coef, x0sq)
+        _lib.check(_lib.load().tesm_hip_mimo_coef(xc.data_ptr(), oc.data_ptr(), hip_ops.dt_code(x.dtype), H, Rm, D,
+                                                  coef.data_ptr(), x0sq.data_ptr(),
+                                                  ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)))
+        return coef, x0sq
 
     def _mimo_layer_plan(self, dt, dev):
         """The prefill descriptor's fields that depend on the module alone (see TESM_SISO._layer_plan)."""
@@ -127,18 +128,17 @@ class TESMMIMO_Optimized(TESM_SISO):
         lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"])
         glob = self.entanglement_window <= 0
         names = ("global_rel_pos_embed", "global_rel_pos_scale", "global_rel_pos_bias") if glob else ("local_entanglement_bias",)
-        biases = [param(self, n) for n in ("decay_bias", "mimo_x", "mimo_o") + names]
+        biases, stamp = stamped(self, ("decay_bias", "mimo_x", "mimo_o") + names)
         packs = packed_weights(lins, dt, 4)
         key = (dt, dev, self.entanglement_window, self.entanglement_threshold, float(self.entanglement_scale),
-               lins[0].bit_eps, self.d_model, self.d_state, self.n_heads, self.ent_rank,
-               tuple((b._version, b.data_ptr(), b.dtype) for b in biases))
+               lins[0].bit_eps, self.d_model, self.d_state, self.n_heads, self.ent_rank, stamp)
         plan = self.__dict__.get("_mimo_plan")
-        if plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
+        if stamp is not None and plan is not None and plan[0] == key and same_packs(plan[1][1], packs):
             return plan[1]
-        decay_bias = self._decay_bias_dt(dt).contiguous()
-        local_bias = None if glob else self._local_bias_f32(dt)
-        gparams = self._global_params_f32(dt) if glob else ()
-        coef, x0sq = self._mimo_coef(dt)
+        decay_bias = self._decay_bias_dt(dt, biases[0]).contiguous()
+        local_bias = None if glob else self._local_bias_f32(dt, biases[3:], stamp and stamp[3:])
+        gparams = self._global_params_f32(dt, biases[3:], stamp and stamp[3:]) if glob else ()
+        coef, x0sq = self._mimo_coef(dt, biases[1:3], stamp and stamp[1:3])
         hip_ops.require_device(decay_bias, local_bias, coef, x0sq, *gparams)
         if decay_bias.device != dev:
             raise RuntimeError(f"hip backend ops need all tensors on one device, got {dev} and {decay_bias.device}")
@@ -162,7 +162,8 @@ class TESMMIMO_Optimized(TESM_SISO):
             desc.local_bias = local_bias.data_ptr()
         desc.mimo_coef, desc.mimo_x0sq = coef.data_ptr(), x0sq.data_ptr()
         keep = packs + [decay_bias, local_bias, gparams, coef, x0sq, biases]
-        self.__dict__["_mimo_plan"] = (key, (desc, keep))
+        if stamp is not None:
+            self.__dict__["_mimo_plan"] = (key, (desc, keep))
         return desc, keep
 
     # -- forward ---------------------------------------------------------------------
@@ -274,9 +275,9 @@ class TESMMIMO_Optimized(TESM_SISO):
         for p in lins[:4 + int(cross)]:
             if p.weight.dtype != dt:
                 raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
-        decay_bias = self._decay_bias_dt(dt).contiguous()
+        decay_bias = self._decay_bias_dt(dt, db).contiguous()
         if lb is not None:
-            local_bias = self._local_bias_f32(dt)
+            local_bias = self._local_bias_f32(dt, *stamped(self, ("local_entanglement_bias",)))
         else:
             # global layers decode over their one-slot rings with no bias (tesm_mimo.py:698, 862-866)
             local_bias = torch.zeros(self.n_heads, W, dtype=torch.float32, device=dev)

@@ -147,3 +147,17 @@ def test_threads_on_their_own_streams():
     assert not errors
     for g, w in zip(got, want):
         assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("kind", ["siso", "global", "mimo"])
+def test_parametrized_decay_bias_under_inference_mode(kind):
+    """There the computed bias is an inference tensor, which has no version a plan could compare."""
+    m, plain, u = _make(kind), _make(kind), _u()
+    rule = _Scale()
+    torch.nn.utils.parametrize.register_parametrization(m, "decay_bias", rule)
+    for factor in (2.0, -1.0, 0.5):
+        rule.factor = factor
+        with torch.no_grad():
+            plain.decay_bias.copy_(m.parametrizations.decay_bias.original * factor)
+        with torch.inference_mode():
+            assert torch.equal(m(u)[0], plain(u)[0]), factor
