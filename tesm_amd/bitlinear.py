@@ -61,11 +61,15 @@ def param(module, name: str):
 
 def stamped(module, names):
     """The parameters ``names`` and what changes when one of them does: each one's version, address and dtype.  The
-    stamp is None, and nothing made from them may be kept for a later call, where one is an inference tensor (such a
-    tensor keeps no version: a parametrization's value, or a new parameter, under torch.inference_mode)."""
-    ts = [param(module, n) for n in names]
+    stamp is None, and nothing made from them may be kept for a later call, where one is computed for every access
+    (parametrized or pruned: a new value may lie where an older one of the same version did) or is an inference tensor
+    (a parameter set under torch.inference_mode: it keeps no version)."""
+    ps = module._parameters
     try:
+        ts = [ps[n] for n in names]
         return ts, [(t._version, t.data_ptr(), t.dtype) for t in ts]
+    except KeyError:
+        return [getattr(module, n) for n in names], None
     except RuntimeError:
         if any(t.is_inference() for t in ts):
             return ts, None

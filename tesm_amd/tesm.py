@@ -113,13 +113,14 @@ class TESM_SISO(nn.Module):
         self.register_buffer("_stats_ternary_buffer", None, persistent=False)  # tesm.py:582-584
         self.register_buffer("_stats_total_buffer", torch.tensor(1.0), persistent=False)
         self._rope = {}
-        self._bias_cache = None
 
-    # descriptor plans hold device addresses (of tensors they keep alive): a copied or loaded module builds its own
-    _PLANS = ("_prefill_plan", "_decode_plan", "_mimo_plan", "_mimo_decode_plan")
+    # descriptor plans and values derived from parameters go by the addresses of tensors they keep alive: a copied or
+    # loaded module makes its own
+    _HELD = ("_prefill_plan", "_decode_plan", "_mimo_plan", "_mimo_decode_plan", "_bias_cache", "_global_cache",
+             "_coef_cache")
 
     def __getstate__(self):
-        return {k: v for k, v in self.__dict__.items() if k not in self._PLANS}
+        return {k: v for k, v in self.__dict__.items() if k not in self._HELD}
 
     # -- cached device constants ---------------------------------------------------
     def rope_table(self, L: int, dtype: torch.dtype, device: torch.device, pos_offset: int = 0) -> torch.Tensor:
@@ -133,11 +134,12 @@ class TESM_SISO(nn.Module):
 
     def _derived(self, slot, ts, stamp, dtype, make):
         """``make(ts)``, values made from parameters for the layer dtype, kept in ``slot`` while the parameters'
-        ``stamp`` (see ``stamped``) stays the same."""
+        ``stamp`` (see ``stamped``) stays the same.  The parameters' storage is kept with them, so that no later one
+        takes its address."""
         held = self.__dict__.get(slot)
         if stamp is None or held is None or held[0] != (stamp, dtype):
             with torch.no_grad():
-                held = ((stamp, dtype), make(ts))
+                held = ((stamp, dtype), make(ts), [t.detach() for t in ts])
             if stamp is not None:
                 self.__dict__[slot] = held
         return held[1]
@@ -225,7 +227,8 @@ class TESM_SISO(nn.Module):
             desc.global_scale, desc.global_bias = scale.data_ptr(), bias.data_ptr()
         else:
             desc.local_bias = local_bias.data_ptr()
-        keep = packs + [decay_bias, local_bias, gparams, biases]  # (biases: none of the key's addresses is reused)
+        # (the biases' storage, too: none of the key's addresses is taken by another)
+        keep = packs + [decay_bias, local_bias, gparams, [b.detach() for b in biases]]
         if stamp is not None:
             self.__dict__["_prefill_plan"] = (key, (desc, keep))
         return desc, keep

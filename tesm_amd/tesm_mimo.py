@@ -64,7 +64,6 @@ class TESMMIMO_Optimized(TESM_SISO):
         self.in_proj = BitLinear(d_model, n_proj, **bl)
         self.state_proj = BitLinear(self.d_state_total, d_model, **bl)
         self.ent_proj = BitLinear(self.d_state_total, d_model, **bl)
-        self._coef_cache = None
         self._stats_totals = {}
 
     # -- entanglement statistics (tesm_mimo.py:458-523) --------------------------------
@@ -161,7 +160,7 @@ class TESMMIMO_Optimized(TESM_SISO):
         else:
             desc.local_bias = local_bias.data_ptr()
         desc.mimo_coef, desc.mimo_x0sq = coef.data_ptr(), x0sq.data_ptr()
-        keep = packs + [decay_bias, local_bias, gparams, coef, x0sq, biases]
+        keep = packs + [decay_bias, local_bias, gparams, coef, x0sq, [b.detach() for b in biases]]
         if stamp is not None:
             self.__dict__["_mimo_plan"] = (key, (desc, keep))
         return desc, keep

@@ -161,3 +161,23 @@ def test_parametrized_decay_bias_under_inference_mode(kind):
             plain.decay_bias.copy_(m.parametrizations.decay_bias.original * factor)
         with torch.inference_mode():
             assert torch.equal(m(u)[0], plain(u)[0]), factor
+
+
+@pytest.mark.parametrize("kind,name", [("siso", "local_entanglement_bias"), ("global", "global_rel_pos_embed"),
+                                       ("global", "global_rel_pos_scale"), ("global", "global_rel_pos_bias"),
+                                       ("mimo", "local_entanglement_bias"), ("mimo", "mimo_x"), ("mimo", "mimo_o")])
+def test_parametrized_parameters_bf16(kind, name):
+    """Values that are rounded or combined before a plan holds them: each of a row of changed ones reaches the call,
+    though the allocator hands out the addresses of earlier ones again."""
+    dt = torch.bfloat16
+    m, plain, u = _make(kind, dt), _make(kind, dt), _u(dt)
+    with torch.no_grad():
+        for x in (m, plain):
+            getattr(x, name).add_(0.25)
+    rule = _Scale()
+    torch.nn.utils.parametrize.register_parametrization(m, name, rule)
+    for factor in (2.0, -1.0, 0.5, 4.0, 2.0, -3.0, 0.25):
+        rule.factor = factor
+        with torch.no_grad():
+            getattr(plain, name).copy_(getattr(m.parametrizations, name).original * factor)
+        assert torch.equal(_out(m, u), _out(plain, u)), factor
