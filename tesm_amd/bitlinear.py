@@ -64,13 +64,17 @@ def stamped(module, names):
     stamp is None, and nothing made from them may be kept for a later call, where one is computed for every access
     (parametrized or pruned: a new value may lie where an older one of the same version did) or is an inference tensor
     (a parameter set under torch.inference_mode: it keeps no version)."""
-    ps = module._parameters
+    ps, ts, stamp = module._parameters, [], []
     try:
-        ts = [ps[n] for n in names]
-        return ts, [(t._version, t.data_ptr(), t.dtype) for t in ts]
+        for n in names:  # (once per decoded token: no comprehension's frame)
+            t = ps[n]
+            ts.append(t)
+            stamp.append((t._version, t.data_ptr(), t.dtype))
+        return ts, stamp
     except KeyError:
         return [getattr(module, n) for n in names], None
     except RuntimeError:
+        ts = [param(module, n) for n in names]
         if any(t.is_inference() for t in ts):
             return ts, None
         raise

@@ -323,34 +323,31 @@ class TESM_SISO(nn.Module):
             "cache_filled": False,
         }
 
-    def _step_key(self, B, dt, dev, cdt, W, cross):
-        """What the decode descriptor depends on: shapes, dtypes, thresholds, and the version and storage
-        of every weight and bias (the packed weights follow tesm.py:226-236's cache rule)."""
-        # modules and parameters read from their dicts: this runs once per decoded token, and
-        # nn.Module.__getattr__ costs a fraction of a microsecond per lookup
-        mods, params = self._modules, self._parameters
-        lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"], mods["cross_layer_q_proj"])
-        db, lb = params["decay_bias"], params["local_entanglement_bias"]
-        lb_key = (lb._version, lb.data_ptr()) if lb is not None else None
-        return (B, dt, dev, cdt, W, cross, self.entanglement_threshold, float(self.entanglement_scale), db._version,
-                db.data_ptr(), db.dtype, lb_key, tuple(p.cache_key() for p in lins))
+    def _step_biases(self):
+        """The decode step's biases (a global layer has no window bias) and their stamp (see ``stamped``)."""
+        glob = self._parameters.get("local_entanglement_bias", self) is None
+        return stamped(self, ("decay_bias",) if glob else ("decay_bias", "local_entanglement_bias"))
 
     def _step_plan(self, B, dt, dev, cdt, W, cross):
-        """The decode descriptor's fields that stay fixed from step to step, rebuilt when a shape, a
-        dtype, a weight or a bias changes (``_step_key``)."""
-        mods, params = self._modules, self._parameters
+        """The decode descriptor's fields that stay fixed from step to step, rebuilt when a shape, a dtype, a
+        threshold, or the version or storage of a weight or bias changes (the packed weights follow
+        tesm.py:226-236's cache rule)."""
+        # modules read from their dict: this runs once per decoded token, and nn.Module.__getattr__ costs a
+        # fraction of a microsecond per lookup
+        mods = self._modules
         lins = (mods["in_proj"], mods["state_proj"], mods["ent_proj"], mods["out_proj"], mods["cross_layer_q_proj"])
-        lb = params["local_entanglement_bias"]
-        key = self._step_key(B, dt, dev, cdt, W, cross)
+        biases, stamp = self._step_biases()
+        key = (B, dt, dev, cdt, W, cross, self.entanglement_threshold, float(self.entanglement_scale), stamp,
+               [p.cache_key() for p in lins])
         plan = self.__dict__.get("_decode_plan")
-        if plan is not None and plan[0] == key:
+        if stamp is not None and plan is not None and plan[0] == key:
             return plan[1]
         for p in lins:
             if p.weight.dtype != dt:
                 raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
-        decay_bias = self._decay_bias_dt(dt, self.decay_bias)
-        if lb is not None:
-            local_bias = self._local_bias_f32(dt, *stamped(self, ("local_entanglement_bias",)))
+        decay_bias = self._decay_bias_dt(dt, biases[0])
+        if len(biases) > 1:
+            local_bias = self._local_bias_f32(dt, biases[1:], stamp and stamp[1:])
         else:
             # global layers decode over their one-slot ring with no bias (tesm.py:633, 1355-1357);
             # adding 0 to a score leaves it unchanged
@@ -374,9 +371,11 @@ class TESM_SISO(nn.Module):
             raise RuntimeError(f"hip backend ops need all tensors on one device, got {decay_bias.device} and {dev}")
         desc.decay_bias = decay_bias.data_ptr()
         desc.local_bias = local_bias.data_ptr()
-        keep = (decay_bias, local_bias) + tuple(p.packed_weight() for p in lins[:4 + int(cross)])
+        keep = (decay_bias, local_bias, [b.detach() for b in biases])
+        keep += tuple(p.packed_weight() for p in lins[:4 + int(cross)])
         nbytes = int(_lib.load().tesm_hip_siso_decode_ws_bytes(ctypes.byref(desc)))
-        self.__dict__["_decode_plan"] = (key, (desc, nbytes, keep))
+        if stamp is not None:
+            self.__dict__["_decode_plan"] = (key, (desc, nbytes, keep))
         return desc, nbytes, keep
 
     def _forward_incremental(self, u, inference_params, cross_layer_state=None):
@@ -405,7 +404,7 @@ class TESM_SISO(nn.Module):
             cs = cross_layer_state.reshape(B, D).to(dt).contiguous()
             if cs.device != dev:
                 raise RuntimeError(f"hip backend ops need all tensors on one device, got {cs.device} and {dev}")
-        desc, nbytes, _ = self._step_plan(B, dt, dev, kc.dtype, W, cs is not None)
+        desc, nbytes, keep = self._step_plan(B, dt, dev, kc.dtype, W, cs is not None)
         y = torch.empty((B, 1, dm), dtype=dt, device=dev)
         state_out = torch.empty_like(state)
         new = torch.empty((B, D), dtype=dt, device=dev)

@@ -264,19 +264,18 @@ class TESMMIMO_Optimized(TESM_SISO):
         """The decode descriptor's fields that stay fixed from step to step, rebuilt when a shape, a
         dtype, a weight or a bias changes."""
         lins = (self.in_proj, self.state_proj, self.ent_proj, self.out_proj, self.cross_layer_q_proj)
-        db, lb = self.decay_bias, self.local_entanglement_bias
-        lb_key = (lb._version, lb.data_ptr()) if lb is not None else None
-        key = (B, dt, dev, cdt, W, cross, self.entanglement_threshold, float(self.entanglement_scale), db._version,
-               db.data_ptr(), db.dtype, lb_key, tuple(p.cache_key() for p in lins))
+        biases, stamp = self._step_biases()
+        key = (B, dt, dev, cdt, W, cross, self.entanglement_threshold, float(self.entanglement_scale), stamp,
+               [p.cache_key() for p in lins])
         plan = self.__dict__.get("_mimo_decode_plan")
-        if plan is not None and plan[0] == key:
+        if stamp is not None and plan is not None and plan[0] == key:
             return plan[1]
         for p in lins[:4 + int(cross)]:
             if p.weight.dtype != dt:
                 raise RuntimeError(f"expected both operands to have the same dtype, got {dt} and {p.weight.dtype}")
-        decay_bias = self._decay_bias_dt(dt, db).contiguous()
-        if lb is not None:
-            local_bias = self._local_bias_f32(dt, *stamped(self, ("local_entanglement_bias",)))
+        decay_bias = self._decay_bias_dt(dt, biases[0]).contiguous()
+        if len(biases) > 1:
+            local_bias = self._local_bias_f32(dt, biases[1:], stamp and stamp[1:])
         else:
             # global layers decode over their one-slot rings with no bias (tesm_mimo.py:698, 862-866)
             local_bias = torch.zeros(self.n_heads, W, dtype=torch.float32, device=dev)
@@ -300,9 +299,11 @@ class TESMMIMO_Optimized(TESM_SISO):
             desc.cross_q_proj = self.cross_layer_q_proj.linear_desc()
         desc.decay_bias = decay_bias.data_ptr()
         desc.local_bias = local_bias.data_ptr()
-        keep = (decay_bias, local_bias) + tuple(p.packed_weight() for p in lins[:4 + int(cross)])
+        keep = (decay_bias, local_bias, [b.detach() for b in biases])
+        keep += tuple(p.packed_weight() for p in lins[:4 + int(cross)])
         nbytes = int(_lib.load().tesm_hip_mimo_decode_ws_bytes(ctypes.byref(desc)))
-        self.__dict__["_mimo_decode_plan"] = (key, (desc, nbytes, keep))
+        if stamp is not None:
+            self.__dict__["_mimo_decode_plan"] = (key, (desc, nbytes, keep))
         return desc, nbytes, keep
 
     def _forward_incremental(self, u, inference_params, cross_layer_state=None):
@@ -339,7 +340,7 @@ class TESMMIMO_Optimized(TESM_SISO):
             cs = cross_layer_state.reshape(B, H, D).to(dt).contiguous()
             if cs.device != dev:
                 raise RuntimeError(f"hip backend ops need all tensors on one device, got {cs.device} and {dev}")
-        desc, nbytes, _ = self._mimo_step_plan(B, dt, dev, kc.dtype, W, cs is not None)
+        desc, nbytes, keep = self._mimo_step_plan(B, dt, dev, kc.dtype, W, cs is not None)
         y = torch.empty((B, 1, dm), dtype=dt, device=dev)
         state_out = torch.empty_like(state)
         new = torch.empty((B, H, D), dtype=dt, device=dev)

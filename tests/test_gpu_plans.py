@@ -181,3 +181,18 @@ def test_parametrized_parameters_bf16(kind, name):
         with torch.no_grad():
             getattr(plain, name).copy_(getattr(m.parametrizations, name).original * factor)
         assert torch.equal(_out(m, u), _out(plain, u)), factor
+
+
+@pytest.mark.parametrize("kind,name", [("siso", "decay_bias"), ("siso", "local_entanglement_bias"), ("global", "decay_bias"),
+                                       ("mimo", "decay_bias"), ("mimo", "local_entanglement_bias")])
+def test_parametrized_biases_in_decode_steps(kind, name):
+    m, plain, u = _make(kind), _make(kind), _u(L=12)
+    rule = _Scale()
+    torch.nn.utils.parametrize.register_parametrization(m, name, rule)
+    caches = [{"state_cache": x.allocate_inference_cache(2, 64)} for x in (m, plain)]
+    for t in range(9):
+        rule.factor = (2.0, -1.0, 0.5)[t % 3]
+        with torch.no_grad():
+            getattr(plain, name).copy_(getattr(m.parametrizations, name).original * rule.factor)
+            y, want = (x(u[:, t:t + 1], inference_params=c)[0] for x, c in zip((m, plain), caches))
+        assert torch.equal(y, want), t

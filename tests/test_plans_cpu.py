@@ -118,3 +118,21 @@ def test_copies_hold_no_derived_values(kind):
     twin = copy.deepcopy(m)
     assert not [k for k in held if twin.__dict__.get(k) is not None]
     assert _prefill_plan(twin, torch.bfloat16)[0].d_state == D
+
+
+@pytest.mark.parametrize("kind,name", [("siso", "decay_bias"), ("siso", "local_entanglement_bias"), ("global", "decay_bias"),
+                                       ("mimo", "decay_bias"), ("mimo", "local_entanglement_bias")])
+@pytest.mark.parametrize("mode", [torch.no_grad, torch.inference_mode])
+def test_decode_plans_take_computed_biases(kind, name, mode):
+    dt, cpu = torch.float32 if name == "decay_bias" else torch.bfloat16, torch.device("cpu")
+    m = _make(kind, dt)
+    rule = _Reused()
+    torch.nn.utils.parametrize.register_parametrization(m, name, rule, unsafe=True)
+    args = (4, dt, cpu, torch.float32, 1 if kind == "global" else 8, False)
+    field = "decay_bias" if name == "decay_bias" else "local_bias"
+    for factor in (2.0, -1.0, 0.5, 2.0):
+        rule.factor = factor
+        with mode():
+            desc, _, keep = m._mimo_step_plan(*args) if kind == "mimo" else m._step_plan(*args)
+        want = (getattr(m.parametrizations, name).original * factor).detach().float().reshape(-1)
+        assert np.array_equal(_floats(getattr(desc, field), want.numel()), want.numpy()), factor
