@@ -138,8 +138,7 @@ class TESM_SISO(nn.Module):
         takes its address."""
         held = self.__dict__.get(slot)
         if stamp is None or held is None or held[0] != (stamp, dtype):
-            with torch.no_grad():
-                held = ((stamp, dtype), make(ts), [t.detach() for t in ts])
+            held = ((stamp, dtype), make(ts), [t.detach() for t in ts])
             if stamp is not None:
                 self.__dict__[slot] = held
         return held[1]
@@ -228,7 +227,7 @@ class TESM_SISO(nn.Module):
         else:
             desc.local_bias = local_bias.data_ptr()
         # (the biases' storage, too: none of the key's addresses is taken by another)
-        keep = packs + [decay_bias, local_bias, gparams, [b.detach() for b in biases]]
+        keep = packs + [decay_bias, local_bias, gparams, [b.detach() for b in biases[1:]]]
         if stamp is not None:
             self.__dict__["_prefill_plan"] = (key, (desc, keep))
         return desc, keep
@@ -371,7 +370,7 @@ class TESM_SISO(nn.Module):
             raise RuntimeError(f"hip backend ops need all tensors on one device, got {decay_bias.device} and {dev}")
         desc.decay_bias = decay_bias.data_ptr()
         desc.local_bias = local_bias.data_ptr()
-        keep = (decay_bias, local_bias, [b.detach() for b in biases])
+        keep = (decay_bias, local_bias, [b.detach() for b in biases[1:]])
         keep += tuple(p.packed_weight() for p in lins[:4 + int(cross)])
         nbytes = int(_lib.load().tesm_hip_siso_decode_ws_bytes(ctypes.byref(desc)))
         if stamp is not None:
