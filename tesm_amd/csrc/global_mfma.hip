@@ -275,6 +275,7 @@ __global__ __launch_bounds__(kGNT, 4) void global_mfma_kernel(GlobalArgs a, cons
       lds_put4((lds_cptr)(reinterpret_cast<const char*>(tab + tid)), nt);  // (every wave is past its scores)
       wg_barrier();
       load_states(k0 + kGK, 1);
+      asm volatile("" ::: "memory");  // the waits count on these loads before the next block's keys and bias entries
       rlo = nlo;
     }
   };
