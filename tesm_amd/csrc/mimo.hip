@@ -324,15 +324,15 @@ __global__ __launch_bounds__(64 * kStNW) void mimo_stats_kernel(MimoStatsArgs a)
     }
   };
   int32_t pos = 0, neg = 0;
-  for (int e0 = 0; e0 < n; e0 += kStNW * ns) {  // (uniform)
-    const int ew = e0 + wv * ns;                // the wave's first score
-    const int nw = n - ew < ns ? n - ew : ns;   // (none: <= 0)
+  for (int64_t e0 = 0; e0 < n; e0 += kStNW * ns) {  // (uniform; the step past the last score may not fit an int)
+    const int64_t ew = e0 + wv * ns;                // the wave's first score
+    const int nw = n - ew < ns ? static_cast<int>(n - ew) : ns;  // (none: <= 0)
     float acc = 0.0f;
     for (int r0 = 0; r0 < T; r0 += sl) {
       const int m = T - r0 < sl ? T - r0 : sl;
       for (int si = 0; si < nw; ++si) {
         int tq, tk, h0;  // (uniform: the divisions are scalar, and only the global branch has one per product)
-        place(__builtin_amdgcn_readfirstlane(ew + si), tq, tk, h0);
+        place(__builtin_amdgcn_readfirstlane(static_cast<int>(ew) + si), tq, tk, h0);
         const int64_t qo = (b * a.L + tq) * a.ld_q, ko = (b * a.L + tk) * a.ld_k;
         const float2 *rq = a.rope + static_cast<int64_t>(tq) * half, *rk = a.rope + static_cast<int64_t>(tk) * half;
 #pragma unroll 4
