@@ -56,28 +56,6 @@ __device__ __forceinline__ void store4(void* out, int64_t idx, const float (&v)[
   }
 }
 
-template <int DT>
-__device__ __forceinline__ void load4(const void* p, int64_t idx, bool vec, float (&v)[4]) {
-  if (vec) {
-    if constexpr (DT == kBF16) {
-      const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(p) + idx);
-      v[0] = __uint_as_float(w.x << 16);
-      v[1] = __uint_as_float(w.x & 0xffff0000u);
-      v[2] = __uint_as_float(w.y << 16);
-      v[3] = __uint_as_float(w.y & 0xffff0000u);
-    } else {
-      const float4 f = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + idx);
-      v[0] = f.x;
-      v[1] = f.y;
-      v[2] = f.z;
-      v[3] = f.w;
-    }
-  } else {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = ld<DT>(p, idx + r);
-  }
-}
-
 // 4-element vector access at element (m * ld + n) is aligned for every m and every n % 4 == 0.
 template <int DT>
 __device__ __forceinline__ bool vec4_ok(const void* p, int64_t ld) {
@@ -122,10 +100,6 @@ __device__ __forceinline__ void gate_act4(const LinearArgs& a, int kind, int64_t
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = rnd<DT>(sigmoidf_(rnd<DT>(v[r])));
   }
-}
-
-__device__ __forceinline__ void lds_dma16(const void* src, char* dst) {
-  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(dst), 16, 0, 0);
 }
 
 // s_waitcnt with only the vector-memory counter constrained (gfx9 encoding: vmcnt bits [3:0] and
