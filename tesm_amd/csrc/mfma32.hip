@@ -520,8 +520,10 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //     that, 26.9 against 26.0; above K 4096 from five CUs in eight (with the quantization: 1400 x 4096 x 11008 78.2,
 //     64x128 84.3; 1200 77.5, 78.6; 1100 no difference).  Grids past two rounds walk 8 M tiles per group, past short K
 //     those past one (3000 x 4096 x 4096 54.5, by fours 59.2), at K above 4096 all (1500 x 4096 x 11008 f32 77.0, by
-//     fours 85.9), and with five M tiles (513 x 11008 x 4096 with the quantization 36.0, by fours 36.6; seven or
-//     eight M tiles of 8192 columns 37.0-40.0, by fours 36.6-39.3).
+//     fours 85.9), and those of five M tiles, where four and one leave one by itself (513 x 12992 x 4096 32.6, by fours
+//     33.5, f32 34.2, 35.8; the less of the fifth tile is filled the more: over 27 sizes of K 1536-4096 from 4.5 %
+//     faster to 0.7 slower, 1.3 in the mean, none at 640 rows).  Other counts gain nothing to speak of: six or seven
+//     3 % faster to 3 slower, 0.4 in the mean; one to four and 8 to 21 within 1.6 %, with 9, 13, 17 and 21 among them.
 //   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
 //     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
 //   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU, past short K one: 8192 x 768 x 768 10.6
@@ -558,7 +560,7 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
   if (a.Kp > 3 * kKTile) {
     const bool most = a.Kp > 4096 ? 8 * big >= 5 * cus : 4 * big >= 3 * cus;
     const bool wide = big >= cus || (most && a.Kp > 1024 && a.M > 64);
-    const bool five = a.M > 512 && a.M <= 640;  // M tiles: groups of four would leave one by itself
+    const bool five = a.M > 512 && a.M <= 640;  // M tiles: by fours the fifth shares no weights in its XCD
     if (big >= 2 * cus || (wide && (a.Kp > 4096 || ((big > cus || five) && a.Kp > 1024)))) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
     if (wide) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
     const int64_t mid = tiles(64, 128);

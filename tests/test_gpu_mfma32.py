@@ -63,6 +63,21 @@ def test_store_products_exact(M, N, K, kernel, dtype):
         assert torch.equal(wide[:, :N], want) and bool((wide[:, N:] == 7.0).all())
 
 
+# grids of one round: five M tiles are walked as one group (the kernel's last argument), others by fours
+@pytest.mark.parametrize("M,N,order", [(512, 13053, 0), (513, 10900, 2), (640, 12800, 2), (641, 9200, 0), (1100, 7000, 0)])
+def test_tile_walk_exact(M, N, order):
+    K = 1100
+    g = torch.Generator().manual_seed(M)
+    x, w = (torch.randn(n, K, generator=g).to(torch.bfloat16).to(DEV) for n in (M, N))
+    s_w, c_w = hip_ops.absmean_scale(w)
+    packed = hip_ops.pack_weight(w, s_w)
+    (q, s, rs), qd = _codes(x)
+    with hip_ops.launch_log() as log:
+        out = hip_ops.bitlinear(q, s, rs, packed, c_w, N, K, torch.bfloat16)
+    assert log.kernels == [f"mfma32_kernel<2,4,2,2,0,1,{order}>"], log.kernels
+    assert torch.equal(out, _expect(qd @ hip_ops.unpack_weight(packed, K).double().t(), s, c_w, torch.bfloat16))
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 200, 2100), (2100, 2050, 1030)])
 def test_bias_and_accumulators(M, N, K):
     """The general epilogue behind a K-group tile and a large one: bias and the accumulator dump."""
