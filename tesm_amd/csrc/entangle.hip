@@ -20,6 +20,7 @@
 #include <cstdlib>
 
 #include "entangle.h"
+#include "linear_dev.h"
 #include "tesm_hip_internal.h"
 
 namespace tesm {
@@ -1469,22 +1470,37 @@ static int64_t eff_window(const EntArgs& a) { return a.mimo ? a.W : std::min(a.W
 
 constexpr int kRegTS = 8;  // positions per thread of the register-mix kernel
 
+template <int DT, int WM, int KI, int NTM, int HV, int MW>
+static void launch_reg_n(const EntArgs& a, int64_t weff, const RegLds& f, dim3 grid, unsigned nt, hipStream_t st) {
+  constexpr int TS = kRegTS;
+  ent_reg_kernel<DT, WM, KI, NTM, TS, HV, MW><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, NTM, TS, HV, MW>)>>>(a, weff, f);
+}
+
 template <int DT, int WM, int KI, int HV>
 static void launch_reg_k(const EntArgs& a, int64_t weff, const RegLds& f, hipStream_t st) {
   constexpr int TS = kRegTS;
-  dim3 grid(static_cast<unsigned>((a.L + HV * TS - 1) / (HV * TS)), static_cast<unsigned>(a.B));
-  const unsigned nt = static_cast<unsigned>(HV * a.D);  // (D > 256: one half of at most 512 threads, two per CU)
+  const dim3 grid(static_cast<unsigned>((a.L + HV * TS - 1) / (HV * TS)), static_cast<unsigned>(a.B));
+  const unsigned nt = static_cast<unsigned>(HV * a.D);  // the register cap follows it (one half: two workgroups per CU)
   if constexpr (HV == 1)
-    ent_reg_kernel<DT, WM, KI, 512, TS, 1, 4><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 512, TS, 1, 4>)>>>(a, weff, f);
+    launch_reg_n<DT, WM, KI, 512, 1, 4>(a, weff, f, grid, nt, st);
+  else if (nt > 768)
+    launch_reg_n<DT, WM, KI, 1024, 2, 1>(a, weff, f, grid, nt, st);
+  else if (nt > 512)
+    launch_reg_n<DT, WM, KI, 768, 2, 1>(a, weff, f, grid, nt, st);
   else
-    ent_reg_kernel<DT, WM, KI, 512, TS, 2, 1><<<grid, nt, f.total, TESM_LOGGED(st, ent_reg_kernel<DT, WM, KI, 512, TS, 2, 1>)>>>(a, weff, f);
+    launch_reg_n<DT, WM, KI, 512, 2, 1>(a, weff, f, grid, nt, st);
+}
+
+// Key staging items per thread of a workgroup of HV halves.
+static int64_t reg_key_items(const EntArgs& a, int64_t weff, int hv) {
+  return ((hv * kRegTS + weff - 1) * (a.R / 2) + hv * a.D - 1) / (hv * a.D);
 }
 
 template <int DT, int HV>
 static void run_reg_hv(const EntArgs& a, int64_t weff, hipStream_t st) {
   const int wm = weff <= 16 ? 16 : 32;
   const RegLds f = reg_lds(a.D, a.R, weff, wm, DT == kBF16 ? 2 : 4, HV * kRegTS);
-  const int64_t ki = ((HV * kRegTS + weff - 1) * (a.R / 2) + HV * a.D - 1) / (HV * a.D);  // first-round key items
+  const int64_t ki = reg_key_items(a, weff, HV);
   if (wm == 16) {
     if (ki <= 2) launch_reg_k<DT, 16, 2, HV>(a, weff, f, st);
     else if (ki == 3) launch_reg_k<DT, 16, 3, HV>(a, weff, f, st);
@@ -1496,14 +1512,39 @@ static void run_reg_hv(const EntArgs& a, int64_t weff, hipStream_t st) {
   }
 }
 
-// Rows of more than 256 channels take one half per workgroup: 8 positions, at most 512 threads, two workgroups per CU
-// (with both halves 1024 threads take a CU, so a grid just past the CUs runs two full rounds, and nothing overlaps the
-// loads).  3 x 1365 tokens, D 512, rank 80, bf16 25.4 us against 32.7; 4 x 8192 115 against 127, 1 x 200 15.1 against
-// 19.6, 3 x 1365 f32 27.0 against 33.6; only a grid of exactly one round of both halves is no faster (1 x 4096 22.9
-// against 21.8).  Narrower rows keep both (1 x 4096, D 256, rank 64, f32 14.0; one half 15.0).
+// One half per workgroup (8 positions, at most 512 threads, two or three workgroups per CU), or both (16 positions, one
+// workgroup of up to 1024 threads per CU)?  Both stage the window's keys once for 16 positions, but run in whole rounds
+// of the CUs, with nothing to overlap the loads.  us, of k one-half workgroups per CU:
+//   * k odd: both would leave half a round or more idle.  One half: 3 x 1365, D 512, rank 80, bf16 25.4 against
+//     32.7, f32 27.0, 33.6; 1 x 200 15.1, 19.6; D 384, rank 96, f32 1 x 2048 13.9, 17.3; 1 x 6144 29.8, 32.4.
+//   * k even, so the rounds of both nearly full: staging once weighs against the overlap, and the more rounds, the
+//     more the overlap is worth.  f32, window 32, by rounds of both: D 512, rank 80 1 18.1 (one half 20.1), 2 34.2
+//     (33.6), 4 65.8 (59.3); D 384, rank 96 1 17.5 (21.0), 2 33.5 (35.6), 4 64.4 (65.9), 6 94.6 (92.8); D 320, rank
+//     64 1 17.3 (17.1).  Short windows have fewer keys to stage twice (1 round, D 512, rank 80, window 16 14.2, 13.4),
+//     wide ranks more (1 round, D 512, rank 256, window 16 16 % slower in one half).
+//   * the one-half forms of bf16, and of float32 with four key items at a short window, take 103-128 registers
+//     instead of up to 96: narrow rows then have two workgroups on a CU instead of three (D 384, rank 128, bf16 2
+//     rounds 38.0, one half 51.8; 6 rounds 101.1, 121.4).
+// The numbers below are where the measured ratios cross one (D 320-512, ranks 32-256, windows 8-32, 96 to 1536
+// workgroups of both); what they leave is within 5 % of the better form but for ranks above 128, within 12.
+static bool reg_one_half(const EntArgs& a, int64_t weff) {
+  if (a.D <= 256) return false;  // (1 x 4096, D 256, rank 64, f32: both 14.0, one half 15.0)
+  const int64_t cus = std::max(device_limits().cus, 1);
+  const int64_t n16 = (a.L + 2 * kRegTS - 1) / (2 * kRegTS) * a.B;  // workgroups of both
+  const int64_t k = ((a.L + kRegTS - 1) / kRegTS * a.B + cus - 1) / cus, rounds = k / 2;
+  const bool wide = a.R > 160, heavy = a.dt == kBF16 || (weff <= 16 && reg_key_items(a, weff, 1) >= 4);
+  if (k % 2) return !heavy || k < 5 || (a.D >= 448 && (k < 9 || !wide || a.D >= 512 || weff <= 16));
+  if (a.D < 384) return !heavy && rounds >= (a.R <= 64 ? 1 : wide ? 4 : 2);
+  if (a.D < 448) return !heavy && !wide && rounds >= 4;
+  if (weff <= 16) return !wide || (rounds == 1 ? 16 * n16 <= 13 * cus : a.D >= 512 || rounds != 3);
+  if (a.dt == kBF16) return a.D >= 512 && rounds >= (wide ? 3 : 2);
+  if (rounds == 1) return a.R <= 96 && 8 * n16 <= 5 * cus;
+  return rounds >= (a.R <= 96 ? 2 : wide ? 4 : 3);
+}
+
 template <int DT>
 static int run_reg(const EntArgs& a, int64_t weff, hipStream_t st) {
-  if (a.D > 256)
+  if (reg_one_half(a, weff))
     run_reg_hv<DT, 1>(a, weff, st);
   else
     run_reg_hv<DT, 2>(a, weff, st);
