@@ -287,78 +287,92 @@ __global__ __launch_bounds__(256) void mimo_final_kernel(const float* S, const f
   if (last) last[i] = v;
 }
 
-// One workgroup of 16 waves per batch row.  A wave takes up to 64 scores at a time: its lanes form their products side
-// by side (rows of q and k read contiguously) into the wave's slab of LDS, a slice of at most kStSL of a score's
-// products at once, then one lane per score adds its slice in natural order.  Bound by the latency of those two phases.
-// With one thread per score (256 threads, each walking its own rows of q and k) 1 x 256 scores of 256 products took
-// 101 us, now 58.
-constexpr int kStNW = 16;               // waves
-constexpr int kStSL = 256;              // products of a score per slice
-constexpr int kStSlab = 2048;           // products per wave and slice
-constexpr int kStPitch = kStSlab + 64;  // slab (floats): rows are padded by one, so a score per lane reads all banks
+// One workgroup of 16 waves per batch row.  The RoPE'd q and k rows of the sampled positions are staged in LDS once per
+// group of hb heads (as many as fill the threads and fit), then a thread forms one score: its products in natural
+// (h, r) order, each rounded, from two rows.  Rows longer than a slice of sl values are staged slice by slice, and the
+// global branch's scores run over all heads.  VEC: rows of whole 16-byte groups; the pitch (R + 4 or R + 1) spreads
+// the lanes' key rows over all banks.
+// Bound by the staging's loads and the chain of additions.  us for 1 x 64 positions (before: one thread per score over
+// its own rows of q and k, bf16 and f32; in brackets a wave's lanes forming a score's products side by side): 4 heads of
+// rank 256, window 64 37 and 33 (97, 39 [49, 45]); rank 64, window 32 30 and 26 (398, 150 [239, 219]); 2 heads of rank
+// 16, window 8 5 (17, 10 [55, 50]); global, 4 heads of rank 32 10 and 11 (190, 71 [76, 68]).  A rank whose rows do not
+// fit whole rotates each pair twice: window 1, rank 400, the layer 142, 131 in the bracketed form.
+constexpr int kStNT = 1024;
+constexpr int kStNW = kStNT / 64;
+constexpr int kStLds = 144 * 1024;
 
-template <int DT>
-__global__ __launch_bounds__(64 * kStNW) void mimo_stats_kernel(MimoStatsArgs a) {
-  extern __shared__ float lds_st[];
+template <int DT, bool VEC>
+__global__ __launch_bounds__(kStNT) void mimo_stats_kernel(MimoStatsArgs a, int hb, int sl, int pitch) {
+  extern __shared__ __attribute__((aligned(16))) float lds_st[];
   __shared__ int32_t cnt[2][kStNW];
   const int64_t b = blockIdx.x;
-  const int half = static_cast<int>(a.R / 2), R = static_cast<int>(a.R), S = static_cast<int>(a.S);
-  const int H = static_cast<int>(a.H), W = static_cast<int>(a.W);
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // window branch: (v, h, w) over V = S - W + 1 complete windows; global branch: (s, t) over S x S, all heads
-  const int n = a.global ? S * S : (S - W + 1) * H * W;
-  const int T = a.global ? H * R : R;  // products per score, in natural (h, r) order
-  const int sl = T < kStSL ? T : kStSL, ns = kStSlab / sl < 64 ? kStSlab / sl : 64;
-  float* slab = lds_st + wv * kStPitch;
-  // score e: its query and key positions and its first head
-  auto place = [&](int e, int& tq, int& tk, int& h0) {
-    if (a.global) {
-      tq = e / S;
-      tk = e % S;
-      h0 = 0;
-    } else {
-      const int v = e / (H * W), w = e % W;
-      h0 = (e / W) % H;
-      tq = W - 1 + v;
-      tk = v + w;
+  const int R = static_cast<int>(a.R), half = R / 2, S = static_cast<int>(a.S), H = static_cast<int>(a.H);
+  const int W = static_cast<int>(a.W), tid = threadIdx.x;
+  // window branch: (v, h, w) over S - W + 1 complete windows; global branch: (s, t) over S x S, all heads
+  const int q0 = a.global ? 0 : W - 1, nq = S - q0, rows = nq + S;
+  const int per = a.global ? S * S : nq * W;  // scores of a head (global: of all)
+  const bool whole = sl >= R;
+  // elements r0 .. r0 + m - 1 of the rows of heads h0 .. h0 + nh - 1 (more than one only where rows are whole)
+  auto stage = [&](int h0, int nh, int r0, int m) {
+    const int width = whole ? half : m, n = nh * rows * width;
+#pragma unroll 4
+    for (int x = tid; x < n; x += kStNT) {
+      const int row = x / width, c = x - row * width, hl = row / rows, rr = row - hl * rows;
+      const int r = whole ? c : r0 + c, i = r < half ? r : r - half;
+      const bool isq = rr < nq;
+      const int64_t t = isq ? q0 + rr : rr - nq;
+      const int64_t o = (b * a.L + t) * (isq ? a.ld_q : a.ld_k) + static_cast<int64_t>(h0 + hl) * R + i;
+      const void* src = isq ? a.q : a.k;
+      float x1, x2;
+      rope_pair<DT>(ld<DT>(src, o), ld<DT>(src, o + half), a.rope[t * half + i], x1, x2);
+      float* dst = lds_st + row * pitch;
+      if (whole) {
+        dst[i] = x1;
+        dst[i + half] = x2;
+      } else {
+        dst[c] = r < half ? x1 : x2;
+      }
     }
   };
   int32_t pos = 0, neg = 0;
-  for (int64_t e0 = 0; e0 < n; e0 += kStNW * ns) {  // (uniform; the step past the last score may not fit an int)
-    const int64_t ew = e0 + wv * ns;                // the wave's first score
-    const int nw = n - ew < ns ? static_cast<int>(n - ew) : ns;  // (none: <= 0)
-    float acc = 0.0f;
-    for (int r0 = 0; r0 < T; r0 += sl) {
-      const int m = T - r0 < sl ? T - r0 : sl;
-      for (int si = 0; si < nw; ++si) {
-        int tq, tk, h0;  // (uniform: the divisions are scalar, and only the global branch has one per product)
-        place(__builtin_amdgcn_readfirstlane(static_cast<int>(ew) + si), tq, tk, h0);
-        const int64_t qo = (b * a.L + tq) * a.ld_q, ko = (b * a.L + tk) * a.ld_k;
-        const float2 *rq = a.rope + static_cast<int64_t>(tq) * half, *rk = a.rope + static_cast<int64_t>(tk) * half;
+  for (int h0 = 0; h0 < (a.global ? 1 : H); h0 += hb) {  // (uniform, as are the loops in it)
+    const int nh = H - h0 < hb ? H - h0 : hb, n = per * nh;
+    for (int e0 = 0; e0 < n; e0 += kStNT) {
+      const int e = e0 + tid, hl = e / per, es = e - hl * per;
+      const int qr = es / (a.global ? S : W), w = es - qr * (a.global ? S : W), kr = a.global ? w : qr + w;
+      float acc = 0.0f;
+      for (int h = h0; h < (a.global ? H : h0 + 1); ++h)
+        for (int r0 = 0; r0 < R; r0 += sl) {
+          const int m = R - r0 < sl ? R - r0 : sl;
+          if (!whole || a.global || e0 == 0) {
+            __syncthreads();  // every thread is done with the rows before
+            stage(h, a.global ? 1 : nh, r0, m);
+            __syncthreads();
+          }
+          if (e >= n) continue;
+          const float* pq = lds_st + (hl * rows + qr) * pitch;
+          const float* pk = lds_st + (hl * rows + nq + kr) * pitch;
+          if constexpr (VEC) {
 #pragma unroll 4
-        for (int x = lane; x < m; x += 64) {
-          const int r = r0 + x, h = a.global ? r / R : h0, rr = a.global ? r % R : r, i = rr < half ? rr : rr - half;
-          const int64_t hr = static_cast<int64_t>(h) * R + i;
-          float q1, q2, k1, k2;
-          rope_pair<DT>(ld<DT>(a.q, qo + hr), ld<DT>(a.q, qo + hr + half), rq[i], q1, q2);
-          rope_pair<DT>(ld<DT>(a.k, ko + hr), ld<DT>(a.k, ko + hr + half), rk[i], k1, k2);
-          slab[si * (m + 1) + x] = rr < half ? rnd<DT>(q1 * k1) : rnd<DT>(q2 * k2);
-        }
-      }
-      __syncthreads();
-      if (lane < nw) {
-        const float* row = slab + lane * (m + 1);
+            for (int r = 0; r < m; r += 4) {
+              const float4 x = *reinterpret_cast<const float4*>(pq + r), y = *reinterpret_cast<const float4*>(pk + r);
+              acc += rnd<DT>(x.x * y.x);
+              acc += rnd<DT>(x.y * y.y);
+              acc += rnd<DT>(x.z * y.z);
+              acc += rnd<DT>(x.w * y.w);
+            }
+          } else {
 #pragma unroll 8
-        for (int r = 0; r < m; ++r) acc += row[r];
+            for (int r = 0; r < m; ++r) acc += rnd<DT>(pq[r] * pk[r]);
+          }
+        }
+      if (e < n) {
+        const float sc = rnd<DT>(rnd<DT>(acc) / a.sqrt_r);
+        const float t = sc > a.thr ? 1.0f : (sc < -a.thr ? -1.0f : 0.0f);
+        pos += t > 0.0f;
+        neg += t < 0.0f;
+        st<DT>(a.ternary, a.global ? b * per + e : ((b * nq + qr) * a.H + h0 + hl) * a.W + w, t);
       }
-      __syncthreads();
-    }
-    if (lane < nw) {
-      const float sc = rnd<DT>(rnd<DT>(acc) / a.sqrt_r);
-      const float t = sc > a.thr ? 1.0f : (sc < -a.thr ? -1.0f : 0.0f);
-      pos += t > 0.0f;
-      neg += t < 0.0f;
-      st<DT>(a.ternary, b * n + ew + lane, t);
     }
   }
   // wave sums, then the workgroup's
@@ -366,12 +380,12 @@ __global__ __launch_bounds__(64 * kStNW) void mimo_stats_kernel(MimoStatsArgs a)
     pos += __shfl_xor(pos, o);
     neg += __shfl_xor(neg, o);
   }
-  if (lane == 0) {
-    cnt[0][wv] = pos;
-    cnt[1][wv] = neg;
+  if ((tid & 63) == 0) {
+    cnt[0][tid >> 6] = pos;
+    cnt[1][tid >> 6] = neg;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     int32_t p = 0, q = 0;
     for (int k = 0; k < kStNW; ++k) {
       p += cnt[0][k];
@@ -379,7 +393,7 @@ __global__ __launch_bounds__(64 * kStNW) void mimo_stats_kernel(MimoStatsArgs a)
     }
     a.counts[b * 3 + 0] = p;
     a.counts[b * 3 + 1] = q;
-    a.counts[b * 3 + 2] = n - p - q;
+    a.counts[b * 3 + 2] = static_cast<int32_t>(per * (a.global ? 1 : a.H)) - p - q;
   }
 }
 
@@ -393,13 +407,24 @@ int launch_mimo_stats(const MimoStatsArgs& a, hipStream_t st) {
                "mimo stats: need 1 <= W <= S <= L");
   TESM_REQUIRE(a.R >= 2 && a.R % 2 == 0 && a.H >= 1, kErrInvalidArg, "mimo stats: need an even R");
   TESM_REQUIRE((a.S - a.W + 1) * a.H * a.W <= 0x7fffffff, kErrUnsupported, "mimo stats: too many scores");
-  TESM_REQUIRE(a.H * a.R <= 0x7fffffff && (!a.global || a.S <= 0x7fff), kErrUnsupported,
-               "mimo stats: too many products");
-  constexpr size_t lds = kStNW * kStPitch * sizeof(float);
-  if (a.dt == kBF16)
-    mimo_stats_kernel<kBF16><<<static_cast<unsigned>(a.B), 64 * kStNW, lds, TESM_LOGGED(st, mimo_stats_kernel<kBF16>)>>>(a);
-  else
-    mimo_stats_kernel<kF32><<<static_cast<unsigned>(a.B), 64 * kStNW, lds, TESM_LOGGED(st, mimo_stats_kernel<kF32>)>>>(a);
+  TESM_REQUIRE(!a.global || a.S <= 0x7fff, kErrUnsupported, "mimo stats: too many scores");
+  // whole rows where they fit, in slices of a multiple of 4 values where not; heads side by side as long as they fit
+  // and the threads are not filled
+  const int64_t rows = (a.global ? a.S : a.S - a.W + 1) + a.S, per = a.global ? a.S * a.S : (a.S - a.W + 1) * a.W;
+  const int64_t room = kStLds / 4 / rows;  // floats of a row
+  TESM_REQUIRE(room >= 16, kErrUnsupported, "mimo stats: too many sampled positions");
+  const bool vec = a.R % 4 == 0;
+  const int64_t whole = a.R + (a.R % 8 == 0 ? 4 : vec ? 8 : 1);
+  const int64_t sl = whole <= room ? a.R : (room - 8) / 8 * 8, pitch = whole <= room ? whole : sl + 4;
+  const int64_t hb = a.global || sl < a.R ? 1 : std::min({a.H, room / pitch, (kStNT + per - 1) / per});
+  const size_t lds = static_cast<size_t>(hb * rows * pitch) * sizeof(float);
+  if (a.dt == kBF16) {
+    if (vec) mimo_stats_kernel<kBF16, true><<<static_cast<unsigned>(a.B), kStNT, lds, TESM_LOGGED(st, mimo_stats_kernel<kBF16, true>)>>>(a, static_cast<int>(hb), static_cast<int>(sl), static_cast<int>(pitch));
+    else mimo_stats_kernel<kBF16, false><<<static_cast<unsigned>(a.B), kStNT, lds, TESM_LOGGED(st, mimo_stats_kernel<kBF16, false>)>>>(a, static_cast<int>(hb), static_cast<int>(sl), static_cast<int>(pitch));
+  } else {
+    if (vec) mimo_stats_kernel<kF32, true><<<static_cast<unsigned>(a.B), kStNT, lds, TESM_LOGGED(st, mimo_stats_kernel<kF32, true>)>>>(a, static_cast<int>(hb), static_cast<int>(sl), static_cast<int>(pitch));
+    else mimo_stats_kernel<kF32, false><<<static_cast<unsigned>(a.B), kStNT, lds, TESM_LOGGED(st, mimo_stats_kernel<kF32, false>)>>>(a, static_cast<int>(hb), static_cast<int>(sl), static_cast<int>(pitch));
+  }
   return check_launch("mimo stats");
 }
 

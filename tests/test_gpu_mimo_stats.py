@@ -1,6 +1,6 @@
 """GPU checks of the sampled MIMO entanglement statistics (mimo_stats_kernel) at the edges of its work split, against the
-oracle: scores of less than, exactly and more than one slice of products, fewer scores than a wave takes and score
-counts that leave waves partly filled, for the window and the global branch."""
+oracle: rows staged whole and in slices, one and several heads side by side, more scores of a head than threads, and
+score counts that leave threads idle, for the window and the global branch."""
 import pytest
 import torch
 
@@ -20,6 +20,9 @@ def _gpu():
 # (B, L, H, R, W): W 0 is the global branch (all heads' products in one score: 2 x 180 and 4 x 64)
 CASES = [(1, 64, 4, 256, 64), (1, 20, 2, 300, 8), (2, 3, 1, 6, 2), (1, 70, 3, 64, 16), (2, 40, 5, 34, 9),
          (1, 1, 2, 16, 4), (1, 33, 2, 180, 0), (2, 9, 4, 64, 0)]
+# rows of more than a slice (rank a multiple of 4 or not; the global branch's too), more than 1024 scores of a head,
+# three heads of a group of two
+CASES += [(1, 64, 1, 400, 1), (1, 64, 2, 402, 2), (1, 40, 2, 604, 0), (1, 64, 2, 20, 32), (1, 64, 3, 250, 64)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
