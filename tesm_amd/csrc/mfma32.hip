@@ -528,9 +528,12 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
 //   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU, past short K one: 8192 x 768 x 768 10.6
 //     (128x256: 10.9), 4095 x 1024 x 2816 15.4 (before 21.5), 1000 x 4096 x 4096 21.2 (before 28.3), 666 x 4096 x 11008
-//     41.0 (two K groups on 32x64: 50.6), 200 x 11008 x 4096 16.7 (20.7).  A K loop of at most
-//     three tiles stays on this shape too: such calls are launch-bound (16384 x 256 x 256 5.9, best 5.7; 512 x 96 x
-//     384 5.4, best 4.2), and it keeps short products to one instantiation.
+//     41.0 (two K groups on 32x64: 50.6), 200 x 11008 x 4096 16.7 (20.7).
+//   * a K loop of at most three tiles, where the first loads and the stores are most of the time: 128x256 tiles when
+//     they give every CU two (32768 x 4096 x 64 63.1, 64x128 82.6; f32 97.9, 101.8) or, in bf16, one (4096 x 2048 x 256
+//     8.6, 9.1; f32 11.1, 32x128 10.4); then 32x128, in bf16 as long as 64x128 ones would not give every CU two (800 x
+//     768 x 384 3.8, 64x128 4.9; 4096 x 768 x 384 5.8, 6.3; 8192 x 768 x 384 8.8, 8.5).  One column tile of up to 512
+//     rows stays on 64x128: its call is bound by the launch (512 x 96 x 384 4.7, 32x128 3.8).
 //   * 32x128 tiles when those do, at short K and up to three 64x128 tiles per two CUs (two per CU where those would be
 //     half empty): 512 x 2944 x 768 4.9 (64x128: 5.8), 666 x 2944 x 768 f32 6.1 (7.1); with the quantization
 //     1300 x 2432 x 768 f32 12.4 (11.8), 1600 13.2 (12.8), 4095 x 768 x 768 12.1 (11.6).  Around the line it also
@@ -570,6 +573,10 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
       if (a.Kp > 1024 && 2 * tiles(32, 128) >= 3 * cus) return run_mfma32k<1, 4, 1, 1, 2, 3, EPI>(a, st);
       return run_mfma32k<1, 2, 1, 1, 2, 3, EPI>(a, st);
     }
+  } else if constexpr (EPI == kEpiStore) {
+    if (a.N > 128 && big >= 2 * cus) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
+    if (a.N > 128 && big >= cus && a.out_dt == kBF16) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
+    if ((a.N > 128 || a.M > 512) && (a.out_dt == kF32 || tiles(64, 128) < 2 * cus)) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
   }
   return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
 }

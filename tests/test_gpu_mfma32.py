@@ -78,6 +78,27 @@ def test_tile_walk_exact(M, N, order):
     assert torch.equal(out, _expect(qd @ hip_ops.unpack_weight(packed, K).double().t(), s, c_w, torch.bfloat16))
 
 
+# K loops of one to three tiles on both sides of the rule's lines: (M, N, K, bf16's kernel, float32's)
+SHORT = [(512, 128, 384, "<1,4,2,1,", "<1,4,2,1,"), (513, 128, 384, "<1,4,1,1,", "<1,4,1,1,"),
+         (33, 129, 60, "<1,4,1,1,", "<1,4,1,1,"), (4030, 1025, 130, "<1,4,2,1,", "<1,4,1,1,"),
+         (3960, 1024, 256, "<1,4,1,1,", "<1,4,1,1,"), (4090, 2040, 300, "<2,4,2,2,", "<1,4,1,1,"),
+         (8190, 2048, 384, "<2,4,2,2,", "<2,4,2,2,")]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,bf16,f32", SHORT)
+def test_short_products_exact(M, N, K, bf16, f32, dtype):
+    g = torch.Generator().manual_seed(M + N)
+    x, w = (torch.randn(n, K, generator=g).to(dtype).to(DEV) for n in (M, N))
+    s_w, c_w = hip_ops.absmean_scale(w)
+    packed = hip_ops.pack_weight(w, s_w)
+    (q, s, rs), qd = _codes(x)
+    with hip_ops.launch_log() as log:
+        out = hip_ops.bitlinear(q, s, rs, packed, c_w, N, K, dtype)
+    assert any(k.startswith("mfma32_kernel" + (bf16 if dtype == torch.bfloat16 else f32)) for k in log.kernels), log.kernels
+    assert torch.equal(out, _expect(qd @ hip_ops.unpack_weight(packed, K).double().t(), s, c_w, dtype))
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 200, 2100), (2100, 2050, 1030)])
 def test_bias_and_accumulators(M, N, K):
     """The general epilogue behind a K-group tile and a large one: bias and the accumulator dump."""
