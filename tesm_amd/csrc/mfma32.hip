@@ -532,8 +532,9 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //   * a K loop of at most three tiles, where the first loads and the stores are most of the time: 128x256 tiles when
 //     they give every CU two (32768 x 4096 x 64 63.1, 64x128 82.6; f32 97.9, 101.8) or, in bf16, one (4096 x 2048 x 256
 //     8.6, 9.1; f32 11.1, 32x128 10.4); then 32x128, in bf16 as long as 64x128 ones would not give every CU two (800 x
-//     768 x 384 3.8, 64x128 4.9; 4096 x 768 x 384 5.8, 6.3; 8192 x 768 x 384 8.8, 8.5).  One column tile of up to 512
-//     rows stays on 64x128: its call is bound by the launch (512 x 96 x 384 4.7, 32x128 3.8).
+//     768 x 384 3.8, 64x128 4.9; 4096 x 768 x 384 5.8, 6.3; 8192 x 768 x 384 8.8, 8.5), and for up to 64 rows (32 x
+//     151936 x 384 7.5, 64x128 10.2, 128x256 14.3; 64 rows 11.3, 11.6, 15.7).  One column tile of up to 512 rows
+//     stays on 64x128: its call is bound by the launch (512 x 96 x 384 4.7, 32x128 3.8).
 //   * 32x128 tiles when those do, at short K and up to three 64x128 tiles per two CUs (two per CU where those would be
 //     half empty): 512 x 2944 x 768 4.9 (64x128: 5.8), 666 x 2944 x 768 f32 6.1 (7.1); with the quantization
 //     1300 x 2432 x 768 f32 12.4 (11.8), 1600 13.2 (12.8), 4095 x 768 x 768 12.1 (11.6).  Around the line it also
@@ -574,9 +575,11 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
       return run_mfma32k<1, 2, 1, 1, 2, 3, EPI>(a, st);
     }
   } else if constexpr (EPI == kEpiStore) {
-    if (a.N > 128 && big >= 2 * cus) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
-    if (a.N > 128 && big >= cus && a.out_dt == kBF16) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
-    if ((a.N > 128 || a.M > 512) && (a.out_dt == kF32 || tiles(64, 128) < 2 * cus)) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
+    const bool full = a.M > 64 && a.N > 128;  // (not most of a 128x256 tile for padding)
+    if (full && big >= 2 * cus) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
+    if (full && big >= cus && a.out_dt == kBF16) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
+    if ((a.N > 128 || a.M > 512) && (a.out_dt == kF32 || a.M <= 64 || tiles(64, 128) < 2 * cus))
+      return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
   }
   return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
 }

@@ -82,7 +82,8 @@ def test_tile_walk_exact(M, N, order):
 SHORT = [(512, 128, 384, "<1,4,2,1,", "<1,4,2,1,"), (513, 128, 384, "<1,4,1,1,", "<1,4,1,1,"),
          (33, 129, 60, "<1,4,1,1,", "<1,4,1,1,"), (4030, 1025, 130, "<1,4,2,1,", "<1,4,1,1,"),
          (3960, 1024, 256, "<1,4,1,1,", "<1,4,1,1,"), (4090, 2040, 300, "<2,4,2,2,", "<1,4,1,1,"),
-         (8190, 2048, 384, "<2,4,2,2,", "<2,4,2,2,")]
+         (8190, 2048, 384, "<2,4,2,2,", "<2,4,2,2,"), (64, 140000, 100, "<1,4,1,1,", "<1,4,1,1,"),
+         (20, 140000, 100, "<1,4,1,1,", "<1,4,1,1,"), (65, 140000, 100, "<2,4,2,2,", "<2,4,2,2,")]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
