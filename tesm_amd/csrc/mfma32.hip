@@ -584,16 +584,38 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
   return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
 }
 
-// The output gate (two accumulator sets, so one 128x256 workgroup per CU): 4096 x 4096 x 2 x 2048 115 (before 118);
-// 64x128 tiles of eight waves when they give every CU one: 4095 x 1024 x 2 x 512 16.2 (before 28.6); else 32x64
-// tiles of two waves: 512 x 768 x 2 x 384 7.6 (before 12.0); at long K with CUs left over, eight K groups on 32x32
-// tiles or four on 32x64: 64 x 4096 x 2 x 8192 24.9 (before 51.4), 100 rows 33.9.
+// The output gate.  us, bf16 / f32 (M x N x 2 x K):
+//   * 128x256 tiles: two accumulator sets, so one workgroup per CU and whole rounds of the CUs; taken where the rounds
+//     are nearly full, the fuller the shorter the K loop: 4096 x 4096 x 2 x 2048 102 / 149 (eight-wave 64x128 115 / 172),
+//     7000 x 1024 x 2 x 4096 74.8 / 98.1 (93.4 / 120), 4095 x 2048 x 2 x 1024 40.5 / 63.2 (41.8 / 69.9); not 7000 x 2432
+//     x 2 x 1280 (2.15 rounds) 116 / 186 (98.2 / 162), 3000 x 4096 x 2 x 2048 (1.5) 95.5 / 141 (86.8 / 126), 8300 x 2050
+//     x 2 x 300 114 / 136 (81.5 / 102).  At two K tiles they stand from two rounds on, though 64x128 ones would be
+//     faster (4095 x 4096 x 2 x 256 58.1 / 104, 49.0 / 104).
+//   * 64x128 tiles when they give every CU one: eight waves in bf16 (4095 x 1024 x 2 x 512 16.2, one-group form 28.6); in
+//     f32 32x64 tiles just past two per CU (2048 x 2432 x 2 x 1280 53.3, 57.4 with 64x128) and four waves beyond (7000 x
+//     2432 x 2 x 1280 155, eight 162; 8300 x 2048 x 2 x 1024 142, 148); at long K 32x64 up to three per two CUs (2048 x
+//     1024 x 2 x 4096 34.9 / 41.5, 40.9 / 47.0).
+//   * else 32x64 tiles of two waves: 512 x 768 x 2 x 384 7.6 (before 12.0); at long K with CUs left over, eight K groups on
+//     32x32 tiles or four on 32x64: 64 x 4096 x 2 x 8192 24.9 (before 51.4), 100 rows 33.9.
 int dispatch_gate32(const LinearArgs& a, hipStream_t st) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
-  const int64_t cus = std::max(device_limits().cus, 1), big = tiles(128, 256);
-  if (big >= 8 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 2>(a, st);
-  if (big >= 2 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 0>(a, st);
-  if (tiles(64, 128) >= cus) return run_mfma32<2, 4, 1, 1, kEpiOutputGate, 0>(a, st);
+  const int64_t cus = std::max(device_limits().cus, 1), big = tiles(128, 256), mid = tiles(64, 128);
+  const int64_t rounds = (big + cus - 1) / cus, fill = 100 * big / (rounds * cus);  // percent of the rounds' CUs
+  const bool f32 = a.out_dt == kF32;
+  const bool wide = a.Kp < 512      ? a.Kp == 256 && big >= 2 * cus
+                    : a.Kp <= 1024  ? fill >= 95 && (f32 || rounds > 1)
+                    : a.Kp < 2048   ? fill >= (a.Kp < 1536 ? 90 : 85)
+                    : a.Kp < 4096   ? fill >= (f32 ? 85 : 75) + (rounds > 1 ? 5 : 0)
+                                    : fill >= 75;
+  if (wide && big >= 8 * cus) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 2>(a, st);
+  if (wide) return run_mfma32<2, 4, 2, 2, kEpiOutputGate, 0>(a, st);
+  if (mid >= cus && !(a.Kp >= 4096 && 2 * mid <= 3 * cus)) {
+    if (f32 && mid > 2 * cus) {
+      if (4 * mid <= 11 * cus) return run_mfma32<1, 2, 1, 1, kEpiOutputGate, 0>(a, st);
+      if (a.Kp > 256) return run_mfma32<1, 4, 2, 1, kEpiOutputGate, 0>(a, st);
+    }
+    return run_mfma32<2, 4, 1, 1, kEpiOutputGate, 0>(a, st);
+  }
   if (a.Kp >= 4096 && tiles(32, 64) < cus) return run_mfma32k<1, 1, 1, 1, 8, 3, kEpiOutputGate>(a, st);
   if (a.Kp >= 4096 && tiles(32, 64) < 2 * cus) return run_mfma32k<1, 2, 1, 1, 4, 3, kEpiOutputGate>(a, st);
   return run_mfma32<1, 2, 1, 1, kEpiOutputGate, 0>(a, st);

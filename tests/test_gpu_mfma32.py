@@ -171,3 +171,20 @@ def test_output_gate_products(M, N, K, kernel, dtype):
     bound = eps * (2 * gs.float().abs() + (local.float() + gs.float()).abs() + want.float().abs()) + 1e-6
     assert bool(((y.float() - want.float()).abs() <= bound).all())
     assert float((y != want).float().mean()) <= (0.5 if dtype == torch.float32 else 0.02)
+
+
+# both sides of the rule's lines: (M, N, K, bf16's kernel, float32's) - rounds of 128x256 tiles nearly full or not, by K;
+# float32's 64x128 tiles just past two per CU and beyond; long K with up to three 64x128 tiles per two CUs
+GATE_LINES = [(1500, 4080, 2050, "<2,4,2,2,1,", "<1,4,2,1,1,"), (2047, 4000, 2050, "<2,4,2,2,1,", "<2,4,2,2,1,"),
+              (2950, 4060, 2050, "<2,4,1,1,1,", "<1,4,2,1,1,"), (3000, 2430, 1280, "<2,4,2,2,1,", "<2,4,2,2,1,"),
+              (4095, 2430, 1280, "<2,4,1,1,1,", "<1,4,2,1,1,"), (2048, 4000, 600, "<2,4,1,1,1,", "<2,4,2,2,1,"), (4095, 4000, 600, "<2,4,2,2,1,", "<2,4,2,2,1,"),
+              (1500, 4080, 4100, "<2,4,2,2,1,", "<2,4,2,2,1,"), (2900, 2430, 1540, "<2,4,2,2,1,", "<2,4,2,2,1,"),
+              (2048, 2430, 600, "<2,4,1,1,1,", "<1,2,1,1,1,"), (8190, 2050, 300, "<2,4,1,1,1,", "<1,4,2,1,1,"),
+              (2900, 1024, 4100, "<1,2,1,1,1,", "<1,2,1,1,1,"), (3200, 1024, 4100, "<2,4,1,1,1,", "<2,4,1,1,1,")]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,bf16,f32", GATE_LINES)
+def test_output_gate_lines(M, N, K, bf16, f32, dtype):
+    test_output_gate_products(M, N, K, f"mfma32_kernel{bf16 if dtype == torch.bfloat16 else f32}", dtype)
+
