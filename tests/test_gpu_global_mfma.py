@@ -47,3 +47,28 @@ def test_one_pass_global_matches_oracle(shape):
     names = [n.split("<")[0] for n in log.kernels]
     assert ("global_mfma_kernel" in names) == one_pass and ("global_scores_kernel" in names) != one_pass, names
     assert torch.equal(y0, y1)
+
+
+def test_longest_one_pass_against_the_general_kernels():
+    """Positions of which many round to one bf16 value: the longest sequence the one-pass kernel takes against the same
+    positions of one that is longer by a token, which takes the general kernels (the layer is causal).  The two add a
+    score's products in another order, so a decision next to the threshold may differ, which moves its row's average by
+    less than two parts in its decision count; a wrong bias entry would show as leaving the bias out does."""
+    L, kw = 32768, dict(d_model=32, d_state=16, ent_rank=16, max_seq_len=33000)
+    m = _siso(TESM_SISO, 3, torch.bfloat16, **kw).to(DEV)
+    u = torch.randn(1, L + 1, 32, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).to(DEV)
+    with torch.no_grad():
+        with hip_ops.launch_log() as log:
+            y = m(u[:, :L].contiguous())[0].float()
+        with hip_ops.launch_log() as log1:
+            long = m(u)[0][:, :L].float()
+        m.global_rel_pos_scale.zero_()
+        m.global_rel_pos_bias.zero_()
+        plain = m(u)[0][:, :L].float()
+    names, names1 = ([n.split("<")[0] for n in lg.kernels] for lg in (log, log1))
+    assert "global_mfma_kernel" in names and "global_mfma_kernel" not in names1 and "global_scores_kernel" in names1
+    for part in (slice(0, 4096), slice(4096, 16384), slice(16384, L)):  # (by how far positions round)
+        d = float((y - long)[:, part].norm() / long[:, part].norm())
+        without = float((plain - long)[:, part].norm() / long[:, part].norm())
+        print(f"positions {part.start}-{part.stop}: rel. L2 {d:.2e}, without the bias {without:.2e}")
+        assert d <= 2.0 ** -8 and d <= without / 10, (part, d, without)
