@@ -364,6 +364,9 @@ SisoPlan plan_siso(const tesm_hip_siso_layer& p, void* base) {
   s.g_qr = s.g_kr = nullptr;
   if (!s.fuse_ent) {
     if (global) {
+      // The one-pass kernel leaves decisions only for taps and uses neither the counts nor the transposed states (nor,
+      // where it quantizes, e_tanh and c_mix).  They are carved for every global layer all the same: which path a call
+      // takes also follows from the alignment and stride of its states, which a size query need not know.
       s.g_tern = c.take<int8_t>(p.B * p.L * global_tern_pitch(p.L));
       s.g_count = c.take<int32_t>(p.B * p.L * 4);
       s.g_table = c.take<float>(2 * p.L * 4);

@@ -17,8 +17,9 @@
 // So the window weights and the float tanh(E) / C never reach memory, and 16 positions x 2048 channels keep
 // 16 waves per CU busy.
 //
-// 4096 positions, D 2048, rank 256, window 64: 35 us, where the scores kernel (114), the mix kernel (309) and the
-// quantization launch (10) took 433; the whole layer (d_model 4096) 927 -> 526 us.
+// 4096 positions, D 2048, rank 256, window 64: 37 us in the layer (33 at best), where the scores kernel (114), the mix
+// kernel (309) and the quantization launch (10) took 433; by this alone the whole layer (d_model 4096) went from 927 to
+// 526 us.
 // Bound by the staging of the states (each CU reads (16 + W - 1) / 16 of its share of them: 5x at window 64,
 // from its XCD's L2) and by the barriers between the blocks; the contractions are a few microseconds.
 #include "entangle.h"

@@ -9,20 +9,22 @@
 // 8*(r/4) + 4*(L/32) + r%4 and activation row L%32.
 //
 // Pipeline.  K tiles go straight from memory to LDS (16-byte buffer loads with the LDS destination, no staging
-// registers) into NS stages.  A fragment's LDS reads are issued one k-step ahead of its MFMAs, across the K tile boundary too: the
-// one barrier of a K tile stands in its middle, where a wave (a) knows its loads of the next tile landed
-// (vmcnt), (b) meets the others, so the next tile may be read from the last k-step on and the previous tile's
+// registers) into NS stages.  A fragment's LDS reads are issued one k-step ahead of its MFMAs, across the K tile
+// boundary too: the one barrier of a K tile stands in its middle, where a wave (a) knows its loads of the next tile
+// landed (vmcnt), (b) meets the others, so the next tile may be read from the last k-step on and the previous tile's
 // stage may be refilled.  With the wait at a tile's start instead, and two stages, every tile paid an LDS round
-// trip and the slowest wave's load (2048 x 4096 x 4096: 37.6 -> 35 us; 4095 x 3744 x 1024: 28.3 -> 21.2).
+// trip and the slowest wave's load (2048 x 4096 x 4096 37.7 us, now 36.8; 4095 x 3744 x 1024 27.5, now 23.8).
 //
-// What bounds it: large products run at 2.1-2.3 POP/s, where the chip's power limit lies for these operands (the
-// library int8 product reaches 2.25 on random codes; the same kernel on all-zero codes is 1.3 times faster; tiles
-// from 128x128 to 256x256, 64x64 to 128x64 per wave and 2 to 4 stages all end within 10 % of each other):
-// 8192 x 34816 x 4096 1055 us, 4096 x 14848 x 4096 231 (the two-stage loop 1111 and 262).  Small
-// ones are bound by the latency of the first tiles and by idle CUs, hence the K groups: KS groups of waves
-// in one workgroup take K tiles g, g + KS, ... into stages of their own, and their exact int32 sums are added in
-// LDS, so a 32 x 64 tile with a quarter of the K loop per group replaces 64 x 128 tiles on a fifth of the CUs
-// (512 x 768 x 3072: 13.7 -> 5.7 us; 512 x 768 x 768: 6.1 -> 4.0).
+// What bounds it: products of many rounds of tiles run at 2.1-2.3 POP/s, where the chip's power limit lies for these
+// operands (the library int8 product reaches 2.25 on random codes; the same kernel on all-zero codes is 1.4 times
+// faster, 167 against 233 us at 4096 x 14848 x 4096; tiles from 128x128 to 256x256, 64x64 to 128x64 per wave and 2 to
+// 4 stages all end within 10 % of each other): 8192 x 34816 x 4096 1025 us, 4096 x 14848 x 4096 233 (the two-stage
+// loop 1099 and 265).  A round or two lose part of that to the first K tiles' latency, the stores and the rounds' ends
+// (2048 x 4096 x 4096 1.87 POP/s, 4095 x 1024 x 2816 1.36, 8192 x 2432 x 768 1.22), the output gate to its one
+// workgroup per CU (4096 x 4096 x 2 x 2048 1.08).  Small ones are bound by the latency of the first tiles and by idle
+// CUs, hence the K groups: KS groups of waves in one workgroup take K tiles g, g + KS, ... into stages of their own,
+// and their exact int32 sums are added in LDS, so a 32 x 64 tile with a quarter of the K loop per group replaces
+// 64 x 128 tiles on a fifth of the CUs (512 x 768 x 3072 11.8 -> 6.0 us; 512 x 768 x 768 5.5 -> 4.3).
 //
 // Two-product epilogues: SwiGLU's products share the activations, so one K loop reads them once against both
 // weight tiles (it ran one K loop after the other: 4095 x 2816 x 1024 53.8 us); the output gate's products follow
@@ -42,7 +44,7 @@ namespace {
 // Loads to LDS through a buffer resource rather than global_load_lds: the compiler counts that instruction as one
 // that may also touch LDS out of order, and waits for every outstanding LDS read (lgkmcnt(0)) wherever one is
 // needed while such a load is in flight, which undoes the fragment prefetch (4096 x 14848 x 4096: 242 us, 231 with
-// buffer loads; 8192 x 34816 x 4096: 1108, 1056).
+// buffer loads; 8192 x 34816 x 4096, then walked by fours: 1108, 1056).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, 0xffffffffu, 0x00027000);
 }
@@ -458,7 +460,8 @@ __global__ __launch_bounds__(WM* WN * 64, WM * WN >= 8 && EPI != kEpiOutputGate 
   mfma32_tile<WM, WN, TM, TN, 1, 3, EPI, OUT_DT>(a, tm * T::BM, tn * T::BN, smem);
 }
 
-// KS groups of WM x WN waves per tile, each with K tiles of its own.
+// KS groups of WM x WN waves per tile, each with K tiles of its own.  (The output gate's eight groups keep 64 of their
+// registers in scratch memory, 244-264 bytes a lane: two products' loads in flight beside two accumulator sets.)
 template <int WM, int WN, int TM, int TN, int KS, int NS, int EPI, int OUT_DT>
 __global__ __launch_bounds__(WM* WN* KS * 64) void mfma32k_kernel(LinearArgs a) {
   using T = Tile32<WM, WN, TM, TN, KS, NS, EPI, OUT_DT>;

@@ -44,8 +44,9 @@ constexpr int kMixLD = 4;            // float4 state loads per thread per block:
 // and walks the window keeping the 2 state rows it needs in registers, so every 8 multiply-adds cost
 // one state and one weight read.  Sums run over w in increasing order.  WT: 64 for mix64, else 0.
 //
-// W = 64 with whole 16-byte rows (the largest window, and the large preset's) takes mix64 below: here a thread reads 24
-// bytes of LDS per 8 multiply-adds, three bytes each where two keep up with the vector units.
+// W = 64 with whole 16-byte rows (the largest window, and the large preset's) takes mix64 below: here a thread reads
+// 24 bytes of LDS per 8 multiply-adds, three bytes each where two keep up with the vector units.  Its loop would serve
+// any window that is a multiple of 8; for smaller ones it is neither instantiated nor measured.
 constexpr int kM64C = 128;                           // channels per block
 constexpr int kM64Rows = kMixTP + 64;                // state rows per block (the last one is not used)
 constexpr int kM64CB = 4;                            // channel blocks per workgroup
@@ -56,9 +57,10 @@ static_assert(2 * kM64Lds <= 160 * 1024, "two workgroups per CU");
 // registers and move up by one, so a slot's 32 multiply-adds cost one state and two weight reads of 16 bytes (half the
 // general form's LDS traffic), and the last slot's rows are the positions' own states.  States go straight to LDS; two
 // workgroups per CU overlap one's loads with the other's sums.  Each sum runs over the window in increasing order, as
-// in the general form (same bits).  32768 positions x 8192 channels: 886 us, before 1017, with the next block's states
-// held in registers instead 951; the vector units alone need 440 us for these 17 G multiply-adds, and weights as scalar
-// operands (16 positions x 1 channel per lane) took 1560, the scalar cache being too small for 20 waves' weights.
+// in the general form (same bits).  32768 positions x 8192 channels: 886 us (925 in the layer on another box), before
+// 1017, with the next block's states held in registers instead 951; the vector units alone need 440 us for these 17 G
+// multiply-adds, and weights as scalar operands (16 positions x 1 channel per lane) took 1560, the scalar cache being
+// too small for 20 waves' weights.
 template <int DT>
 __device__ __forceinline__ void mix64(const MimoMixArgs& a, float* lds) {
   float* srow = lds;                         // [kM64Rows][kM64C]
@@ -287,16 +289,16 @@ __global__ __launch_bounds__(256) void mimo_final_kernel(const float* S, const f
   if (last) last[i] = v;
 }
 
-// One workgroup of 16 waves per batch row.  The RoPE'd q and k rows of the sampled positions are staged in LDS once per
-// group of hb heads (as many as fill the threads and fit), then a thread forms one score: its products in natural
+// One workgroup of 16 waves per batch row.  The RoPE'd q and k rows of the sampled positions are staged in LDS once
+// per group of hb heads (as many as fill the threads and fit), then a thread forms one score: its products in natural
 // (h, r) order, each rounded, from two rows.  Rows longer than a slice of sl values are staged slice by slice, and the
 // global branch's scores run over all heads.  VEC: rows of whole 16-byte groups; the pitch (R + 4 or R + 1) spreads
-// the lanes' key rows over all banks.
-// Bound by the staging's loads and the chain of additions.  us for 1 x 64 positions (before: one thread per score over
-// its own rows of q and k, bf16 and f32; in brackets a wave's lanes forming a score's products side by side): 4 heads of
-// rank 256, window 64 37 and 33 (97, 39 [49, 45]); rank 64, window 32 30 and 26 (398, 150 [239, 219]); 2 heads of rank
-// 16, window 8 5 (17, 10 [55, 50]); global, 4 heads of rank 32 10 and 11 (190, 71 [76, 68]).  A rank whose rows do not
-// fit whole rotates each pair twice: window 1, rank 400, the layer 142, 131 in the bracketed form.
+// the lanes' key rows over all banks. Bound by the staging's loads and the chain of additions.  us for 1 x 64
+// positions (before: one thread per score over its own rows of q and k, bf16 and f32; in brackets a wave's lanes
+// forming a score's products side by side): 4 heads of rank 256, window 64 37 and 33 (97, 39 [49, 45]); rank 64,
+// window 32 30 and 26 (398, 150 [239, 219]); 2 heads of rank 16, window 8 5 (17, 10 [55, 50]); global, 4 heads of rank
+// 32 10 and 11 (190, 71 [76, 68]).  A rank whose rows do not fit whole rotates each pair twice: window 1, rank 400,
+// the layer 142, 131 in the bracketed form.
 constexpr int kStNT = 1024;
 constexpr int kStNW = kStNT / 64;
 constexpr int kStLds = 144 * 1024;
