@@ -6,6 +6,7 @@
 //   states_r = S * mimo_x[:, r]^2,  sum_r entangled_r * mimo_o[:, r] = E * c,  c = sum_r mimo_x_r^2 mimo_o_r,
 // with S the scan of write * tanh(sv) and E its entangled state.  Here the one scan and the one mix
 // run on S and the merge is a per-channel factor (float32 throughout, as the reference's rank tensors).
+#include "linear_dev.h"
 #include "mimo.h"
 
 namespace tesm {
@@ -458,9 +459,15 @@ int launch_mimo_mix(const MimoMixArgs& a, hipStream_t st) {
   const bool vec = a.D % 4 == 0 && (a.H * a.D) % 4 == 0 && reinterpret_cast<uintptr_t>(a.S) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(a.te) % (a.dt == kBF16 ? 8 : 16) == 0 &&
                    reinterpret_cast<uintptr_t>(a.cc) % (a.dt == kBF16 ? 8 : 16) == 0;
-  const bool m64 = vec && a.W == 64 && a.D < (int64_t(1) << 30);
-  const int64_t nb64 = (a.D + kM64C - 1) / kM64C;
+  // mix64's blocks are 128 channels, the general form's 32, so a last block that is mostly padding costs more there than
+  // the form gains.  The layer in us, mix64 and (general): 8 x 800 positions, 8 heads, f32 D 64 140 (133), 96 169 (164),
+  // 112 178 (181), 192 246 (239), 256 279 (282); 1 x 4000, 4 heads, whose workgroups are all resident at once, D 32 81.5
+  // (80.0), 64 84.8 (85.9), 132 109 (107), 160 107 (108), 192 112 (115).
+  const int64_t nb64 = (a.D + kM64C - 1) / kM64C, last = a.D - (nb64 - 1) * kM64C;
   const dim3 g64(static_cast<unsigned>((nb64 + kM64CB - 1) / kM64CB), grid.y, grid.z);
+  const bool resident = static_cast<int64_t>(g64.x) * g64.y * g64.z <= 2 * std::max(device_limits().cus, 1);
+  const bool full = 6 * (kM64C - last) <= nb64 * kM64C || (resident && last >= (nb64 == 1 ? kM64C / 2 : kM64C / 4));
+  const bool m64 = vec && a.W == 64 && a.D < (int64_t(1) << 30) && full;
   if (a.dt == kBF16) {
     if (m64) mimo_mix_kernel<kBF16, true, 64><<<g64, 256, kM64Lds, TESM_LOGGED(st, mimo_mix_kernel<kBF16, true, 64>)>>>(a);
     else if (vec) mimo_mix_kernel<kBF16, true, 0><<<grid, 256, lds, TESM_LOGGED(st, mimo_mix_kernel<kBF16, true, 0>)>>>(a);
