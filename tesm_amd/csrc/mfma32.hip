@@ -527,6 +527,9 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //     33.5, f32 34.2, 35.8; the less of the fifth tile is filled the more: over 27 sizes of K 1536-4096 from 4.5 %
 //     faster to 0.7 slower, 1.3 in the mean, none at 640 rows).  Other counts gain nothing to speak of: six or seven
 //     3 % faster to 3 slower, 0.4 in the mean; one to four and 8 to 21 within 1.6 %, with 9, 13, 17 and 21 among them.
+//     Up to K 2048 only when 64x128 tiles would go past three per CU: below that the rows or columns they need not fill
+//     up count for more (402 x 12544 x 1100 13.2, 64x128 12.4, f32 14.6, 13.7; x 2048 17.9, 17.0, f32 19.7, 18.0; with
+//     outputs not in whole 16-byte rows 402 x 12442 x 1100 18.8, 15.5; past the line 700 x 8960 x 3000 24.1, 28.6).
 //   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
 //     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
 //   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU, past short K one: 8192 x 768 x 768 10.6
@@ -566,11 +569,11 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
   }
   if (a.Kp > 3 * kKTile) {
     const bool most = a.Kp > 4096 ? 8 * big >= 5 * cus : 4 * big >= 3 * cus;
-    const bool wide = big >= cus || (most && a.Kp > 1024 && a.M > 64);
+    const int64_t mid = tiles(64, 128);
+    const bool wide = big >= cus || (most && a.Kp > 1024 && a.M > 64 && (a.Kp > 2048 || mid >= 3 * cus));
     const bool five = a.M > 512 && a.M <= 640;  // M tiles: by fours the fifth shares no weights in its XCD
     if (big >= 2 * cus || (wide && (a.Kp > 4096 || ((big > cus || five) && a.Kp > 1024)))) return run_mfma32<2, 4, 2, 2, EPI, 2>(a, st);
     if (wide) return run_mfma32<2, 4, 2, 2, EPI, 0>(a, st);
-    const int64_t mid = tiles(64, 128);
     if (2 * mid < (a.M <= 32 ? 4 : 3) * cus && a.Kp <= 1024 && tiles(32, 128) >= cus) return run_mfma32<1, 4, 1, 1, EPI, 0>(a, st);
     if (mid < cus || a.M <= 32) {
       if (a.Kp >= 2048 && tiles(32, 64) < 2 * cus) return run_mfma32k<1, 2, 1, 1, 4, 3, EPI>(a, st);

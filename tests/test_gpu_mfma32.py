@@ -84,6 +84,9 @@ SHORT = [(512, 128, 384, "<1,4,2,1,", "<1,4,2,1,"), (513, 128, 384, "<1,4,1,1,",
          (3960, 1024, 256, "<1,4,1,1,", "<1,4,1,1,"), (4090, 2040, 300, "<2,4,2,2,", "<1,4,1,1,"),
          (8190, 2048, 384, "<2,4,2,2,", "<2,4,2,2,"), (64, 140000, 100, "<1,4,1,1,", "<1,4,1,1,"),
          (20, 140000, 100, "<1,4,1,1,", "<1,4,1,1,"), (65, 140000, 100, "<2,4,2,2,", "<2,4,2,2,")]
+# under one 128x256 tile per CU, K to 2048 and past it: three 64x128 tiles per CU and fewer
+SHORT += [(402, 12544, 1100, "<1,4,2,1,", "<1,4,2,1,"), (402, 12442, 2048, "<1,4,2,1,", "<1,4,2,1,"),
+          (449, 12288, 1100, "<2,4,2,2,", "<2,4,2,2,"), (402, 12442, 2049, "<2,4,2,2,", "<2,4,2,2,")]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
