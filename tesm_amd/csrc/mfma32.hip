@@ -233,12 +233,11 @@ __device__ __forceinline__ void mfma32_loop(const LinearArgs& a, int64_t m0, int
 // Orders a wave's own LDS accesses (its slab is private: no other wave waits for it).
 __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
 
-// A wave's 32 rows x TN column tiles, four consecutive columns per lane and group: written to its LDS slab and
-// read back as 16-byte row-contiguous chunks, so a store instruction covers whole row segments (128 bytes for two
-// bf16 tiles).  v(j, g, out) gives the four values of tile j's group g (columns 8g + 4*(lane/32) ..).
+// A wave's 32 rows x TN column tiles to its LDS slab, four consecutive columns per lane and group.  v(j, g, out)
+// gives the four values of tile j's group g (columns 8g + 4*(lane/32) ..).
 template <int OUT_DT, int TN, class F>
-__device__ __forceinline__ void store_tiles32(const LinearArgs& a, char* slab, int64_t mb, int64_t nb, F v) {
-  constexpr int ES = OUT_DT == kBF16 ? 2 : 4, RB = TN * 32 * ES, PITCH = RB + 16, CPR = RB / 16, VPC = 16 / ES;
+__device__ __forceinline__ void fill_slab32(char* slab, F v) {
+  constexpr int ES = OUT_DT == kBF16 ? 2 : 4, PITCH = TN * 32 * ES + 16;
   const int lane = threadIdx.x & 63;
   wave_lds_fence();  // the slab's previous contents are consumed
 #pragma unroll
@@ -254,6 +253,13 @@ __device__ __forceinline__ void store_tiles32(const LinearArgs& a, char* slab, i
         *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
     }
   wave_lds_fence();
+}
+
+// The slab's rows as 16-byte chunks, so a store instruction covers whole row segments (128 bytes for two bf16 tiles).
+template <int OUT_DT, int TN>
+__device__ __forceinline__ void store_tiles32(const LinearArgs& a, const char* slab, int64_t mb, int64_t nb) {
+  constexpr int ES = OUT_DT == kBF16 ? 2 : 4, RB = TN * 32 * ES, PITCH = RB + 16, CPR = RB / 16, VPC = 16 / ES;
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int it = 0; it < 32 * CPR / 64; ++it) {
     const int idx = it * 64 + lane, row = idx / CPR, ch = idx % CPR;
@@ -272,6 +278,34 @@ __device__ __forceinline__ void store_tiles32(const LinearArgs& a, char* slab, i
           reinterpret_cast<uint32_t*>(dst)[e] = wd[e];
       }
     }
+  }
+}
+
+// The slab's rows to outputs that are not in whole 16-byte rows: U (an element, or a bf16 pair where rows start on
+// four bytes) per lane, a store instruction covering whole rows again.  From the accumulators, four columns of 32 rows
+// per instruction, the stores touched a memory line per lane and cost as much as the product (us, M x N x K: 4093 x 4093
+// x 512 31.6 -> 20.3, f32 4093 x 3965 x 512 57.0 -> 19.3; 964 x 7932 x 1100 20.7 -> 16.6, f32 964 x 7835 x 4096 54.4 ->
+// 35.9; geometric mean of 120 sizes 1.48).
+template <class U, int ES, int RB>
+__device__ __forceinline__ void store_rows32(const LinearArgs& a, const char* slab, int64_t mb, int64_t nb) {
+  constexpr int S = sizeof(U), UPR = RB / S, RPI = 64 / UPR, PITCH = RB + 16;  // units per row, rows per instruction
+  static_assert(UPR <= 64 && 64 % UPR == 0);
+  const int lane = threadIdx.x & 63, u = lane % UPR;
+  const int64_t n = nb + u * (S / ES), rows = a.M - mb;
+  if (n >= a.N) return;
+  const bool whole = n + S / ES <= a.N;  // (else the first element of a pair)
+  const char* src = slab + (lane / UPR) * PITCH + u * S;
+  char* dst = static_cast<char*>(a.out) + ((mb + lane / UPR) * a.ldo + n) * ES;
+#pragma unroll 8
+  for (int row = lane / UPR; row < 32; row += RPI) {
+    if (row >= rows) break;
+    const U d = *reinterpret_cast<const U*>(src);
+    if (whole)
+      *reinterpret_cast<U*>(dst) = d;
+    else
+      *reinterpret_cast<uint16_t*>(dst) = static_cast<uint16_t>(d);
+    src += RPI * PITCH;
+    dst += RPI * a.ldo * ES;
   }
 }
 
@@ -310,7 +344,7 @@ __device__ __forceinline__ void epilogue32(const LinearArgs& a, const v16i (&acc
       int kind[TN];
 #pragma unroll
       for (int j = 0; j < TN; ++j) kind[j] = EPI == kEpiGates ? gate_region(a, nb + 32 * j) : 0;
-      store_tiles32<OUT_DT, TN>(a, slab, m0 + (wm * TM + i) * 32, nb, [&](int j, int g, float (&v)[4]) {
+      fill_slab32<OUT_DT, TN>(slab, [&](int j, int g, float (&v)[4]) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = (static_cast<float>(acc[0][i][j][4 * g + r] - rs0[i]) * inv0[i]) * cws;
         if constexpr (EPI == kEpiGates) gate_act4<OUT_DT>(a, kind[j], nb + 32 * j + 8 * g + 4 * (lane >> 5), v);
@@ -322,13 +356,31 @@ __device__ __forceinline__ void epilogue32(const LinearArgs& a, const v16i (&acc
           }
         }
       });
+      store_tiles32<OUT_DT, TN>(a, slab, m0 + (wm * TM + i) * 32, nb);
     }
     return;
   }
-  // General form: per-row weight scales, bias, accumulator dump, unaligned outputs, and the output gate.  The
-  // gate's inputs of one 32 x 32 tile (four groups of four columns per lane) are requested together in
-  // straight-line code (indices clamped into range, raw bits) before any is used, so the tile waits for
-  // memory once instead of once per group.
+  if (EPI == kEpiStore && tensor && !a.bias) {  // unaligned: apart, so that the aligned stores stay as short
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int64_t mb = m0 + (wm * TM + i) * 32, nb = n0 + wn * TN * 32;
+      fill_slab32<OUT_DT, TN>(slab, [&](int j, int g, float (&v)[4]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = (static_cast<float>(acc[0][i][j][4 * g + r] - rs0[i]) * inv0[i]) * cws;
+      });
+      if constexpr (OUT_DT == kBF16)
+        if ((reinterpret_cast<uintptr_t>(a.out) | static_cast<uintptr_t>(a.ldo * es)) % 4 != 0) {
+          store_rows32<uint16_t, es, TN * 32 * es>(a, slab, mb, nb);
+          continue;
+        }
+      store_rows32<uint32_t, es, TN * 32 * es>(a, slab, mb, nb);
+    }
+    return;
+  }
+  // General form: per-row weight scales, bias, accumulator dump, unaligned outputs of SwiGLU and the gates, and the
+  // output gate.  The gate's inputs of one 32 x 32 tile (four groups of four columns per lane) are requested together
+  // in straight-line code (indices clamped into range, raw bits) before any is used, so the tile waits for memory once
+  // instead of once per group.
   const bool vout = vec4_ok<OUT_DT>(a.out, a.ldo);
   const bool vin = EPI == kEpiOutputGate && vec4_ok<OUT_DT>(a.local, a.ld_local) &&
                    vec4_ok<OUT_DT>(a.gate, a.ld_gate) && a.N % 4 == 0;
@@ -528,8 +580,8 @@ int run_mfma32k(const LinearArgs& a, hipStream_t st) {
 //     faster to 0.7 slower, 1.3 in the mean, none at 640 rows).  Other counts gain nothing to speak of: six or seven
 //     3 % faster to 3 slower, 0.4 in the mean; one to four and 8 to 21 within 1.6 %, with 9, 13, 17 and 21 among them.
 //     Up to K 2048 only when 64x128 tiles would go past three per CU: below that the rows or columns they need not fill
-//     up count for more (402 x 12544 x 1100 13.2, 64x128 12.4, f32 14.6, 13.7; x 2048 17.9, 17.0, f32 19.7, 18.0; with
-//     outputs not in whole 16-byte rows 402 x 12442 x 1100 18.8, 15.5; past the line 700 x 8960 x 3000 24.1, 28.6).
+//     up count for more (402 x 12544 x 1100 13.2, 64x128 12.4, f32 14.6, 13.7; x 2048 17.9, 17.0, f32 19.7, 18.0; past
+//     the line 700 x 8960 x 1100 13.5, 14.8).
 //   * with short K and a narrow remainder past two tiles per CU (the SISO in_proj, 8192 x 2432 x 768), the split
 //     kernel: 23.5 against 26.1 for 128x256 tiles throughout.
 //   * 64x128 tiles (4 waves of 64x32) when they give two workgroups per CU, past short K one: 8192 x 768 x 768 10.6

@@ -103,6 +103,25 @@ def test_short_products_exact(M, N, K, bf16, f32, dtype):
     assert torch.equal(out, _expect(qd @ hip_ops.unpack_weight(packed, K).double().t(), s, c_w, dtype))
 
 
+# outputs at each offset from 16 bytes, in rows of odd and even lengths: one per tile shape, K groups, the split kernel
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(97, 70, 640), (33, 65, 128), (600, 1001, 60), (1025, 8199, 513), (8190, 2402, 520)])
+def test_unaligned_outputs(M, N, K, dtype):
+    g = torch.Generator().manual_seed(M + K)
+    x, w = (torch.randn(n, K, generator=g).to(dtype).to(DEV) for n in (M, N))
+    s_w, c_w = hip_ops.absmean_scale(w)
+    packed = hip_ops.pack_weight(w, s_w)
+    (q, s, rs), qd = _codes(x)
+    want = _expect(qd @ hip_ops.unpack_weight(packed, K).double().t(), s, c_w, dtype)
+    for ld in (N + 8 - N % 8 + 8, N + 9 - N % 8 + 8, N + 10 - N % 8 + 8):
+        for off in (0, 1, 2, 3, 5):
+            wide = torch.full((M + 2, ld), 7.0, dtype=dtype, device=DEV)
+            hip_ops.bitlinear(q, s, rs, packed, c_w, N, K, dtype, out=wide[1:M + 1, off:off + N])
+            assert torch.equal(wide[1:M + 1, off:off + N], want), (ld, off)
+            wide[1:M + 1, off:off + N] = 7.0
+            assert bool((wide == 7.0).all()), (ld, off)
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 200, 2100), (2100, 2050, 1030)])
 def test_bias_and_accumulators(M, N, K):
     """The general epilogue behind a K-group tile and a large one: bias and the accumulator dump."""
