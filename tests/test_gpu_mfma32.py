@@ -210,3 +210,28 @@ GATE_LINES = [(1500, 4080, 2050, "<2,4,2,2,1,", "<1,4,2,1,1,"), (2047, 4000, 205
 def test_output_gate_lines(M, N, K, bf16, f32, dtype):
     test_output_gate_products(M, N, K, f"mfma32_kernel{bf16 if dtype == torch.bfloat16 else f32}", dtype)
 
+
+
+# rows of whole 16-byte chunks take the inputs and outputs through LDS, others go one by one: the same results
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(33, 1104, 4100), (70, 8200, 4100), (40, 72, 300), (64, 8, 60), (1025, 2056, 300),
+                                   (4100, 4104, 200), (8190, 2056, 300)])
+def test_output_gate_aligned(M, N, K, dtype):
+    g = torch.Generator().manual_seed(M + K)
+    te, cc = (torch.randn(M, K, generator=g).to(dtype).to(DEV) for _ in range(2))
+    ws = [torch.randn(N, K, generator=g).to(dtype).to(DEV) for _ in range(2)]
+    sc = [hip_ops.absmean_scale(w) for w in ws]
+    pk = [hip_ops.pack_weight(w, s[0]) for w, s in zip(ws, sc)]
+    qt, qc = hip_ops.quant_act(te), hip_ops.quant_act(cc)
+    local, gate = (torch.randn(M, N, generator=g).to(dtype).to(DEV) for _ in range(2))
+    ys = []
+    for ld, at in ((2 * N + 16, (8, N + 8)), (2 * N + 5, (0, N + 5)), (2 * N + 16, (4, N + 8)), (2 * N + 16, (8, N + 10))):
+        lg = torch.full((M, ld), float("nan"), dtype=dtype, device=DEV)
+        lg[:, at[0]:at[0] + N] = local
+        lg[:, at[1]:at[1] + N] = gate
+        y, _ = hip_ops.output_gate(qt, qc, pk[0], sc[0][1], pk[1], sc[1][1], lg[:, at[0]:at[0] + N],
+                                   lg[:, at[1]:at[1] + N], K, quantize=False)
+        ys.append(y)
+    assert not bool(ys[0].isnan().any())
+    for y in ys[1:]:
+        assert torch.equal(ys[0], y)
