@@ -21,7 +21,7 @@
 // 4 stages all end within 10 % of each other): 8192 x 34816 x 4096 1025 us, 4096 x 14848 x 4096 233 (the two-stage
 // loop 1099 and 265).  A round or two lose part of that to the first K tiles' latency, the stores and the rounds' ends
 // (2048 x 4096 x 4096 1.87 POP/s, 4095 x 1024 x 2816 1.36, 8192 x 2432 x 768 1.22), the output gate to its one
-// workgroup per CU (4096 x 4096 x 2 x 2048 1.08).  Small ones are bound by the latency of the first tiles and by idle
+// workgroup per CU (4096 x 4096 x 2 x 2048 1.64).  Small ones are bound by the latency of the first tiles and by idle
 // CUs, hence the K groups: KS groups of waves in one workgroup take K tiles g, g + KS, ... into stages of their own,
 // and their exact int32 sums are added in LDS, so a 32 x 64 tile with a quarter of the K loop per group replaces
 // 64 x 128 tiles on a fifth of the CUs (512 x 768 x 3072 11.8 -> 6.0 us; 512 x 768 x 768 5.5 -> 4.3).
@@ -716,19 +716,21 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
   return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
 }
 
-// The output gate.  us, bf16 / f32 (M x N x 2 x K):
+// The output gate.  us, bf16 / f32 (M x N x 2 x K), with inputs and output in whole 16-byte rows:
 //   * 128x256 tiles: two accumulator sets, so one workgroup per CU and whole rounds of the CUs; taken where the rounds
-//     are nearly full, the fuller the shorter the K loop: 4096 x 4096 x 2 x 2048 102 / 149 (eight-wave 64x128 115 / 172),
-//     7000 x 1024 x 2 x 4096 74.8 / 98.1 (93.4 / 120), 4095 x 2048 x 2 x 1024 40.5 / 63.2 (41.8 / 69.9); not 7000 x 2432
-//     x 2 x 1280 (2.15 rounds) 116 / 186 (98.2 / 162), 3000 x 4096 x 2 x 2048 (1.5) 95.5 / 141 (86.8 / 126), 8300 x 2050
-//     x 2 x 300 114 / 136 (81.5 / 102).  At two K tiles they stand from two rounds on, though 64x128 ones would be
-//     faster (4095 x 4096 x 2 x 256 58.1 / 104, 49.0 / 104).
-//   * 64x128 tiles when they give every CU one: eight waves in bf16 (4095 x 1024 x 2 x 512 16.2, one-group form 28.6); in
-//     f32 32x64 tiles just past two per CU (2048 x 2432 x 2 x 1280 53.3, 57.4 with 64x128) and four waves beyond (7000 x
-//     2432 x 2 x 1280 155, eight 162; 8300 x 2048 x 2 x 1024 142, 148); at long K 32x64 up to three per two CUs (2048 x
-//     1024 x 2 x 4096 34.9 / 41.5, 40.9 / 47.0).
-//   * else 32x64 tiles of two waves: 512 x 768 x 2 x 384 7.6 (before 12.0); at long K with CUs left over, eight K groups on
-//     32x32 tiles or four on 32x64: 64 x 4096 x 2 x 8192 24.9 (before 51.4), 100 rows 33.9.
+//     are nearly full, the fuller the shorter the K loop: 4096 x 4096 x 2 x 2048 83.3 / 91.4 (eight-wave 64x128 102 / 107),
+//     7000 x 1024 x 2 x 4096 64.7 / 67.2 (86.1 / 88.7), 4095 x 2048 x 2 x 1024 29.4 / 32.2 (34.6 / 37.6: bf16 stays on it,
+//     as inputs and outputs in other rows are no faster with the large tiles); not 7000 x 2432 x 2 x 1280 (2.15 rounds)
+//     83.7 / 88.1 (79.9 / 87.0), 3000 x 4096 x 2 x 2048 (1.5) 74.0 / 79.5 (75.8 / 79.6, other rows 95.5 / 141, 86.8 /
+//     126), 8300 x 2050 x 2 x 300 116 / 140 (82.7 / 101).  At two K tiles they stand from two rounds on, though 64x128
+//     ones would be a little faster (4095 x 4096 x 2 x 256 38.1 / 47.5, 36.1 / 45.6; 4100 x 4104 x 2 x 200 47.5 / 52.7,
+//     38.9 / 47.8; other rows 4100 x 4100 x 2 x 200 77.2 / 154, 51.7 / 117).
+//   * 64x128 tiles when they give every CU one: eight waves in bf16 (4095 x 1024 x 2 x 512 13.2, one-group form 27.8); in
+//     f32 32x64 tiles just past two per CU (3000 x 1536 x 2 x 768 23.2, 25.9 with 64x128; 2048 x 2432 x 2 x 1280 32.4,
+//     32.9) and four waves beyond (7000 x 2432 x 2 x 1280 82.7, eight 87.0; 8300 x 2048 x 2 x 1024 72.6, 77.3); at long K
+//     32x64 up to three per two CUs (2048 x 1024 x 2 x 4096 32.2 / 32.8, 38.4 / 39.0).
+//   * else 32x64 tiles of two waves: 512 x 768 x 2 x 384 5.9 (one-group form 12.3); at long K with CUs left over, eight K
+//     groups on 32x32 tiles or four on 32x64: 64 x 4096 x 2 x 8192 21.9 (51.8), 100 rows 31.5.
 int dispatch_gate32(const LinearArgs& a, hipStream_t st) {
   auto tiles = [&](int64_t bm, int64_t bn) { return ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
   const int64_t cus = std::max(device_limits().cus, 1), big = tiles(128, 256), mid = tiles(64, 128);
