@@ -281,8 +281,8 @@ __device__ __forceinline__ void store_tiles32(const LinearArgs& a, const char* s
   }
 }
 
-// The slab's rows to outputs that are not in whole 16-byte rows: U (an element, or a bf16 pair where rows start on
-// four bytes) per lane, a store instruction covering whole rows again.  From the accumulators, four columns of 32 rows
+// The slab's rows to outputs that are not in whole 16-byte rows: U (an element, a bf16 pair where rows start on four
+// bytes, or 8 bytes where all rows are in whole ones) per lane, a store instruction covering whole rows again.  From the accumulators, four columns of 32 rows
 // per instruction, the stores touched a memory line per lane and cost as much as the product (us, M x N x K: 4093 x 4093
 // x 512 31.6 -> 20.3, f32 4093 x 3965 x 512 57.0 -> 19.3; 964 x 7932 x 1100 20.7 -> 16.6, f32 964 x 7835 x 4096 54.4 ->
 // 35.9; geometric mean of 120 sizes 1.48).
@@ -325,13 +325,9 @@ __device__ __forceinline__ void load_rows32(const LinearArgs& a, const void* p, 
   }
 }
 
-// ... and through the slab into the accumulators' order: f[j][g] holds the lane's four columns of tile j's group g,
-// float32 bits or two bf16 pairs.
-template <int OUT_DT>
-using Group4 = uint32_t __attribute__((ext_vector_type(OUT_DT == kBF16 ? 2 : 4)));
+// ... to the slab, ...
 template <int OUT_DT, int TN>
-__device__ __forceinline__ void slab_groups32(char* slab, const Chunk16 (&d)[TN * (OUT_DT == kBF16 ? 2 : 4)],
-                                              Group4<OUT_DT> (&f)[TN][4]) {
+__device__ __forceinline__ void slab_chunks32(char* slab, const Chunk16 (&d)[TN * (OUT_DT == kBF16 ? 2 : 4)]) {
   constexpr int ES = OUT_DT == kBF16 ? 2 : 4, PITCH = TN * 32 * ES + 16, CPR = TN * 2 * ES;
   const int lane = threadIdx.x & 63;
   wave_lds_fence();  // the slab's previous contents are consumed
@@ -339,6 +335,35 @@ __device__ __forceinline__ void slab_groups32(char* slab, const Chunk16 (&d)[TN 
   for (int it = 0; it < TN * ES; ++it)
     *reinterpret_cast<Chunk16*>(slab + (it * 64 + lane) / CPR * PITCH + lane % CPR * 16) = d[it];
   wave_lds_fence();
+}
+
+// (both for rows that are not in whole 16-byte chunks: an element per lane, or a bf16 pair or 8 bytes where all rows
+// are in whole ones)
+template <class U, int ES, int RB>
+__device__ __forceinline__ void slab_units32(const LinearArgs& a, char* slab, const void* p, int64_t ld, int64_t mb,
+                                             int64_t nb) {
+  constexpr int S = sizeof(U), UPR = RB / S, RPI = 64 / UPR, PITCH = RB + 16;  // units per row, rows per instruction
+  static_assert(UPR <= 64 && 64 % UPR == 0);
+  const int lane = threadIdx.x & 63, u = lane % UPR, r0 = lane / UPR;
+  const int64_t n = nb + u * (S / ES);
+  const char* src = static_cast<const char*>(p) + (n < a.N ? n : a.N - S / ES) * ES;
+  wave_lds_fence();  // the slab's previous contents are consumed
+#pragma unroll 4
+  for (int r = 0; r < 32; r += RPI) {
+    const int64_t m = mb + r + r0;
+    *reinterpret_cast<U*>(slab + (r + r0) * PITCH + u * S) = *reinterpret_cast<const U*>(src + (m < a.M ? m : a.M - 1) * ld * ES);
+  }
+  wave_lds_fence();
+}
+
+// ... and into the accumulators' order: f[j][g] holds the lane's four columns of tile j's group g, float32 bits or two
+// bf16 pairs.
+template <int OUT_DT>
+using Group4 = uint32_t __attribute__((ext_vector_type(OUT_DT == kBF16 ? 2 : 4)));
+template <int OUT_DT, int TN>
+__device__ __forceinline__ void slab_groups32(const char* slab, Group4<OUT_DT> (&f)[TN][4]) {
+  constexpr int ES = OUT_DT == kBF16 ? 2 : 4, PITCH = TN * 32 * ES + 16;
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int j = 0; j < TN; ++j)
 #pragma unroll
@@ -424,19 +449,36 @@ __device__ __forceinline__ void epilogue32(const LinearArgs& a, const v16i (&acc
     // most of the time, and in the accumulators' order each touches a memory line per lane (4095 x 5056 x 2 x 64 55.0 us ->
     // 37.9, f32 121.6 -> 44.2; 4096 x 4096 x 2 x 2048 103.5 -> 83.7, 147.7 -> 91.5; 512 x 768 x 2 x 384 7.9 -> 5.9; over
     // 330 sizes 1.38 times faster).
-    auto rows16 = [](const void* p, int64_t ld) {
-      return reinterpret_cast<uintptr_t>(p) % 16 == 0 && (ld * es) % 16 == 0;
-    };
-    if (a16 && tensor && rows16(a.local, a.ld_local) && rows16(a.gate, a.ld_gate) && (a.N * es) % 16 == 0) {
+    // Other rows go by smaller units (3000 x 2050 x 2 x 300 38.4 us -> 25.7, f32 4095 x 2050 55.0
+    // -> 36.5), in code of their own: inside one loop with these they cost the whole chunks 2 %.
+    constexpr int RB = TN * 32 * es;
+    auto bits = [](const void* p, int64_t ld) { return reinterpret_cast<uintptr_t>(p) | static_cast<uintptr_t>(ld * es); };
+    const uintptr_t in = bits(a.local, a.ld_local) | bits(a.gate, a.ld_gate) | static_cast<uintptr_t>(a.N * es);
+    auto rows = [&](auto chunks) {
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
         const int64_t mb = m0 + (wm * TM + i) * 32, nb = n0 + wn * TN * 32;
-        Chunk16 dl[TN * es], dg[TN * es];
-        load_rows32<OUT_DT, TN>(a, a.local, a.ld_local, mb, nb, dl);
-        load_rows32<OUT_DT, TN>(a, a.gate, a.ld_gate, mb, nb, dg);
         Group4<OUT_DT> lo[TN][4], gt[TN][4];
-        slab_groups32<OUT_DT, TN>(slab, dl, lo);
-        slab_groups32<OUT_DT, TN>(slab, dg, gt);
+        if constexpr (decltype(chunks)::value) {
+          Chunk16 dl[TN * es], dg[TN * es];
+          load_rows32<OUT_DT, TN>(a, a.local, a.ld_local, mb, nb, dl);
+          load_rows32<OUT_DT, TN>(a, a.gate, a.ld_gate, mb, nb, dg);
+          slab_chunks32<OUT_DT, TN>(slab, dl);
+          slab_groups32<OUT_DT, TN>(slab, lo);
+          slab_chunks32<OUT_DT, TN>(slab, dg);
+          slab_groups32<OUT_DT, TN>(slab, gt);
+        } else {
+          auto units = [&](const void* p, int64_t ld) {
+            if (in % 8 == 0) return slab_units32<uint64_t, es, RB>(a, slab, p, ld, mb, nb);
+            if constexpr (OUT_DT == kBF16)
+              if (in % 4 != 0) return slab_units32<uint16_t, es, RB>(a, slab, p, ld, mb, nb);
+            slab_units32<uint32_t, es, RB>(a, slab, p, ld, mb, nb);
+          };
+          units(a.local, a.ld_local);
+          slab_groups32<OUT_DT, TN>(slab, lo);
+          units(a.gate, a.ld_gate);
+          slab_groups32<OUT_DT, TN>(slab, gt);
+        }
         fill_slab32<OUT_DT, TN>(slab, [&](int j, int g, float (&v)[4]) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -446,15 +488,29 @@ __device__ __forceinline__ void epilogue32(const LinearArgs& a, const v16i (&acc
                                          group_at<OUT_DT>(gt[j][g], r));
           }
         });
-        store_tiles32<OUT_DT, TN>(a, slab, mb, nb);
+        if constexpr (decltype(chunks)::value) {
+          store_tiles32<OUT_DT, TN>(a, slab, mb, nb);
+        } else {
+          if ((bits(a.out, a.ldo) | static_cast<uintptr_t>(a.N * es)) % 8 == 0) {
+            store_rows32<uint64_t, es, RB>(a, slab, mb, nb);
+            continue;
+          }
+          if constexpr (OUT_DT == kBF16)
+            if (bits(a.out, a.ldo) % 4 != 0) {
+              store_rows32<uint16_t, es, RB>(a, slab, mb, nb);
+              continue;
+            }
+          store_rows32<uint32_t, es, RB>(a, slab, mb, nb);
+        }
       }
-      return;
-    }
+    };
+    if (a16 && tensor && in % 16 == 0) return rows(std::true_type{});
+    if (tensor) return rows(std::false_type{});
   }
-  // General form: per-row weight scales, bias, accumulator dump, and what is not in whole 16-byte rows of SwiGLU, the
-  // gates and the output gate.  The output gate's inputs of one 32 x 32 tile (four groups of four columns per lane) are
-  // requested together in straight-line code (indices clamped into range, raw bits) before any is used, so the tile
-  // waits for memory once instead of once per group.
+  // General form: per-row weight scales, bias, accumulator dump, and what is not in whole 16-byte rows of SwiGLU and the
+  // gates.  The output gate's inputs of one 32 x 32 tile (four groups of four columns per lane) are requested together in
+  // straight-line code (indices clamped into range, raw bits) before any is used, so the tile waits for memory once
+  // instead of once per group.
   const bool vout = vec4_ok<OUT_DT>(a.out, a.ldo);
   const bool vin = EPI == kEpiOutputGate && vec4_ok<OUT_DT>(a.local, a.ld_local) &&
                    vec4_ok<OUT_DT>(a.gate, a.ld_gate) && a.N % 4 == 0;
@@ -716,15 +772,15 @@ int dispatch_store32(const LinearArgs& a, hipStream_t st) {
   return run_mfma32<1, 4, 2, 1, EPI, 2>(a, st);
 }
 
-// The output gate.  us, bf16 / f32 (M x N x 2 x K), with inputs and output in whole 16-byte rows:
+// The output gate.  us, bf16 / f32 (M x N x 2 x K):
 //   * 128x256 tiles: two accumulator sets, so one workgroup per CU and whole rounds of the CUs; taken where the rounds
 //     are nearly full, the fuller the shorter the K loop: 4096 x 4096 x 2 x 2048 83.3 / 91.4 (eight-wave 64x128 102 / 107),
-//     7000 x 1024 x 2 x 4096 64.7 / 67.2 (86.1 / 88.7), 4095 x 2048 x 2 x 1024 29.4 / 32.2 (34.6 / 37.6: bf16 stays on it,
-//     as inputs and outputs in other rows are no faster with the large tiles); not 7000 x 2432 x 2 x 1280 (2.15 rounds)
-//     83.7 / 88.1 (79.9 / 87.0), 3000 x 4096 x 2 x 2048 (1.5) 74.0 / 79.5 (75.8 / 79.6, other rows 95.5 / 141, 86.8 /
-//     126), 8300 x 2050 x 2 x 300 116 / 140 (82.7 / 101).  At two K tiles they stand from two rounds on, though 64x128
-//     ones would be a little faster (4095 x 4096 x 2 x 256 38.1 / 47.5, 36.1 / 45.6; 4100 x 4104 x 2 x 200 47.5 / 52.7,
-//     38.9 / 47.8; other rows 4100 x 4100 x 2 x 200 77.2 / 154, 51.7 / 117).
+//     7000 x 1024 x 2 x 4096 64.7 / 67.2 (86.1 / 88.7), 4095 x 2048 x 2 x 1024 29.4 / 32.2 (34.6 / 37.6); not 7000 x 2432
+//     x 2 x 1280 (2.15 rounds) 83.7 / 88.1 (79.9 / 87.0), 3000 x 4096 x 2 x 2048 (1.5) 74.0 / 79.5 (75.8 / 79.6).  These
+//     lines were drawn when bf16 inputs and outputs went in the accumulators' order, which favoured small tiles: bf16 at
+//     one round and K up to 1024 would now gain from the large ones, as above.  At two K tiles they stand from two rounds
+//     on, though 64x128 ones would be a little faster (4095 x 4096 x 2 x 256 38.1 / 47.5, 36.1 / 45.6; 4100 x 4104 x 2 x
+//     200 47.5 / 52.7, 38.9 / 47.8).
 //   * 64x128 tiles when they give every CU one: eight waves in bf16 (4095 x 1024 x 2 x 512 13.2, one-group form 27.8); in
 //     f32 32x64 tiles just past two per CU (3000 x 1536 x 2 x 768 23.2, 25.9 with 64x128; 2048 x 2432 x 2 x 1280 32.4,
 //     32.9) and four waves beyond (7000 x 2432 x 2 x 1280 82.7, eight 87.0; 8300 x 2048 x 2 x 1024 72.6, 77.3); at long K

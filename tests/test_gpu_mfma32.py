@@ -235,3 +235,13 @@ def test_output_gate_aligned(M, N, K, dtype):
     assert not bool(ys[0].isnan().any())
     for y in ys[1:]:
         assert torch.equal(ys[0], y)
+
+
+# rows of odd lengths: single elements, the last one alone in its pair's place
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,kernel", [(41, 71, 300, "mfma32_kernel<1,2,1,1,1,"), (33, 1, 60, "mfma32_kernel<1,2,1,1,1,"),
+                                          (33, 1103, 4100, "mfma32k_kernel<1,1,1,1,8,3,1,"),
+                                          (1025, 2051, 300, "mfma32_kernel<2,4,1,1,1,"),
+                                          (4099, 4097, 200, "mfma32_kernel<2,4,2,2,1,")])
+def test_output_gate_odd_rows(M, N, K, kernel, dtype):
+    test_output_gate_products(M, N, K, kernel, dtype)
